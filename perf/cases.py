@@ -265,14 +265,17 @@ def _offsets(n):
 # States
 # ---------------------------------------------------------------------------
 class _Ptr:
-    """A device array the library owns, for torch.as_tensor."""
+    """A device array of a session, for torch.as_tensor; the tensor keeps the session's handle alive."""
 
-    def __init__(self, ptr, n, typestr="<i4"):
+    def __init__(self, ptr, n, handle, typestr="<i4"):
+        self.handle = handle
         self.__cuda_array_interface__ = {"data": (ptr, False), "shape": (n,), "typestr": typestr, "version": 2}
 
 
-class Session:
-    def __init__(self, max_blocks=16):
+class _Handle:
+    """Owns an xg_session: destroyed with the last state or output that refers to it."""
+
+    def __init__(self, max_blocks):
         self.lib = capi.load()
         self.s = ctypes.c_void_p()
         capi.check(self.lib.xg_session_create(ctypes.byref(self.s), max_blocks), "session")
@@ -281,10 +284,17 @@ class Session:
         if self.s:
             self.lib.xg_session_destroy(self.s)
 
+
+class Session:
+    def __init__(self, max_blocks=16):
+        self.handle = _Handle(max_blocks)
+        self.lib, self.s = self.handle.lib, self.handle.s
+
     def outputs(self, n, ncand):
         c, b = ctypes.c_void_p(), ctypes.c_void_p()
         capi.check(self.lib.xg_session_outputs(self.s, ctypes.byref(c), ctypes.byref(b)), "outputs")
-        return [torch.as_tensor(_Ptr(c.value, n * ncand), device=DEV), torch.as_tensor(_Ptr(b.value, 4 * n), device=DEV)]
+        return [torch.as_tensor(_Ptr(c.value, n * ncand, self.handle), device=DEV),
+                torch.as_tensor(_Ptr(b.value, 4 * n, self.handle), device=DEV)]
 
 
 def _empty(n, dtype=torch.int32):
