@@ -1,0 +1,79 @@
+"""The bounded integer searches (block-sum elimination) against the oracle's
+exhaustive one, on content that takes each of their paths: textures (few
+candidates left), flat noise (too many left: the exhaustive list), extreme
+samples (the largest sums), repeated texture and constant planes (ties in
+raster order), windows cut at an odd column, and rate weights past the rule."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from tests.helpers import ptr
+from xin26x_amd import capi, workloads as wl
+from xin26x_amd.device import DevicePicture, refine_cfg
+
+pytestmark = pytest.mark.gpu
+
+
+def content(kind, h, w, seed=3):
+    """Current plane and two reference planes."""
+    r = np.random.default_rng(seed)
+    if kind == "texture":
+        f = wl.smooth_field(h + 80, w + 80, seed)
+        cut = lambda dy, dx: f[40 + dy:40 + dy + h, 40 + dx:40 + dx + w]
+        out = [cut(0, 0) + r.integers(-4, 5, (h, w)), cut(9, -23), cut(-31, 14) + r.integers(-2, 3, (h, w))]
+    elif kind == "flat":
+        out = [500 + np.rint(r.normal(0, 4, (h, w))) for _ in range(3)]
+    elif kind == "half":
+        a, b = content("texture", h, w, seed), content("flat", h, w, seed)
+        out = [np.where(np.arange(w) < w // 2, p, q) for p, q in zip(a, b)]
+    elif kind == "extreme":
+        out = [r.integers(0, 2, (h // 8 + 1, w // 8 + 1)).repeat(8, 0).repeat(8, 1)[:h, :w] * 1023 for _ in range(3)]
+    elif kind == "periodic":
+        t = r.integers(0, 1024, (8, 12))
+        out = [np.tile(np.roll(t, k, 1), (h // 8 + 1, w // 12 + 1))[:h, :w] for k in range(3)]
+    else:
+        out = [np.full((h, w), v) for v in (1023, 0, 1023)]
+    return [np.ascontiguousarray(np.clip(p, 0, 1023).astype(np.uint16)) for p in out]
+
+
+def oracle_search(oracle, cur, ref, bw, bh, rng, lam, ctu, pad):
+    h, w = cur.shape
+    nb = (w // bw) * (h // bh)
+    refp = np.ascontiguousarray(np.pad(ref, pad, mode="edge"))
+    mx, my = np.zeros(nb, np.int16), np.zeros(nb, np.int16)
+    c, s = np.zeros(nb, np.uint32), np.zeros(nb, np.uint32)
+    oracle.or_FullSearchFrame(ptr(cur), w, ptr(refp, pad * (w + 2 * pad) + pad), w + 2 * pad, w, h, bw, bh, rng, lam, ctu,
+                              0, nb, ptr(mx), ptr(my), ptr(c), ptr(s))
+    return mx, my, c, s
+
+
+@pytest.mark.parametrize("kind,rng,ctu,lam", [
+    ("texture", 64, 64, 1024), ("texture", 33, 64, 0), ("texture", 7, 16, 300), ("texture", 64, 33, 1024),
+    ("texture", 0, 64, 1024), ("texture", 64, 64, 1 << 21), ("texture", 40, 64, (1 << 21) + 1), ("flat", 64, 64, 1024),
+    ("half", 64, 64, 1024), ("extreme", 64, 64, 1024), ("periodic", 50, 64, 0), ("constant", 64, 31, 0)])
+def test_pipeline_full_search(oracle, kind, rng, ctu, lam):
+    lib = capi.load()
+    h, w, pad = 64, 112, 152
+    planes = content(kind, h, w)
+    half = lambda p: np.ascontiguousarray(p[::2, ::2])
+    pics = [DevicePicture([p, half(p), half(p)], pad) for p in planes]
+    pred = DevicePicture.empty(w, h)
+    nb = (w // 16) * (h // 16)
+    s = ctypes.c_void_p()
+    assert lib.xg_session_create(ctypes.byref(s), nb) == 0
+    try:
+        cfg = capi.XgPipelineCfg()
+        cfg.range, cfg.sadLambda, cfg.ctuSize = rng, lam, ctu
+        cfg.refine = refine_cfg([(0, 0)], wl.LAMBDA_REFINE)
+        for mode in (capi.MODE_BATCHED, capi.MODE_GRAPH, capi.MODE_GRAPH):
+            assert lib.xg_me_pipeline(s, ctypes.byref(cfg), pics[0].ref(), pics[1].ref(), pics[2].ref(), pred.ref(),
+                                      mode) == 0
+            full = np.zeros((nb, 2, 2), np.int16)
+            assert lib.xg_me_pipeline_read(s, full.ctypes.data, None, None, None, None, None) == 0
+            for r in (0, 1):
+                mx, my, _, _ = oracle_search(oracle, planes[0], planes[1 + r], 16, 16, rng, lam, ctu, pad)
+                # the frame search reports quarter pel, the pipeline integer pel
+                assert np.array_equal(full[:, r, 0], mx >> 2) and np.array_equal(full[:, r, 1], my >> 2), (mode, r)
+    finally:
+        lib.xg_session_destroy(s)
