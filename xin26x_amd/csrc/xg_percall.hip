@@ -1,10 +1,12 @@
 // xg_percall.hip -- the per-call primitives of the xin_func_struct mirror.
 //
-// Each entry point takes the reference's host pointers, stages exactly the
+// Each entry point takes the reference's host pointers and stages exactly the
 // samples the reference function reads into pinned memory (samples it does
-// not read are zero-filled and only ever meet zero filter taps), copies them
-// to HBM on the calling thread's stream, runs one kernel and copies the
-// result back before returning.
+// not read are zero-filled and only ever meet zero filter taps).  Where the
+// kernel reads each sample once (SAD, SATD, interpolation, the searches), it
+// reads them there and writes its result there, over the mapping the device
+// has of pinned memory: a call is one launch and one wait.  The others copy to
+// HBM on the calling thread's stream and the result back.
 //
 // Interpolation: every table slot (Copy, Hor, Vet, HorVet and their S16
 // variants) runs the same separable kernel with a phase-0 filter in the
@@ -53,23 +55,42 @@ bool device_init()
 // ---------------------------------------------------------------------------
 
 // Separable interpolation of a packed region: src holds (h+TAPS-1) rows of
-// (w+TAPS-1) samples starting TAPS/2-1 samples above/left of the block.
+// (w+TAPS-1) samples starting TAPS/2-1 samples above/left of the block.  A
+// workgroup forms kInterpRows rows of up to 64 columns: it reads its samples
+// once, coalesced (src and dst may be mapped host memory, where every access is
+// a bus transfer), runs the first pass into LDS and the second from there.
+constexpr int kInterpRows = 8;
+
 template <int TAPS, bool S16>
-__global__ void k_interp(const uint16_t *__restrict__ src, int w, int h, int fx, int fy, int fi,
-                         void *__restrict__ dst)
+__global__ void __launch_bounds__(256) k_interp(const uint16_t *__restrict__ src, int w, int h, int fx, int fy, int fi,
+                                                void *__restrict__ dst)
 {
-    const int x = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y;
-    if (x >= w || y >= h) return;
-    const int ss = w + TAPS - 1;
+    __shared__ uint16_t win[(kInterpRows + TAPS - 1) * (64 + TAPS)];
+    __shared__ int16_t mid[(kInterpRows + TAPS - 1) * 64];
+    const int x0 = blockIdx.x * 64, y0 = blockIdx.y * kInterpRows;
+    const int cols = min(64, w - x0), rows = min(kInterpRows, h - y0);
+    const int ss = w + TAPS - 1, wc = cols + TAPS - 1, wr = rows + TAPS - 1;
+    for (int i = threadIdx.x; i < wr * wc; i += 256) {
+        const int r = i / wc, c = i - r * wc;
+        win[r * (64 + TAPS) + c] = src[(y0 + r) * ss + x0 + c];
+    }
+    __syncthreads();
     const int8_t *ch = taps_for<TAPS>(fx, fi);
     const int8_t *cv = taps_for<TAPS>(fy, fi);
-    const uint16_t *p = src + y * ss + x;
-    int acc = 0;
+    for (int i = threadIdx.x; i < wr * cols; i += 256) {
+        const int r = i / cols, c = i - r * cols;
+        mid[r * 64 + c] = (int16_t)hpass<TAPS>(&win[r * (64 + TAPS) + c], ch);
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < rows * cols; i += 256) {
+        const int r = i / cols, c = i - r * cols;
+        int acc = 0;
 #pragma unroll
-    for (int k = 0; k < TAPS; k++) acc += (int)cv[k] * hpass<TAPS>(p + k * ss, ch);
-    if constexpr (S16) ((int16_t *)dst)[y * w + x] = (int16_t)vfinal_s16(acc);
-    else ((uint16_t *)dst)[y * w + x] = (uint16_t)vfinal_pix(acc);
+        for (int k = 0; k < TAPS; k++) acc += (int)cv[k] * (int)mid[(r + k) * 64 + c];
+        const int o = (y0 + r) * w + x0 + c;
+        if constexpr (S16) ((int16_t *)dst)[o] = (int16_t)vfinal_s16(acc);
+        else ((uint16_t *)dst)[o] = (uint16_t)vfinal_pix(acc);
+    }
 }
 
 // Vertical pass over an S16 first-pass buffer (VetS16U8 / VetS16S16):
@@ -287,7 +308,7 @@ static void interp_u16(int taps, bool outS16, Dir dir, const uint16_t *src, intp
     if (fi < 0 || fi > 2) fi = 0;   // the reference treats any other index as the default filter
     const int hb = taps / 2 - 1, rw = (int)w + taps - 1, rh = (int)h + taps - 1;
     const size_t inB = align_up((size_t)rw * rh * 2, 256), outB = (size_t)w * h * 2;
-    CallCtx *c = call_ctx(inB + outB, inB + outB);
+    CallCtx *c = call_ctx(0, inB + outB);
     if (!c) return;
     uint16_t *hin = (uint16_t *)c->host;
     memset(hin, 0, (size_t)rw * rh * 2);
@@ -296,9 +317,8 @@ static void interp_u16(int taps, bool outS16, Dir dir, const uint16_t *src, intp
     const int c0 = cols ? 0 : hb, c1 = cols ? rw : hb + (int)w;
     for (int r = r0; r < r1; r++)
         memcpy(hin + (size_t)r * rw + c0, src + (intptr_t)(r - hb) * ss + (c0 - hb), (size_t)(c1 - c0) * 2);
-    char *din = c->dev, *dout = c->dev + inB;
-    if (!XG_HIP(hipMemcpyAsync(din, hin, (size_t)rw * rh * 2, hipMemcpyHostToDevice, c->stream))) return;
-    dim3 grid((w + 63) / 64, h), block(64);
+    char *din = c->view, *dout = c->view + inB;
+    dim3 grid((w + 63) / 64, (h + kInterpRows - 1) / kInterpRows), block(256);
     if (taps == 8) {
         if (outS16) k_interp<8, true><<<grid, block, 0, c->stream>>>((uint16_t *)din, w, h, fx, fy, fi, dout);
         else k_interp<8, false><<<grid, block, 0, c->stream>>>((uint16_t *)din, w, h, fx, fy, fi, dout);
@@ -308,7 +328,6 @@ static void interp_u16(int taps, bool outS16, Dir dir, const uint16_t *src, intp
     }
     if (!XG_HIP(hipGetLastError())) return;
     char *hout = c->host + inB;
-    if (!XG_HIP(hipMemcpyAsync(hout, dout, outB, hipMemcpyDeviceToHost, c->stream))) return;
     if (!finish(c)) return;
     unpack2d(dst, ds, hout, (int)w, (int)h, 2);
 }
@@ -368,17 +387,14 @@ static void sad_multi(const uint16_t *in, intptr_t is, const uint16_t *const *re
     if (!check_wh(w, h, 128, 128, fn)) return;
     const size_t npix = (size_t)w * h, blk = align_up(npix * 2, 256);
     const size_t bytes = blk * (1 + nref) + 256;
-    CallCtx *c = call_ctx(bytes, bytes);
+    CallCtx *c = call_ctx(0, bytes);
     if (!c) return;
     pack2d(c->host, in, is, (int)w, (int)h, 2);
     for (int k = 0; k < nref; k++) pack2d(c->host + blk * (1 + k), refs[k], rs, (int)w, (int)h, 2);
-    if (!XG_HIP(hipMemcpyAsync(c->dev, c->host, blk * (1 + nref), hipMemcpyHostToDevice, c->stream))) return;
-    uint32_t *dres = (uint32_t *)(c->dev + blk * (1 + nref));
-    k_sad<<<nref, 256, 0, c->stream>>>((uint16_t *)c->dev, (uint16_t *)(c->dev + blk), (int)npix, (int)(blk / 2),
-                                       dres);
+    k_sad<<<nref, 256, 0, c->stream>>>((uint16_t *)c->view, (uint16_t *)(c->view + blk), (int)npix, (int)(blk / 2),
+                                       (uint32_t *)(c->view + blk * (1 + nref)));
     if (!XG_HIP(hipGetLastError())) return;
     uint32_t *hres = (uint32_t *)(c->host + blk * (1 + nref));
-    if (!XG_HIP(hipMemcpyAsync(hres, dres, 4 * nref, hipMemcpyDeviceToHost, c->stream))) return;
     if (!finish(c)) return;
     for (int k = 0; k < nref; k++) out[k] = hres[k];
 }
@@ -431,15 +447,13 @@ static void satd_call(const uint16_t *in, intptr_t is, const uint16_t *pr, intpt
         return;
     }
     const size_t npix = (size_t)w * h, blk = align_up(npix * 2, 256);
-    CallCtx *c = call_ctx(2 * blk + 256, 2 * blk + 256);
+    CallCtx *c = call_ctx(0, 2 * blk + 256);
     if (!c) return;
     pack2d(c->host, in, is, (int)w, (int)h, 2);
     pack2d(c->host + blk, pr, ps, (int)w, (int)h, 2);
-    if (!XG_HIP(hipMemcpyAsync(c->dev, c->host, 2 * blk, hipMemcpyHostToDevice, c->stream))) return;
-    k_satd<<<1, 256, 0, c->stream>>>((uint16_t *)c->dev, (uint16_t *)(c->dev + blk), (int)w, (int)h,
-                                     (uint32_t *)(c->dev + 2 * blk));
+    k_satd<<<1, 256, 0, c->stream>>>((uint16_t *)c->view, (uint16_t *)(c->view + blk), (int)w, (int)h,
+                                     (uint32_t *)(c->view + 2 * blk));
     if (!XG_HIP(hipGetLastError())) return;
-    if (!XG_HIP(hipMemcpyAsync(c->host + 2 * blk, c->dev + 2 * blk, 4, hipMemcpyDeviceToHost, c->stream))) return;
     if (!finish(c)) return;
     *out = *(uint32_t *)(c->host + 2 * blk);
 }

@@ -87,13 +87,14 @@ CallCtx *call_ctx(size_t devBytes, size_t hostBytes)
     }
     if (hostBytes > c->hostCap) {
         if (c->host) (void)hipHostFree(c->host);
-        c->host = nullptr;
+        c->host = c->view = nullptr;
         c->hostCap = 0;
         size_t cap = align_up(hostBytes < (1u << 20) ? (1u << 20) : hostBytes, 4096);
-        if (!XG_HIP(hipHostMalloc((void **)&c->host, cap, hipHostMallocDefault))) {
+        if (!XG_HIP(hipHostMalloc((void **)&c->host, cap, hipHostMallocMapped | hipHostMallocCoherent))) {
             set_error(XG_ERR_NOMEM, "pinned staging of %zu bytes failed", cap);
             return nullptr;
         }
+        if (!XG_HIP(hipHostGetDevicePointer((void **)&c->view, c->host, 0))) return nullptr;
         c->hostCap = cap;
     }
     return c;

@@ -28,6 +28,7 @@ struct CallCtx {
     hipStream_t stream = nullptr;
     char *dev = nullptr;   size_t devCap = 0;
     char *host = nullptr;  size_t hostCap = 0;
+    char *view = nullptr;  // the device's address of `host` (page-locked memory is mapped)
 };
 
 // Returns the calling thread's context with at least devBytes of device

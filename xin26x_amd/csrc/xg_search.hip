@@ -10,7 +10,7 @@
 //    (XIN_COST_FRACTION 8, common/include/h26x_definition.h:88; MVD in
 //    quarter pel as CALC_MVD_BIT is used at h266_sub_pel_refine.c:155-156).
 //  * Xg26xMotionEstDia: start candidates then small-diamond descent, one
-//    workgroup, SADs reduced across its 256 threads.
+//    workgroup, a position per wave.
 //  * Xg266FullSubPelMe: the half-pel and quarter-pel rings of
 //    h266_encoder/source/h266_sub_pel_refine.c:81-212 with the 8-tap luma
 //    interpolation (filterIndex 0) and SAD.
@@ -34,18 +34,6 @@ __device__ __forceinline__ unsigned long long block_min_u64(unsigned long long v
     __syncthreads();
     unsigned long long r = red[0];
     for (int i = 1; i < (int)(blockDim.x >> 6); i++) r = red[i] < r ? red[i] : r;
-    __syncthreads();
-    return r;
-}
-
-__device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, uint32_t *red)
-{
-    v = (uint32_t)group_sum<64>((int)v);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) red[wid] = v;
-    __syncthreads();
-    uint32_t r = 0;
-    for (int i = 0; i < (int)(blockDim.x >> 6); i++) r += red[i];
     __syncthreads();
     return r;
 }
@@ -319,47 +307,119 @@ __global__ void __launch_bounds__(256) k_full_search_one(const uint16_t *gwin, i
     }
 }
 
-// SAD of the block at integer offset (mx, my) inside a packed region whose
-// origin is (rx0, ry0) relative to the co-located position; block-wide sum.
-__device__ uint32_t region_sad(const uint16_t *reg, int rstride, int rx0, int ry0, const uint16_t *cur, int bw,
-                               int bh, int mx, int my, uint32_t *red)
+// Region and block (na and nb packed samples, 16-byte aligned, readable to a
+// multiple of 8) into LDS at dst and dst + align8(na), 16 bytes a thread and
+// load, every load of a thread issued before its first store: over the bus each
+// round trip costs about 2 us.
+__host__ __device__ constexpr int align8(int n) { return (n + 7) & ~7; }
+
+__device__ __forceinline__ void stage_packed(uint16_t *dst, const uint16_t *a, int na, const uint16_t *b, int nb)
 {
-    const uint16_t *w = reg + (my - ry0) * rstride + (mx - rx0);
-    uint32_t s = 0;
-    for (int i = threadIdx.x; i < bw * bh; i += blockDim.x) {
-        const int r = i / bw, c = i % bw;
-        s += (uint32_t)abs((int)cur[i] - (int)w[r * rstride + c]);
+    const int qa = (na + 7) >> 3, n = qa + ((nb + 7) >> 3);
+    const uint4 *pa = reinterpret_cast<const uint4 *>(a), *pb = reinterpret_cast<const uint4 *>(b) - qa;
+    for (int i0 = threadIdx.x; i0 < n; i0 += 8 * (int)blockDim.x) {
+        uint4 v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int i = min(i0 + k * (int)blockDim.x, n - 1);
+            v[k] = *(i < qa ? pa + i : pb + i);
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int i = i0 + k * (int)blockDim.x;
+            if (i < n) reinterpret_cast<uint4 *>(dst)[i] = v[k];
+        }
     }
-    return block_sum_u32(s, red);
 }
 
-// Diamond search in one workgroup; the region covers every position the
-// search can read.  out: bestX, bestY (integer pel), cost, sad.
-__global__ void __launch_bounds__(256) k_dia_one(const uint16_t *reg, int rstride, int rx0, int ry0,
-                                                 const uint16_t *cur, int bw, int bh, const int16_t *cand,
-                                                 int ncand, int mnx, int mny, int mxx, int mxy, int cx, int cy,
+// SAD of the block at integer offset (mx, my) inside a packed region whose
+// origin is (rx0, ry0) relative to the co-located position, by the calling wave;
+// every lane gets it.
+__device__ uint32_t wave_sad(const uint16_t *reg, int rstride, int rx0, int ry0, const uint16_t *cur, int bw, int bh,
+                             int mx, int my)
+{
+    const int lane = threadIdx.x & 63, dr = 64 / bw, dc = 64 - dr * bw;
+    const uint16_t *w = reg + (my - ry0) * rstride + (mx - rx0);
+    int r = lane / bw, c = lane - r * bw;
+    uint32_t s = 0;
+    for (int i = lane; i < bw * bh; i += 64) {
+        s += (uint32_t)abs((int)cur[i] - (int)w[r * rstride + c]);
+        r += dr;
+        c += dc;
+        if (c >= bw) {
+            c -= bw;
+            r++;
+        }
+    }
+    return (uint32_t)group_sum<64>((int)s);
+}
+
+// Diamond search in one workgroup of four waves; the region covers every
+// position the search can read.  Each wave costs one of four positions at a time
+// (start candidates, then the diamond's four), so a step is one barrier pair.
+// STAGE: region and block are read once into LDS (they may be mapped host
+// memory).  out: bestX, bestY (integer pel), cost, sad.
+struct DiaCands {
+    int16_t v[24];                 // (x, y) of up to 12
+};
+
+template <bool STAGE>
+__global__ void __launch_bounds__(256) k_dia_one(const uint16_t *greg, int rstride, int rrows, int rx0, int ry0,
+                                                 const uint16_t *gcur, int bw, int bh, DiaCands cands, int ncand, int mnx, int mny, int mxx, int mxy, int cx, int cy,
                                                  int sw, int sh, uint32_t lambda, int pmx, int pmy, uint32_t *out)
 {
-    __shared__ uint32_t red[4];
+    extern __shared__ __align__(16) uint16_t smem[];
+    __shared__ uint32_t sads[12];
+    __shared__ int16_t cand[24];
+    const int wave = threadIdx.x >> 6;
+    const uint16_t *reg = greg, *cur = gcur;
+    if (STAGE) {
+        stage_packed(smem, greg, rstride * rrows, gcur, bw * bh);
+        reg = smem;
+        cur = smem + align8(rstride * rrows);
+    }
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int i = 0; i < 24; i++) cand[i] = cands.v[i];
+    __syncthreads();
+    for (int i = wave; i < ncand; i += 4) {
+        const int mx = min(max((int)cand[2 * i], mnx), mxx), my = min(max((int)cand[2 * i + 1], mny), mxy);
+        const uint32_t s = wave_sad(reg, rstride, rx0, ry0, cur, bw, bh, mx, my);
+        if ((threadIdx.x & 63) == 0) sads[i] = s;
+    }
+    __syncthreads();
     uint32_t best = 0xFFFFFFFFu, bestSad = 0xFFFFFFFFu;
     int bx = 0, by = 0;
     for (int i = 0; i < ncand; i++) {
         const int mx = min(max((int)cand[2 * i], mnx), mxx), my = min(max((int)cand[2 * i + 1], mny), mxy);
-        const uint32_t sad = region_sad(reg, rstride, rx0, ry0, cur, bw, bh, mx, my, red);
-        const uint32_t c = (sad << 8) + (eg_bits(4 * mx - pmx) + eg_bits(4 * my - pmy)) * lambda;
-        if (c < best) { best = c; bestSad = sad; bx = mx; by = my; }
+        const uint32_t c = (sads[i] << 8) + (eg_bits(4 * mx - pmx) + eg_bits(4 * my - pmy)) * lambda;
+        if (c < best) { best = c; bestSad = sads[i]; bx = mx; by = my; }
     }
     const int dxs[4] = {-1, 1, 0, 0}, dys[4] = {0, 0, -1, 1};
     for (int it = 0; it < sw + sh; it++) {
-        int nx = bx, ny = by;
-        uint32_t nb = best, ns = bestSad;
+        bool ok[4];
+#pragma unroll
         for (int k = 0; k < 4; k++) {
             const int mx = bx + dxs[k], my = by + dys[k];
-            if (mx < mnx || mx > mxx || my < mny || my > mxy) continue;
-            if (mx < cx - sw || mx > cx + sw || my < cy - sh || my > cy + sh) continue;
-            const uint32_t sad = region_sad(reg, rstride, rx0, ry0, cur, bw, bh, mx, my, red);
-            const uint32_t c = (sad << 8) + (eg_bits(4 * mx - pmx) + eg_bits(4 * my - pmy)) * lambda;
-            if (c < nb) { nb = c; ns = sad; nx = mx; ny = my; }
+            ok[k] = mx >= mnx && mx <= mxx && my >= mny && my <= mxy && mx >= cx - sw && mx <= cx + sw &&
+                    my >= cy - sh && my <= cy + sh;
+        }
+        const int ox = wave == 0 ? -1 : wave == 1 ? 1 : 0, oy = wave == 2 ? -1 : wave == 3 ? 1 : 0;
+        const bool mine = wave == 0 ? ok[0] : wave == 1 ? ok[1] : wave == 2 ? ok[2] : ok[3];
+        __syncthreads();                             // the previous step's readers of sads are done
+        if (mine) {
+            const uint32_t s = wave_sad(reg, rstride, rx0, ry0, cur, bw, bh, bx + ox, by + oy);
+            if ((threadIdx.x & 63) == 0) sads[wave] = s;
+        }
+        __syncthreads();
+        int nx = bx, ny = by;
+        uint32_t nb = best, ns = bestSad;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (!ok[k]) continue;
+            const int mx = bx + dxs[k], my = by + dys[k];
+            const uint32_t c = (sads[k] << 8) + (eg_bits(4 * mx - pmx) + eg_bits(4 * my - pmy)) * lambda;
+            if (c < nb) { nb = c; ns = sads[k]; nx = mx; ny = my; }
         }
         if (nx == bx && ny == by) break;
         bx = nx; by = ny; best = nb; bestSad = ns;
@@ -375,36 +435,83 @@ __global__ void __launch_bounds__(256) k_dia_one(const uint16_t *reg, int rstrid
 // Half-pel then quarter-pel ring around (qx, qy) (quarter pel).  reg: luma
 // samples whose first row/column is (rx0, ry0) relative to the co-located
 // block position (the host stages integer positions -1..+1 plus 8-tap reach).
-__global__ void __launch_bounds__(256) k_subpel_one(const uint16_t *reg, int rstride, int rx0, int ry0,
-                                                    const uint16_t *cur, int bw, int bh, int qx, int qy,
+// A ring's eight positions have three horizontal and three vertical offsets:
+// the first pass runs once per horizontal offset into LDS (strips of up to
+// `strip` rows), and each thread forms the eight second passes of its samples
+// from there.  STAGE: region and block are read once into LDS (they may be
+// mapped host memory).  LDS: 3 (strip + 9) bw first-pass values, then those.
+template <bool STAGE>
+__global__ void __launch_bounds__(256) k_subpel_one(const uint16_t *greg, int rstride, int rrows, int rx0, int ry0,
+                                                    const uint16_t *gcur, int bw, int bh, int strip, int qx, int qy,
                                                     uint32_t bestCost, int pmx, int pmy, uint32_t lambda,
                                                     uint32_t *out)
 {
-    __shared__ uint32_t red[4];
-    const int ring_x[8] = {-1, 1, 0, 0, -1, 1, -1, 1}, ring_y[8] = {0, 0, -1, 1, -1, -1, 1, 1};
+    extern __shared__ __align__(16) uint16_t smem[];
+    __shared__ uint32_t part[4][8];
+    int16_t *mid = reinterpret_cast<int16_t *>(smem);
+    const int mrows = strip + 9;
+    const uint16_t *reg = greg, *cur = gcur;
+    if (STAGE) {
+        uint16_t *s = smem + align8(3 * mrows * bw);
+        stage_packed(s, greg, rstride * rrows, gcur, bw * bh);
+        reg = s;
+        cur = s + align8(rstride * rrows);
+    }
+    __syncthreads();
+    constexpr int ring_x[8] = {-1, 1, 0, 0, -1, 1, -1, 1}, ring_y[8] = {0, 0, -1, 1, -1, -1, 1, 1};
     int mx = qx, my = qy;
     uint32_t best = bestCost;
     for (int pass = 0; pass < 2; pass++) {
-        const int step = pass == 0 ? 2 : 1;
-        const int cx = mx, cy = my;
+        const int step = pass == 0 ? 2 : 1, cx = mx, cy = my;
+        // window row of the first tap of the ring's top row, and each vertical offset's rows below it
+        const int top = ((4 * (cy - step)) >> 4) - 3 - ry0;
+        int dyr[3];
+        const int8_t *cv[3];
+#pragma unroll
+        for (int v = 0; v < 3; v++) {
+            const int y16 = 4 * (cy + (v - 1) * step);
+            dyr[v] = (y16 >> 4) - 3 - ry0 - top;
+            cv[v] = c_luma[0][y16 & 15];
+        }
+        uint32_t e[8] = {};
+        for (int y0 = 0; y0 < bh; y0 += strip) {
+            const int rows = min(strip, bh - y0), need = rows + 7 + dyr[2];
+            __syncthreads();                         // the previous strip's readers are done
+            for (int i = threadIdx.x; i < 3 * need * bw; i += 256) {
+                const int hr = i / bw, c = i - hr * bw, u = hr / need, r = hr - u * need;
+                const int x16 = 4 * (cx + (u - 1) * step);
+                mid[(u * mrows + r) * bw + c] =
+                    (int16_t)hpass<8>(reg + (top + y0 + r) * rstride + (x16 >> 4) - 3 - rx0 + c, c_luma[0][x16 & 15]);
+            }
+            __syncthreads();
+            for (int i = threadIdx.x; i < rows * bw; i += 256) {
+                const int r = i / bw, c = i - r * bw;
+                const int s = (int)cur[(y0 + r) * bw + c];
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const int u = ring_x[k] + 1, v = ring_y[k] + 1;
+                    const int16_t *m = mid + (u * mrows + r + dyr[v]) * bw + c;
+                    int acc = 0;
+#pragma unroll
+                    for (int j = 0; j < 8; j++) acc += (int)cv[v][j] * (int)m[j * bw];
+                    e[k] += (uint32_t)abs(s - vfinal_pix(acc));
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const uint32_t t = (uint32_t)group_sum<64>((int)e[k]);
+            if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6][k] = t;
+        }
+        __syncthreads();
+#pragma unroll
         for (int k = 0; k < 8; k++) {
             const int tx = cx + ring_x[k] * step, ty = cy + ring_y[k] * step;
-            const int m16x = tx * 4, m16y = ty * 4;
-            const int8_t *ch = c_luma[0][m16x & 15], *cv = c_luma[0][m16y & 15];
-            const int ix = (m16x >> 4) - 3 - rx0, iy = (m16y >> 4) - 3 - ry0;
-            uint32_t s = 0;
-            for (int i = threadIdx.x; i < bw * bh; i += blockDim.x) {
-                const int r = i / bw, c = i % bw;
-                const uint16_t *p = reg + (iy + r) * rstride + ix + c;
-                int acc = 0;
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc += (int)cv[j] * hpass<8>(p + j * rstride, ch);
-                s += (uint32_t)abs((int)cur[i] - vfinal_pix(acc));
-            }
-            const uint32_t sad = block_sum_u32(s, red);
+            const uint32_t sad = part[0][k] + part[1][k] + part[2][k] + part[3][k];
             const uint32_t cost = (sad << 8) + (eg_bits(tx - pmx) + eg_bits(ty - pmy)) * lambda;
             if (cost < best) { best = cost; mx = tx; my = ty; }
         }
+        __syncthreads();                             // the readers of part are done
     }
     if (threadIdx.x == 0) {
         out[0] = (uint32_t)mx;
@@ -412,6 +519,9 @@ __global__ void __launch_bounds__(256) k_subpel_one(const uint16_t *reg, int rst
         out[2] = best;
     }
 }
+
+// Dynamic LDS of the per-call searches.
+constexpr size_t kCallLds = 60 * 1024;         // (a 16-byte round-up more at most)
 
 static inline int clampi_h(int v, int lo, int hi) { return std::min(std::max(v, lo), hi); }
 
@@ -496,18 +606,15 @@ void Xg26xMotionEstFull(xg_me_struct *me)
         return;
     }
     const size_t wB = align_up((size_t)ws * wh * 2, 256), cB = align_up((size_t)bw * bh * 2, 256);
-    CallCtx *c = call_ctx(wB + cB + 256, wB + cB + 256);
+    CallCtx *c = call_ctx(0, wB + cB + 256);
     if (!c) return;
     pack2d(c->host, me->ref + (intptr_t)y0 * me->refStride + x0, me->refStride, ws, wh, 2);
     pack2d(c->host + wB, me->input, me->inputStride, bw, bh, 2);
-    if (!XG_HIP(hipMemcpyAsync(c->dev, c->host, wB + cB, hipMemcpyHostToDevice, c->stream))) return;
-    uint32_t *dout = (uint32_t *)(c->dev + wB + cB);
-    k_full_search_one<<<1, 256, lds, c->stream>>>((uint16_t *)c->dev, ws, wh, (uint16_t *)(c->dev + wB), bw, bh,
+    k_full_search_one<<<1, 256, lds, c->stream>>>((uint16_t *)c->view, ws, wh, (uint16_t *)(c->view + wB), bw, bh,
                                                   x0, x1, y0, y1, me->sadLambda, me->predMv.mvX,
-                                                  me->predMv.mvY, dout);
+                                                  me->predMv.mvY, (uint32_t *)(c->view + wB + cB));
     if (!XG_HIP(hipGetLastError())) return;
     uint32_t *hout = (uint32_t *)(c->host + wB + cB);
-    if (!XG_HIP(hipMemcpyAsync(hout, dout, 16, hipMemcpyDeviceToHost, c->stream))) return;
     if (!XG_HIP(hipStreamSynchronize(c->stream))) return;
     me->bestMv.mvX = (int16_t)(4 * (int)hout[0]);
     me->bestMv.mvY = (int16_t)(4 * (int)hout[1]);
@@ -528,7 +635,8 @@ void Xg26xMotionEstDia(xg_me_struct *me)
     // bounding box of every position the search may read
     int x0 = std::max(cx - me->searchWidth, mnx), x1 = std::min(cx + me->searchWidth, mxx);
     int y0 = std::max(cy - me->searchHeight, mny), y1 = std::min(cy + me->searchHeight, mxy);
-    int16_t cand[24];
+    DiaCands cands = {};
+    int16_t *cand = cands.v;
     for (uint32_t i = 0; i < me->candNum; i++) {
         const int mx = clampi_h(me->meCand[i].mvX, mnx, mxx), my = clampi_h(me->meCand[i].mvY, mny, mxy);
         cand[2 * i] = me->meCand[i].mvX;
@@ -539,20 +647,22 @@ void Xg26xMotionEstDia(xg_me_struct *me)
     }
     const int rw = x1 - x0 + bw, rh = y1 - y0 + bh;
     const size_t rB = align_up((size_t)rw * rh * 2, 256), cB = align_up((size_t)bw * bh * 2, 256);
-    CallCtx *c = call_ctx(rB + cB + 512, rB + cB + 512);
+    // what fits is read once into LDS from the mapped staging; a wider region is copied to HBM first
+    const size_t lds = ((size_t)align8(rw * rh) + (size_t)align8(bw * bh)) * 2;
+    const bool staged = lds <= kCallLds;
+    CallCtx *c = call_ctx(staged ? 0 : rB + cB + 512, rB + cB + 512);
     if (!c) return;
     pack2d(c->host, me->ref + (intptr_t)y0 * me->refStride + x0, me->refStride, rw, rh, 2);
     pack2d(c->host + rB, me->input, me->inputStride, bw, bh, 2);
-    memcpy(c->host + rB + cB, cand, sizeof(cand));
-    if (!XG_HIP(hipMemcpyAsync(c->dev, c->host, rB + cB + sizeof(cand), hipMemcpyHostToDevice, c->stream))) return;
-    uint32_t *dout = (uint32_t *)(c->dev + rB + cB + 256);
-    k_dia_one<<<1, 256, 0, c->stream>>>((uint16_t *)c->dev, rw, x0, y0, (uint16_t *)(c->dev + rB), bw, bh,
-                                        (int16_t *)(c->dev + rB + cB), (int)me->candNum, mnx, mny, mxx, mxy, cx, cy,
-                                        me->searchWidth, me->searchHeight, me->sadLambda, me->predMv.mvX,
-                                        me->predMv.mvY, dout);
+    if (!staged && !XG_HIP(hipMemcpyAsync(c->dev, c->host, rB + cB, hipMemcpyHostToDevice, c->stream))) return;
+    char *d = staged ? c->view : c->dev;
+    auto *kernel = staged ? &k_dia_one<true> : &k_dia_one<false>;
+    kernel<<<1, 256, staged ? lds : 0, c->stream>>>((uint16_t *)d, rw, rh, x0, y0, (uint16_t *)(d + rB), bw, bh,
+                                                    cands, (int)me->candNum, mnx, mny, mxx, mxy, cx,
+                                                    cy, me->searchWidth, me->searchHeight, me->sadLambda,
+                                                    me->predMv.mvX, me->predMv.mvY, (uint32_t *)(c->view + rB + cB + 256));
     if (!XG_HIP(hipGetLastError())) return;
     uint32_t *hout = (uint32_t *)(c->host + rB + cB + 256);
-    if (!XG_HIP(hipMemcpyAsync(hout, dout, 16, hipMemcpyDeviceToHost, c->stream))) return;
     if (!XG_HIP(hipStreamSynchronize(c->stream))) return;
     me->bestMv.mvX = (int16_t)(4 * (int)hout[0]);
     me->bestMv.mvY = (int16_t)(4 * (int)hout[1]);
@@ -576,17 +686,23 @@ void Xg266FullSubPelMe(xg_me_struct *me)
     const int rx0 = (qx >> 2) - 1 - 3, ry0 = (qy >> 2) - 1 - 3;
     const int rw = bw + 10, rh = bh + 10;
     const size_t rB = align_up((size_t)rw * rh * 2, 256), cB = align_up((size_t)bw * bh * 2, 256);
-    CallCtx *c = call_ctx(rB + cB + 256, rB + cB + 256);
+    // as above; the first-pass strips take what the samples leave of the LDS (at least 16 rows)
+    const size_t row = 3 * (size_t)bw * 2, samples = ((size_t)align8(rw * rh) + (size_t)align8(bw * bh)) * 2;
+    const bool staged = samples + row * (std::min(bh, 16) + 9) <= kCallLds;
+    const int strip = std::min<int>(bh, (int)((kCallLds - (staged ? samples : 0)) / row) - 9);
+    const size_t lds = align_up(row * (strip + 9), 16) + (staged ? samples : 0);
+    CallCtx *c = call_ctx(staged ? 0 : rB + cB + 256, rB + cB + 256);
     if (!c) return;
     pack2d(c->host, me->ref + (intptr_t)ry0 * me->refStride + rx0, me->refStride, rw, rh, 2);
     pack2d(c->host + rB, me->input, me->inputStride, bw, bh, 2);
-    if (!XG_HIP(hipMemcpyAsync(c->dev, c->host, rB + cB, hipMemcpyHostToDevice, c->stream))) return;
-    uint32_t *dout = (uint32_t *)(c->dev + rB + cB);
-    k_subpel_one<<<1, 256, 0, c->stream>>>((uint16_t *)c->dev, rw, rx0, ry0, (uint16_t *)(c->dev + rB), bw, bh,
-                                           qx, qy, me->bestCost, me->predMv.mvX, me->predMv.mvY, me->sadLambda, dout);
+    if (!staged && !XG_HIP(hipMemcpyAsync(c->dev, c->host, rB + cB, hipMemcpyHostToDevice, c->stream))) return;
+    char *d = staged ? c->view : c->dev;
+    auto *kernel = staged ? &k_subpel_one<true> : &k_subpel_one<false>;
+    kernel<<<1, 256, lds, c->stream>>>((uint16_t *)d, rw, rh, rx0, ry0, (uint16_t *)(d + rB), bw, bh, strip, qx, qy,
+                                       me->bestCost, me->predMv.mvX, me->predMv.mvY, me->sadLambda,
+                                       (uint32_t *)(c->view + rB + cB));
     if (!XG_HIP(hipGetLastError())) return;
     uint32_t *hout = (uint32_t *)(c->host + rB + cB);
-    if (!XG_HIP(hipMemcpyAsync(hout, dout, 12, hipMemcpyDeviceToHost, c->stream))) return;
     if (!XG_HIP(hipStreamSynchronize(c->stream))) return;
     me->bestMv.mvX = (int16_t)hout[0];
     me->bestMv.mvY = (int16_t)hout[1];
