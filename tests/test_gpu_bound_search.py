@@ -4,6 +4,7 @@ candidates left), flat noise (too many left: the exhaustive list), extreme
 samples (the largest sums), repeated texture and constant planes (ties in
 raster order), windows cut at an odd column, and rate weights past the rule."""
 import ctypes
+from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
 import pytest
@@ -43,8 +44,15 @@ def oracle_search(oracle, cur, ref, bw, bh, rng, lam, ctu, pad):
     refp = np.ascontiguousarray(np.pad(ref, pad, mode="edge"))
     mx, my = np.zeros(nb, np.int16), np.zeros(nb, np.int16)
     c, s = np.zeros(nb, np.uint32), np.zeros(nb, np.uint32)
-    oracle.or_FullSearchFrame(ptr(cur), w, ptr(refp, pad * (w + 2 * pad) + pad), w + 2 * pad, w, h, bw, bh, rng, lam, ctu,
-                              0, nb, ptr(mx), ptr(my), ptr(c), ptr(s))
+    # block ranges in threads: these are whole frames
+    step = -(-nb // 8)
+
+    def part(b0):
+        oracle.or_FullSearchFrame(ptr(cur), w, ptr(refp, pad * (w + 2 * pad) + pad), w + 2 * pad, w, h, bw, bh, rng, lam,
+                                  ctu, b0, min(nb, b0 + step), ptr(mx), ptr(my), ptr(c), ptr(s))
+
+    with ThreadPoolExecutor(8) as ex:
+        list(ex.map(part, range(0, nb, step)))
     return mx, my, c, s
 
 
@@ -54,7 +62,7 @@ def oracle_search(oracle, cur, ref, bw, bh, rng, lam, ctu, pad):
     ("half", 64, 64, 1024), ("extreme", 64, 64, 1024), ("periodic", 50, 64, 0), ("constant", 64, 31, 0)])
 def test_pipeline_full_search(oracle, kind, rng, ctu, lam):
     lib = capi.load()
-    h, w, pad = 64, 112, 152
+    h, w, pad = 496, 848, 152          # 1,643 blocks: the bounded form's sizes, CTUs cut at both edges
     planes = content(kind, h, w)
     half = lambda p: np.ascontiguousarray(p[::2, ::2])
     pics = [DevicePicture([p, half(p), half(p)], pad) for p in planes]
@@ -66,13 +74,14 @@ def test_pipeline_full_search(oracle, kind, rng, ctu, lam):
         cfg = capi.XgPipelineCfg()
         cfg.range, cfg.sadLambda, cfg.ctuSize = rng, lam, ctu
         cfg.refine = refine_cfg([(0, 0)], wl.LAMBDA_REFINE)
+        exp = [oracle_search(oracle, planes[0], planes[1 + r], 16, 16, rng, lam, ctu, pad)[:2] for r in (0, 1)]
         for mode in (capi.MODE_BATCHED, capi.MODE_GRAPH, capi.MODE_GRAPH):
             assert lib.xg_me_pipeline(s, ctypes.byref(cfg), pics[0].ref(), pics[1].ref(), pics[2].ref(), pred.ref(),
                                       mode) == 0
             full = np.zeros((nb, 2, 2), np.int16)
             assert lib.xg_me_pipeline_read(s, full.ctypes.data, None, None, None, None, None) == 0
             for r in (0, 1):
-                mx, my, _, _ = oracle_search(oracle, planes[0], planes[1 + r], 16, 16, rng, lam, ctu, pad)
+                mx, my = exp[r]
                 # the frame search reports quarter pel, the pipeline integer pel
                 assert np.array_equal(full[:, r, 0], mx >> 2) and np.array_equal(full[:, r, 1], my >> 2), (mode, r)
     finally:

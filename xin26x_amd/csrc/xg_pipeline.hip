@@ -50,6 +50,76 @@ constexpr int kPipeQuads = 3;                              // candidate quads pe
 constexpr int kPipeWinW = 2 * kPipeMaxRange + kPB + 4 * kPipeQuads + 2;   // 158
 constexpr int kPipeWinH = 2 * kPipeMaxRange + kPB + 1;    // 145: a two-row item may read one row past the window
 
+// Box sums of a plane over positions x0 .. x0 + w - 1, y0 .. y0 + h - 1: the
+// sum of the 8x8 (s8) and of the 4x4 samples (s4) from (x, y), at
+// [(y - y0) * stride + (x - x0)].  x0, w and stride even, rows of whole dwords.
+// 10-bit samples keep 8x8 sums (at most 65,472) in 16 bits.
+struct SeaPlane {
+    const uint16_t *src;           // sample (0, 0) of the plane
+    intptr_t rs;                   // its stride (even)
+    uint16_t *s8, *s4;
+    int stride;                    // sums per row
+    int x0, y0, w, h;              // covered positions; the samples read end at x0 + w + 8, y0 + h + 7
+};
+
+struct SeaPlanes {
+    SeaPlane p[2];
+};
+
+// Both sums, two columns per thread, kBoxRows rows by sliding sums: row sums of
+// 4 samples at columns +0 and +4, their 4-row sums V and V', s4 = V and
+// s8(y) = (V + V')(y) + (V + V')(y + 4).  Also clears *zero (a counter of the
+// launches that follow), when set.  Memory-bound: 2 bytes read and 4 written
+// per position.
+constexpr int kBoxRows = 32;
+
+__global__ void __launch_bounds__(256) k_box_sums(SeaPlanes pl, int *zero)
+{
+    const SeaPlane &P = pl.p[blockIdx.z];
+    if (zero && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) *zero = 0;
+    const int j = (int)(blockIdx.x * blockDim.x + threadIdx.x), r0 = (int)blockIdx.y * kBoxRows;
+    if (2 * j >= P.w) return;
+    const gdword *q = (const gdword *)(P.src + (intptr_t)P.y0 * P.rs + P.x0 + 2 * j);
+    const int sp = (int)(P.rs >> 1), op = P.stride >> 1, last = P.h - 1 + 7;
+    uint32_t *o8 = reinterpret_cast<uint32_t *>(P.s8) + j, *o4 = reinterpret_cast<uint32_t *>(P.s4) + j;
+    v2s va = {0, 0}, vb = {0, 0}, ra[4], rb[4], t[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) ra[k] = rb[k] = t[k] = (v2s){0, 0};
+    // row y of the samples completes s4 of row y - 3 and s8 of row y - 7
+    for (int y = r0; y < r0 + kBoxRows + 7 && y <= last; y += 4) {
+        uint32_t D[4][5];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+#pragma unroll
+            for (int c = 0; c < 5; c++) D[k][c] = q[(intptr_t)min(y + k, last) * sp + c];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            v2s e[4];
+#pragma unroll
+            for (int c = 0; c < 4; c++) e[c] = as_v2s(D[k][c]) + as_v2s(align16(D[k][c + 1], D[k][c], 16));
+            const v2s ha = e[0] + e[1], hb = e[2] + e[3];
+            va += ha - ra[k];
+            vb += hb - rb[k];
+            ra[k] = ha;
+            rb[k] = hb;
+            const v2s s = va + vb;
+            const int y4 = y + k - 3, y8 = y + k - 7;
+            if (y4 >= r0 && y4 < r0 + kBoxRows && y4 < P.h) o4[(size_t)y4 * op] = as_u32(va);
+            if (y8 >= r0 && y8 < r0 + kBoxRows && y8 < P.h) o8[(size_t)y8 * op] = as_u32(s + t[k]);
+            t[k] = s;
+        }
+    }
+}
+
+// One launch over n (1 or 2) planes of one size.
+inline void box_sums_enqueue(hipStream_t st, const SeaPlane *p, int n, int *zero)
+{
+    SeaPlanes a;
+    a.p[0] = p[0];
+    a.p[1] = p[n - 1];
+    k_box_sums<<<dim3((p[0].w / 2 + 255) / 256, (p[0].h + kBoxRows - 1) / kBoxRows, n), 256, 0, st>>>(a, zero);
+}
+
 // The full search of a block and reference: the lowest (cost << 32 | position)
 // costed, position (my + 128) << 8 | (mx + 128) (raster order), and how many
 // candidates the bounded search's scan left.
@@ -86,13 +156,6 @@ __device__ __forceinline__ IWin int_window(int x, int y, int fw, int fh, int ctu
     return w;
 }
 
-// v_sad_u16 on packed pairs: |a.lo - b.lo| + |a.hi - b.hi| + acc (checked on
-// gfx950: both 16-bit halves take part).
-__device__ __forceinline__ uint32_t sad2(uint32_t a, uint32_t b, uint32_t acc)
-{
-    return __builtin_amdgcn_sad_u16(a, b, acc);
-}
-
 __device__ __forceinline__ unsigned long long min_u64(unsigned long long a, unsigned long long b)
 {
     return a < b ? a : b;
@@ -106,22 +169,22 @@ __device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long k)
 }
 
 // ---------------------------------------------------------------------------
-// 1. Full search, exhaustive form: the blocks of the list a.dense (every block
-// when it is null), a workgroup per block and reference at a time
+// 1. Full search, exhaustive form: a workgroup per block and reference; LISTED:
+// those of the list a.dense, one after the other
 // ---------------------------------------------------------------------------
 // Each lane costs NQ quads (4 * NQ horizontally adjacent candidates) of one
 // search row: the window row's dwords D and their one-sample realignment F are
 // shared by all of them, so the loads and v_alignbit per v_sad_u16 fall as NQ
 // grows.
-template <int NQ>
+template <int NQ, bool LISTED>
 __global__ void __launch_bounds__(256) k_pipe_full(PipeArgs a)
 {
     __shared__ __align__(16) uint16_t win[kPipeWinH * kPipeWinW];
     __shared__ __align__(16) uint32_t curL[kPB * kPB / 2];     // packed pairs
     __shared__ unsigned long long red[4];
-    const int listed = a.dense ? a.dense[0] : 2 * a.nb;
+    const int listed = LISTED ? a.dense[0] : (int)blockIdx.x + 1;
     for (int li = blockIdx.x; li < listed; li += gridDim.x) {
-    const int id = a.dense ? a.dense[1 + li] : li;
+    const int id = LISTED ? a.dense[1 + li] : li;
     const int b = id >> 1, r = id & 1;
     const int x = (b % a.nbx) * kPB, y = (b / a.nbx) * kPB;
     const IWin w = int_window(x, y, a.fw, a.fh, a.ctu);
@@ -131,7 +194,7 @@ __global__ void __launch_bounds__(256) k_pipe_full(PipeArgs a)
     const xg_plane &RP = a.pics[r ? a.refSlot1 : a.refSlot0].plane[0];
     const xg_plane &CP = a.pics[a.curSlot].plane[0];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    __syncthreads();                                // the previous block's readers are done
+    if (LISTED) __syncthreads();                    // the previous block's readers are done
     {   // window rows (ny + 15) x (nx + 15) samples: a wave per row, lanes along it,
         // 4 rows x 3 columns of loads in flight per lane
         const int rows = ny + kPB - 1, cols = nx + kPB - 1;
@@ -451,7 +514,7 @@ __global__ void __launch_bounds__(64 * kBoundWaves) __attribute__((amdgpu_waves_
         const uint32_t kh = (uint32_t)__builtin_amdgcn_readfirstlane((int)(k >> 32)), kl = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)k);
         best = min_u64(best, ((unsigned long long)kh << 32) | kl);
     };
-    SeaColumn<8, kBoundNd> sc;
+    SeaColumn<8> sc;
     {
         uint32_t key = 0xFFFFFFFFu;
         int kpos = 0;
@@ -459,7 +522,7 @@ __global__ void __launch_bounds__(64 * kBoundWaves) __attribute__((amdgpu_waves_
         for (int i0 = 0; i0 == 0 || i0 + 32 < n2; i0 += 64) {
             const int it = min(i0 + lane, n2 - 1), k0 = item_row(it), j = it - k0 * nc, rr = 4 * k0, dx = 2 * j - p;
             uint32_t kl = 0xFFFFFFFFu, kh = 0xFFFFFFFFu;
-            sc.open(Sw, j, rr, lastRow);
+            sc.open(Sw, kBoundNd, j, rr, lastRow);
             for (int t = 0, dy = rr; t < steps; t++, dy += 16) {
                 uint32_t l0, h0, l1, h1;
                 sc.step(C8, by[dy], by[dy + 8], l0, h0, l1, h1);
@@ -518,7 +581,7 @@ __global__ void __launch_bounds__(64 * kBoundWaves) __attribute__((amdgpu_waves_
     auto scan = [&](bool in, int it, int u0, int un) {
         const int k0 = item_row(it), j = it - k0 * nc, dx = 2 * j - p;
         int dy = k0 + 16 * u0;
-        sc.open(Sw, j, dy, lastRow);
+        sc.open(Sw, kBoundNd, j, dy, lastRow);
         const uint32_t ql = bc[dx], qh = bc[dx + 1];
         for (int u = 0; u < un; u++, dy += 16) {
             uint32_t l0, h0, l1, h1;
@@ -913,6 +976,12 @@ static uint64_t hmix(uint64_t h, uint64_t v)
 // window (kBoundOver) costs more than any candidate and no sum wraps.  The
 // encoder's lambdas are below 2^19; larger ones search exhaustively.
 constexpr uint32_t kBoundLambda = 1u << 21;
+// Fewest blocks of the bounded search.  Below, the CTUs' workgroups and the short
+// waves after them leave most of the chip idle and the three launches show:
+// whole frames of 920 blocks take 122 us against 106 exhaustively at +/-24 and
+// 390 blocks 147 against 117 at +/-64; 2,040 blocks take 140 against 148 at
+// +/-16 and 188 against 398 at +/-64, 3,600 blocks 163 against 217 at +/-8.
+constexpr int kBoundBlocks = 1600;
 
 // Sum planes of both references over every position the searches read, and
 // the list of the exhaustive search.
@@ -931,7 +1000,7 @@ static bool sums_prepare(PipeState *p, const xg_plane &r0, const xg_plane &r1, i
         if (!XG_HIP(hipMalloc((void **)&p->dSums, need * sizeof(uint16_t)))) return false;
         p->sumsCap = need;
     }
-    if (!p->denseGrid) p->denseGrid = resident_slots((const void *)k_pipe_full<kPipeQuads>, 256);
+    if (!p->denseGrid) p->denseGrid = resident_slots((const void *)k_pipe_full<kPipeQuads, true>, 256);
     for (int k = 0; k < 2; k++) {
         const xg_plane &R = k ? r1 : r0;
         p->args.sums[k] = {R.data, R.stride, p->dSums + 2 * k * one, p->dSums + (2 * k + 1) * one, stride,
@@ -953,9 +1022,9 @@ static bool enqueue_pipe(const PipeState *p, hipStream_t st, xg_session *s, bool
         k_pipe_bound<<<8 * per, 64 * kBoundWaves, 0, st>>>(p->args, per);
         const int perLeft = ((2 * p->nb + 3) / 4 + 7) / 8;
         k_pipe_left<<<8 * perLeft, 256, 0, st>>>(p->args, perLeft);
-        k_pipe_full<kPipeQuads><<<std::min(2 * p->nb, p->denseGrid), 256, 0, st>>>(p->args);
+        k_pipe_full<kPipeQuads, true><<<std::min(2 * p->nb, p->denseGrid), 256, 0, st>>>(p->args);
     } else {
-        k_pipe_full<kPipeQuads><<<2 * p->nb, 256, 0, st>>>(p->args);
+        k_pipe_full<kPipeQuads, false><<<2 * p->nb, 256, 0, st>>>(p->args);
     }
     if (t3) session_timer_end(s, 3, ev);
     k_pipe_dia<<<2 * p->nb, 64, 0, st>>>(p->args);
@@ -1064,7 +1133,7 @@ int32_t xg_me_pipeline(xg_session *s, const xg_pipeline_cfg *cfg, const xg_pictu
     A.dense = nullptr;
     A.found = p->dFound;
     A.left = nullptr;
-    p->bounded = cfg->sadLambda <= kBoundLambda;
+    p->bounded = cfg->sadLambda <= kBoundLambda && nb >= kBoundBlocks;
     if (p->bounded && !sums_prepare(p, ref0->plane[0], ref1->plane[0], cfg->range, cfg->ctuSize, v.stream))
         return XG_ERR_NOMEM;
     int ev[2];
