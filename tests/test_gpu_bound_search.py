@@ -86,3 +86,50 @@ def test_pipeline_full_search(oracle, kind, rng, ctu, lam):
                 assert np.array_equal(full[:, r, 0], mx >> 2) and np.array_equal(full[:, r, 1], my >> 2), (mode, r)
     finally:
         lib.xg_session_destroy(s)
+
+
+@pytest.mark.parametrize("kind,size,bs,rng,ctu,lam,shift", [
+    ("texture", (560, 816), 16, 16, 64, 1024, 0), ("texture", (489, 485), 8, 24, 64, 1024, 1),
+    ("texture", (713, 709), 16, 32, 32, 0, 1), ("texture", (480, 480), 8, 48, 48, 500, 0),
+    ("texture", (713, 709), 16, 40, 7, 1024, 1), ("texture", (479, 800), 16, 16, 64, 1024, 0),
+    ("texture", (560, 816), 16, 15, 64, 1024, 0), ("texture", (560, 816), 16, 49, 64, 1024, 1),
+    ("texture", (28007, 24), 16, 17, 64, 1024, 1), ("texture", (13, 28004), 8, 16, 64, 1024, 0),
+    ("texture", (480, 480), 8, 16, 64, 1 << 21, 0), ("texture", (480, 480), 8, 16, 64, (1 << 21) + 1, 0),
+    ("flat", (713, 709), 16, 32, 64, 1024, 0), ("flat", (489, 485), 8, 17, 64, 0, 1), ("half", (713, 709), 16, 30, 64, 1024, 0),
+    ("extreme", (560, 816), 16, 24, 64, 1024, 0), ("extreme", (489, 485), 8, 24, 64, 1024, 1),
+    ("periodic", (480, 480), 8, 20, 64, 0, 0), ("periodic", (713, 709), 16, 31, 64, 0, 1),
+    ("constant", (560, 816), 16, 33, 13, 0, 0), ("constant", (489, 485), 8, 33, 9, 0, 1)])
+def test_frame_search(oracle, kind, size, bs, rng, ctu, lam, shift):
+    """shift: the reference plane starts at an odd sample and has an odd stride (rows of every alignment)."""
+    import torch
+    lib = capi.load()
+    h, w = size
+    pad = rng + 5
+    cur, ref, _ = content(kind, h, w)
+    refp = np.pad(ref, pad, mode="edge")
+    rs = refp.shape[1] + (1 - refp.shape[1] % 2 if shift else refp.shape[1] % 2)      # odd when shifted, else even
+    buf = np.zeros(shift + rs * refp.shape[0], np.uint16)
+    buf[shift:].reshape(refp.shape[0], rs)[:, :refp.shape[1]] = refp
+    cs = w + w % 2
+    cbuf = np.zeros((h, cs), np.uint16)
+    cbuf[:, :w] = cur
+    dr, dc = (torch.from_numpy(b.view(np.int16)).cuda() for b in (buf, cbuf))
+    pc = capi.XgPlane(dc.data_ptr(), cs, w, h, 0)
+    pr = capi.XgPlane(dr.data_ptr() + 2 * (shift + pad * rs + pad), rs, w, h, pad)
+    nb = (w // bs) * (h // bs)
+    mv = torch.zeros(2 * nb, dtype=torch.int16, device="cuda")
+    cost, sad = (torch.zeros(nb, dtype=torch.int32, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    s = ctypes.c_void_p()
+    assert lib.xg_session_create(ctypes.byref(s), 16) == 0
+    try:
+        assert lib.xg_full_search_frame(s, ctypes.byref(pc), ctypes.byref(pr), bs, bs, rng, lam, ctu, mv.data_ptr(),
+                                        cost.data_ptr(), sad.data_ptr()) == 0
+        assert lib.xg_session_sync(s) == 0
+    finally:
+        lib.xg_session_destroy(s)
+    emx, emy, ec, es = oracle_search(oracle, cur, ref, bs, bs, rng, lam, ctu, pad)
+    g = mv.cpu().numpy().reshape(nb, 2)
+    assert np.array_equal(g[:, 0], emx) and np.array_equal(g[:, 1], emy)
+    assert np.array_equal(cost.cpu().numpy().view(np.uint32), ec)
+    assert np.array_equal(sad.cpu().numpy().view(np.uint32), es)

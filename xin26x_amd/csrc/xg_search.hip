@@ -19,6 +19,7 @@
 
 #include "xg_device.hpp"
 #include "xg_runtime.hpp"
+#include "xg_sea.hpp"
 
 namespace xg {
 
@@ -278,6 +279,393 @@ __global__ void __launch_bounds__(1024) k_full_search_frame_p(FsFrameArgs a, int
             a.bestCost[b] = (uint32_t)(best >> 32);
             a.bestSad[b] = sad;
         }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Bounded frame form (8x8 and 16x16 grids): the results of k_full_search_frame
+// from block-sum bounds (xg_sea.hpp) instead of every SAD
+//
+// A workgroup of four waves takes 2 x 2 blocks, whose windows overlap almost
+// wholly: their union is staged once in LDS, and the sums of K x K samples at
+// each of its positions (K half the block side: four sub-blocks a block) are
+// formed beside it.  Each wave then searches one block alone: (1) a limit: the
+// lowest bounds of its 16 4-lane groups on some of the search rows are costed,
+// then the neighbours of the best for as long as that lowers it; (2) a scan:
+// every candidate with a bound within the limit goes to the block's list.  Then
+// all four waves cost the four lists together, from the window in LDS, so one
+// long list does not hold the workgroup; a block whose list overflows (flat
+// content) they search exhaustively.
+// Bounds are compared in units of 256 (one SAD), the two shares of the rate
+// rounded down.  Positions are dy << 8 | dx, in raster order.
+//
+// Bound by VALU issue (staging and sums about a third, the scan the rest) and,
+// on small frames, by the latency of one workgroup's phases: about 20 us for a
+// lone 16x16 search at range 16, where the exhaustive form takes 12.  Measured,
+// exhaustive then this form, several calls in flight, texture with noise:
+//   1920x1080 16x16 range 16: 108 -> 33 us; range 40: 606 -> 125; 12: 54 -> 29
+//   1920x1080 8x8 range 16: 168 -> 87; range 12: 100 -> 80; range 6: 43 -> 67
+//   832x480 16x16 range 16: 22 -> 17; range 12: 13.5 -> 15
+//   640x360 16x16 range 16: 14 -> 15; 8x8 range 16: 21 -> 15; 8x8 range 12: 14 -> 14
+//   320x320 8x8 range 16: 11 -> 12; 480x400 8x8 range 16: 18 -> 14
+// With noise of +-64, where nearly every block is searched exhaustively, 1080p
+// range 16: 16x16 109 -> 109, 8x8 168 -> 200.
+// A lone 832x480 16x16 call at range 16 takes 37 -> 40 us, 640x360 8x8 34.5 -> 33.
+// The rule: range 16 and over, and 1,750 blocks of 16x16 or 3,500 of 8x8.
+// ---------------------------------------------------------------------------
+constexpr int kSeaMinRange = 16;
+constexpr int kSeaMinWork = 28000;               // blocks times their side
+constexpr int kSeaList = 768;                    // list entries of a block
+constexpr int kSeaMaxRange = 48;
+constexpr uint32_t kSeaOver = 1u << 22;          // over any limit (a cost >> 8)
+constexpr uint32_t kSeaLambda = 1u << 21;        // past it the marks above could be undercut: exhaustive
+
+struct SeaFrameArgs {
+    FsFrameArgs f;
+    int ngx;                                     // groups per row
+    int wp, sp;                                  // LDS pitches of window and sums in dwords (odd)
+    int rows;                                    // LDS rows of the window
+    int aligned;                                 // reference rows are dword aligned
+};
+
+// LDS dwords of the window, of the sums and in all for a range
+static inline void sea_frame_lds(int bs, int range, int *wp, int *sp, int *rows, size_t *bytes)
+{
+    const int n = 2 * range + 2 * bs;            // window samples a side
+    *wp = (n / 2 + 3) | 1;
+    *sp = *wp;
+    *rows = n;
+    *bytes = ((size_t)(*wp + *sp) * n + 2 * (2 * range + 1 + 2 * bs)) * 4 + 4 * kSeaList * 2 + 4 * (size_t)bs * bs * 2 + 16;
+}
+
+template <int BS>
+__global__ void __launch_bounds__(256) k_search_bound(SeaFrameArgs a)
+{
+    constexpr int K = BS / 2, LR = BS;           // lanes that cost one candidate: a row each
+    constexpr int ND = BS / 2;
+    extern __shared__ uint32_t smem32[];
+    __shared__ unsigned long long found[4];      // lowest (cost, position) of each block
+    __shared__ int lists[4];                     // entries of each list; over kSeaList: exhaustive
+    const FsFrameArgs &f = a.f;
+    const int R = f.range, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    uint32_t *win = smem32, *S = win + a.wp * a.rows;
+    uint32_t *byq = S + a.sp * a.rows, *bxq = byq + 2 * R + 1 + 2 * BS;
+    uint32_t *curL = bxq + 2 * R + 1 + 2 * BS;   // the four blocks, BS rows of ND dwords each
+    uint16_t *list = reinterpret_cast<uint16_t *>(curL + 4 * BS * ND);
+    const int nby = f.fh / BS;
+    const int gx = (int)blockIdx.x % a.ngx, gy = (int)blockIdx.x / a.ngx;
+    const int xl = 2 * gx * BS, yl = 2 * gy * BS;
+    const int xr = min(2 * gx + 1, f.nbx - 1) * BS, yr = min(2 * gy + 1, nby - 1) * BS;
+    // the union of the windows: their starts and ends grow with the block's position
+    const int ux = max(xl - R, -f.ctu - 8), uy = max(yl - R, -f.ctu - 8);
+    const int ue = min(xr + R, f.fw + f.ctu - BS + 8) + BS, ve = min(yr + R, f.fh + f.ctu - BS + 8) + BS;   // exclusive
+    const int rows = ve - uy;
+    // dword loads start at the even column at or left of ux (it shares ux's dword)
+    const int lead = a.aligned ? (int)(((reinterpret_cast<uintptr_t>(f.ref) >> 1) + ux) & 1) : 0, cols = ue - ux + lead;
+    const uint16_t *src = f.ref + (intptr_t)uy * f.rs + ux - lead;
+    if (a.aligned) {
+        const int nd = (cols + 1) >> 1;
+        for (int r0 = wave; r0 < rows; r0 += 32)
+            for (int c = lane; c < nd; c += 64) {
+                uint32_t v[8];
+#pragma unroll
+                for (int k = 0; k < 8; k++) v[k] = *(const gdword *)(src + (intptr_t)min(r0 + 4 * k, rows - 1) * f.rs + 2 * c);
+#pragma unroll
+                for (int k = 0; k < 8; k++)
+                    if (r0 + 4 * k < rows) win[(r0 + 4 * k) * a.wp + c] = v[k];
+            }
+    } else {
+        for (int r0 = wave; r0 < rows; r0 += 32)
+            for (int c = lane; c < cols; c += 64) {
+                uint16_t v[8];
+#pragma unroll
+                for (int k = 0; k < 8; k++) v[k] = src[(intptr_t)min(r0 + 4 * k, rows - 1) * f.rs + c];
+#pragma unroll
+                for (int k = 0; k < 8; k++)
+                    if (r0 + 4 * k < rows) reinterpret_cast<uint16_t *>(win + (r0 + 4 * k) * a.wp)[c] = v[k];
+            }
+    }
+    if (tid < 2 * R + 1 + 2 * BS) {
+        byq[tid] = tid <= 2 * R ? (eg_bits(4 * (tid - R)) * f.lambda) >> 8 : kSeaOver;
+        bxq[tid] = tid >= 1 && tid <= 2 * R + 1 ? (eg_bits(4 * (tid - 1 - R)) * f.lambda) >> 8 : kSeaOver;
+    }
+    // the wave's block and the lane's row of it
+    const int bx = 2 * gx + (wave & 1), byb = 2 * gy + (wave >> 1);
+    const bool exists = bx < f.nbx && byb < nby;
+    const int x = min(bx, f.nbx - 1) * BS, y = min(byb, nby - 1) * BS;
+    uint32_t c[ND];
+    {
+        const gdword *cp = (const gdword *)(f.cur + (intptr_t)(y + lane % LR) * f.cs + x);
+#pragma unroll
+        for (int j = 0; j < ND; j++) c[j] = cp[j];
+        if (lane < LR) {
+#pragma unroll
+            for (int j = 0; j < ND; j++) curL[(wave * BS + lane) * ND + j] = c[j];
+        }
+    }
+    __syncthreads();
+    // sums of K x K samples: a column pair and a run of rows per thread, sliding
+    {
+        const int nj = (cols - K + 2) >> 1, ns = rows - K + 1;
+        const int runs = max(1, 256 / nj), len = (ns + runs - 1) / runs;
+        const int run = tid / nj, j = tid - run * nj, y0 = run * len, y1 = min(ns, y0 + len);
+        if (run < runs && y0 < y1) {
+            auto hsum = [&](int r) {
+                uint32_t D[K / 2 + 1];
+#pragma unroll
+                for (int k = 0; k <= K / 2; k++) D[k] = win[r * a.wp + j + k];
+                v2s h = {0, 0};
+#pragma unroll
+                for (int k = 0; k < K / 2; k++) h += as_v2s(D[k]) + as_v2s(align16(D[k + 1], D[k], 16));
+                return h;
+            };
+            v2s acc = {0, 0};
+            for (int r = y0; r < y0 + K - 1; r++) acc += hsum(r);
+            for (int r = y0; r < y1; r++) {
+                acc += hsum(r + K - 1);
+                S[r * a.sp + j] = as_u32(acc);
+                acc -= hsum(r);
+            }
+        }
+    }
+    __syncthreads();
+
+    // What a block's search needs to know of its window: candidate (0, 0) is
+    // column p of dword 0 of W (window) and S (sums), row 0.
+    struct View {
+        int x0, y0, nx, ny, p;
+        const uint32_t *W, *S;
+        int lastRow;
+    };
+    auto view = [&](int bxv, int byv) {
+        View v;
+        const int xv = bxv * BS, yv = byv * BS;
+        const int mnx = (int16_t)(-xv - f.ctu - 8), mny = (int16_t)(-yv - f.ctu - 8);
+        const int mxx = (int16_t)(f.fw + (f.ctu - BS + 8) - xv), mxy = (int16_t)(f.fh + (f.ctu - BS + 8) - yv);
+        v.x0 = max(-R, mnx);
+        v.y0 = max(-R, mny);
+        v.nx = min(R, mxx) - v.x0 + 1;
+        v.ny = min(R, mxy) - v.y0 + 1;
+        const int o = xv + v.x0 - ux + lead, oy = yv + v.y0 - uy;
+        v.p = o & 1;
+        v.W = win + oy * a.wp + (o >> 1);
+        v.S = S + oy * a.sp + (o >> 1);
+        v.lastRow = rows - K - oy;
+        return v;
+    };
+    // SADs of 64 / LR positions at once: the LR lanes of a group cost that group's position against the
+    // row c of the block, in every lane of it
+    auto cost_of = [&](const View &v, const uint32_t *c, int pos) {
+        const int cy = pos >> 8, cx = (pos & 255) + v.p;
+        const uint32_t *w = v.W + (cy + lane % LR) * a.wp + (cx >> 1);
+        const uint32_t sh = (uint32_t)(cx & 1) << 4;
+        uint32_t D[ND + 1], e = 0;
+#pragma unroll
+        for (int j = 0; j <= ND; j++) D[j] = w[j];
+#pragma unroll
+        for (int j = 0; j < ND; j++) e = sad2(align16(D[j + 1], D[j], sh), c[j], e);
+        e = (uint32_t)group_sum<LR>((int)e);
+        return (e << 8) + (eg_bits(4 * (v.x0 + (pos & 255))) + eg_bits(4 * (v.y0 + cy))) * f.lambda;
+    };
+    // lowest key of the groups, in every lane
+    auto lowest = [&](uint32_t cost, int pos) {
+        unsigned long long k = ((unsigned long long)cost << 32) | (uint32_t)pos;
+#pragma unroll
+        for (int m = LR; m < 64; m <<= 1) {
+            const unsigned long long q = (unsigned long long)__shfl_xor((long long)k, m, 64);
+            k = q < k ? q : k;
+        }
+        return k;
+    };
+    if (exists) {
+    // the block's four sums, a pair per row of sub-blocks: lanes 0 .. K - 1 hold the upper rows
+    uint32_t C[2];
+    {
+        int l = 0, h = 0;
+#pragma unroll
+        for (int j = 0; j < ND / 2; j++) {
+            l = dot2(c[j], 0x00010001u, l);
+            h = dot2(c[ND / 2 + j], 0x00010001u, h);
+        }
+        uint32_t v = (uint32_t)l | ((uint32_t)h << 16);              // each half at most 65,472 when summed
+        v += (uint32_t)shfl_xor<1>((int)v);
+        v += (uint32_t)shfl_xor<2>((int)v);
+        if (K == 8) v += (uint32_t)shfl_xor<4>((int)v);
+        C[0] = (uint32_t)__builtin_amdgcn_readlane((int)v, 0);
+        C[1] = (uint32_t)__builtin_amdgcn_readlane((int)v, K);
+    }
+    const View v = view(bx, byb);
+    const int nx = v.nx, ny = v.ny, p = v.p;
+    const uint32_t *by = byq + v.y0 + R, *bc = bxq + v.x0 + R + 1;
+    const int nc = (nx + p + 1) >> 1, steps = (ny + 2 * K - 1) / (2 * K);
+    const uint32_t rcp = (65536u + (uint32_t)nc - 1) / (uint32_t)nc;   // it / nc, exact for it < 1024
+    auto item_row = [&](int it) { return (int)(((uint32_t)it * rcp) >> 16); };
+    unsigned long long best = ~0ull;                 // lowest (cost, position), wave-uniform
+    auto lower = [&](uint32_t cost, int pos) {
+        const unsigned long long k = lowest(cost, pos);
+        const uint32_t kh = (uint32_t)__builtin_amdgcn_readfirstlane((int)(k >> 32)),
+                       kl = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)k);
+        const unsigned long long u = ((unsigned long long)kh << 32) | kl;
+        best = u < best ? u : best;
+    };
+    SeaColumn<K> sc;
+    {
+        uint32_t key = 0xFFFFFFFFu;
+        int kpos = 0;
+        const int n2 = 2 * nc;                       // rows 0 and K / 2 modulo K
+        for (int i0 = 0; i0 == 0 || i0 + 32 < n2; i0 += 64) {
+            const int it = min(i0 + lane, n2 - 1), k0 = item_row(it), j = it - k0 * nc, rr = (K / 2) * k0, dx = 2 * j - p;
+            uint32_t kl = 0xFFFFFFFFu, kh = 0xFFFFFFFFu;
+            sc.open(v.S, a.sp, j, rr, v.lastRow);
+            for (int t = 0, dy = rr; t < steps; t++, dy += 2 * K) {
+                uint32_t l0, h0, l1, h1;
+                sc.step(C, by[dy], by[dy + K], l0, h0, l1, h1);
+                kl = min(min(kl, (l0 << 5) | (uint32_t)(2 * t)), (l1 << 5) | (uint32_t)(2 * t + 1));
+                kh = min(min(kh, (h0 << 5) | (uint32_t)(2 * t)), (h1 << 5) | (uint32_t)(2 * t + 1));
+            }
+            kl += bc[dx] << 5;
+            kh += bc[dx + 1] << 5;
+            const uint32_t k = min(kl, kh);
+            const int px = min(max(dx + (kh < kl), 0), nx - 1), py = min(rr + K * (int)(k & 31u), ny - 1);
+            kpos = k < key ? py << 8 | px : kpos;
+            key = min(key, k);
+        }
+        // the lowest of each 4 lanes, costed 64 / LR at a time
+        const unsigned long long m = __ballot(key == min4(key));
+        const int low = __shfl(kpos, (lane & 60) + __ffs((int)((m >> (lane & 60)) & 15)) - 1, 64);
+#pragma unroll
+        for (int k = 0; k < LR / 4; k++) {
+            const int pos = __shfl(low, (lane / LR) * LR + 4 * k, 64);
+            lower(cost_of(v, c, pos), pos);
+        }
+        for (int k = 0; k < 8; k++) {
+            const int bp = (int)(uint32_t)best, g = (lane / LR) & 3;
+            const int ax = min(max((bp & 255) + (g == 2) - (g == 3), 0), nx - 1);
+            const int ay = min(max((bp >> 8) + (g == 0) - (g == 1), 0), ny - 1);
+            lower(cost_of(v, c, ay << 8 | ax), ay << 8 | ax);
+            if ((int)(uint32_t)best == bp) break;
+        }
+    }
+
+    uint16_t *mine = list + wave * kSeaList;
+    const uint32_t limit = (uint32_t)(best >> 40);
+    int n = 0;
+    const int items = K * nc, rem = items & 63;
+    const bool spread = 2 * ((rem * steps + 63) >> 6) < steps;
+    const int whole = spread ? items - rem : items, tasks = spread ? rem * steps : 0;
+    for (int i0 = 0; i0 < whole + tasks && n <= kSeaList; i0 += 64) {
+        const int i = i0 + lane;
+        int it, u0 = 0;
+        bool in;
+        if (i0 < whole) {                            // whole rounds first: whole is a multiple of 64 when tasks follow
+            it = min(i, items - 1);
+            in = i < whole;
+        } else {
+            const int t = i - whole, k = min(t / steps, rem - 1);
+            it = whole + k;
+            u0 = min(t - k * steps, steps - 1);
+            in = t < tasks;
+        }
+        const int un = i0 < whole ? steps : 1;
+        const int k0 = item_row(it), j = it - k0 * nc, dx = 2 * j - p;
+        int dy = k0 + 2 * K * u0;
+        sc.open(v.S, a.sp, j, dy, v.lastRow);
+        const uint32_t ql = bc[dx], qh = bc[dx + 1];
+        for (int u = 0; u < un; u++, dy += 2 * K) {
+            uint32_t l0, h0, l1, h1;
+            sc.step(C, by[dy], by[dy + K], l0, h0, l1, h1);
+            if (!__any((int)min(l0, l1) <= (int)(limit - ql) || (int)min(h0, h1) <= (int)(limit - qh))) continue;
+            auto push = [&](uint32_t q, int ddx, int ddy) {
+                const bool ok = in && q <= limit && ddx >= 0 && ddx < nx && ddy < ny;
+                const unsigned long long m = __ballot(ok);
+                if (!m) return;
+                const int at = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                if (ok && at < kSeaList) mine[at] = (uint16_t)(ddy << 8 | ddx);
+                n += __popcll(m);
+            };
+            push(l0 + ql, dx, dy);
+            push(h0 + qh, dx + 1, dy);
+            push(l1 + ql, dx, dy + K);
+            push(h1 + qh, dx + 1, dy + K);
+        }
+    }
+    if (lane == 0) {
+        found[wave] = best;
+        lists[wave] = n;
+    }
+    } else if (lane == 0) {
+        lists[wave] = 0;
+    }
+    __syncthreads();
+
+    // all waves: every block's list, or every candidate of a block whose list overflowed
+    for (int q = 0; q < 4; q++) {
+        const int n = lists[q];
+        if (!n) continue;
+        const View v = view(2 * gx + (q & 1), 2 * gy + (q >> 1));
+        const uint32_t *cl = curL + q * BS * ND;
+        unsigned long long k = ~0ull;
+        if (n <= kSeaList) {
+            const uint32_t *cr = cl + (lane % LR) * ND;
+#pragma unroll
+            for (int j = 0; j < ND; j++) c[j] = cr[j];
+            for (int i = wave * (64 / LR); i < n; i += 4 * (64 / LR)) {
+                const int pos = list[q * kSeaList + min(i + lane / LR, n - 1)];
+                const unsigned long long o = ((unsigned long long)cost_of(v, c, pos) << 32) | (uint32_t)pos;
+                k = o < k ? o : k;
+            }
+        } else {
+            // four adjacent candidates of a row a thread, which come in raster order: strict < keeps the earliest
+            const int nq = (v.nx + v.p + 3) >> 2;
+            uint32_t bcst = 0xFFFFFFFFu;
+            int bpos = 0;
+            for (int it = tid; it < v.ny * nq; it += 256) {
+                const int dy = it / nq, qd = it - dy * nq;
+                const uint32_t *w = v.W + dy * a.wp + 2 * qd;
+                uint32_t acc[4] = {0, 0, 0, 0};
+#pragma unroll 2
+                for (int r = 0; r < BS; r++) {
+                    uint32_t D[ND + 2];
+#pragma unroll
+                    for (int j = 0; j < ND + 2; j++) D[j] = w[r * a.wp + j];
+#pragma unroll
+                    for (int j = 0; j < ND; j++) {
+                        const uint32_t cj = cl[r * ND + j];
+                        acc[0] = sad2(D[j], cj, acc[0]);
+                        acc[1] = sad2(align16(D[j + 1], D[j], 16), cj, acc[1]);
+                        acc[2] = sad2(D[j + 1], cj, acc[2]);
+                        acc[3] = sad2(align16(D[j + 2], D[j + 1], 16), cj, acc[3]);
+                    }
+                }
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    const int dx = 4 * qd + m - v.p;
+                    const uint32_t cost = (acc[m] << 8) + (eg_bits(4 * (v.x0 + dx)) + eg_bits(4 * (v.y0 + dy))) * f.lambda;
+                    if (dx >= 0 && dx < v.nx && cost < bcst) {
+                        bcst = cost;
+                        bpos = dy << 8 | dx;
+                    }
+                }
+            }
+            k = ((unsigned long long)bcst << 32) | (uint32_t)bpos;
+        }
+#pragma unroll
+        for (int m = 1; m < 64; m <<= 1) {
+            const unsigned long long o = (unsigned long long)__shfl_xor((long long)k, m, 64);
+            k = o < k ? o : k;
+        }
+        if (lane == 0) atomicMin(&found[q], k);
+    }
+    __syncthreads();
+    if (exists && lane == 0) {
+        const View v = view(bx, byb);
+        const unsigned long long best = found[wave];
+        const int b = byb * f.nbx + bx, pos = (int)(uint32_t)best, mx = v.x0 + (pos & 255), my = v.y0 + (pos >> 8);
+        const uint32_t cost = (uint32_t)(best >> 32);
+        f.bestMv[2 * b] = (int16_t)(4 * mx);
+        f.bestMv[2 * b + 1] = (int16_t)(4 * my);
+        f.bestCost[b] = cost;
+        f.bestSad[b] = (cost - (eg_bits(4 * mx) + eg_bits(4 * my)) * f.lambda) >> 8;
     }
 }
 
@@ -797,9 +1185,21 @@ int32_t xg::full_search_frame_on(hipStream_t st, xg_session *timer, const xg_pla
     a.fw = cur->width; a.fh = cur->height; a.bw = bw; a.bh = bh; a.range = range; a.ctu = ctuSize; a.nbx = nbx;
     a.lambda = sadLambda;
     a.bestMv = bestMv; a.bestCost = bestCost; a.bestSad = bestSad;
+    SeaFrameArgs b;
+    size_t seaLds = 0;
+    sea_frame_lds(bw, range, &b.wp, &b.sp, &b.rows, &seaLds);
+    const bool bounded = bw == bh && (bw == 8 || bw == 16) && packed && range >= kSeaMinRange && range <= kSeaMaxRange &&
+                         (int64_t)nbx * nby * bw >= kSeaMinWork && seaLds <= 64 * 1024 && sadLambda <= kSeaLambda;
     int ev[2];
     const bool timed = timer && session_timer_begin(timer, 3, ev);
-    if (packed) {
+    if (bounded) {
+        b.f = a;
+        b.ngx = (nbx + 1) / 2;
+        b.aligned = (a.rs & 1) == 0;
+        const int groups = b.ngx * ((nby + 1) / 2);
+        if (bw == 8) k_search_bound<8><<<groups, 256, seaLds, st>>>(b);
+        else k_search_bound<16><<<groups, 256, seaLds, st>>>(b);
+    } else if (packed) {
         const int threads = packed_threads(nxm, kFrameK);
         if (bw == 8)
             k_full_search_frame_p<8><<<nbx * nby, threads, ldsP, st>>>(a, wsP);
