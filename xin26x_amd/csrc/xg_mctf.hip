@@ -22,13 +22,16 @@
 //     MVs x 2), full resolution (16x16, +/-5, x 2), then 8x8 blocks at full
 //     resolution (range 0, lower MVs x 1, fractional rounds).
 //
-// Mapping: one 64-lane workgroup per block.  Candidates are costed one by one
-// from a staged (bs + 7)^2 window with the two-pass filter (exact for integer
-// MVs too); the integer search stages its (2 range + bs)^2 window once and
-// each lane costs raster positions, reduced by a 64-bit (SSD << 32 | index)
-// minimum; each fractional round gives one position to each of 49 lanes,
-// which filters its block column by column from one staged window that
-// covers both rounds.
+// Mapping: one 64-lane workgroup per block, templated on the block side.  A
+// 3x3-and-zero candidate set of integer MVs is costed with a lane per row (four
+// or eight candidates at once, straight from the reference); sets with a
+// fractional MV one by one from a staged (bs + 7)^2 window with the two-pass
+// filter.  The integer search stages its (2 range + bs)^2 window once and each
+// lane costs raster positions; the fractional rounds are described at frac_round.
+//
+// Bound by VALU issue.  1920x1080, before -> now: the 8x8 level with its two
+// fractional rounds 280 -> 93 us (49.5 M vector instructions, which take 81 us to
+// issue), the three 16x16 levels 41 -> 23 us on average.
 #include <algorithm>
 #include <mutex>
 #include <vector>
@@ -41,13 +44,15 @@ namespace xg {
 constexpr int kMctfMaxRange = 8;
 constexpr int kMctfMaxBs = 16;
 
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 struct MctfArgs {
     const uint16_t *cur;
     intptr_t cs;
     const uint16_t *ref;
     intptr_t rs;
     int w, h, pad;
-    int bs, range, frac, factor;
+    int range, rcp, factor;        // rcp: 65536 / (2 range + 1) rounded up, so (p * rcp) >> 16 divides p <= 288
     const int2 *lower;
     int lowerBw, lowerBh;
     int2 *mv;
@@ -55,25 +60,27 @@ struct MctfArgs {
     int nbx;
 };
 
-// Shared first pass of a fractional round of 8x8 blocks: 7 horizontal
-// offsets x 16 row pairs x 8 columns, each dword the first-pass values of two
-// consecutive window rows (low half the upper row) of one column.
-constexpr int kMctfFracBs = 8;
-constexpr int kMctfFracPairs = kMctfFracBs + 8;    // rows bs + 7 + up to 2 of spread, as pairs
+// LDS windows are staged shifted, so that column 0 is their first sample
+// whatever its address; rows are an odd number of dwords apart.
+constexpr int kWinRows = 2 * kMctfMaxRange + kMctfMaxBs;    // 32, also >= bs + 10 of a fractional round
+constexpr int kWinDw = kWinRows / 2;                        // dwords staged of a row at most
+constexpr int kWinPitch = 19;
 
+template <int BS>
 struct MctfLds {
-    uint16_t win[(2 * kMctfMaxRange + kMctfMaxBs) * (2 * kMctfMaxRange + kMctfMaxBs)];  // 32 x 32
-    int16_t tmp[(kMctfMaxBs + 7) * kMctfMaxBs];
-    uint16_t blk[kMctfMaxBs * kMctfMaxBs];
+    uint32_t win[kWinRows * kWinPitch];
+    uint32_t blk[BS * BS / 2];                              // the current block, BS / 2 dwords a row
+    int16_t tmp[(BS + 7) * BS];
 };
 
 // Whether the 8-tap reach of a prediction at MV (mx, my) for the block at
 // (x, y) stays inside the reference's padding.
+template <int BS>
 __device__ __forceinline__ bool mctf_valid(const MctfArgs &a, int x, int y, int mx, int my)
 {
     const int px = x + (mx >> 4), py = y + (my >> 4);
-    return px - 3 >= -a.pad && py - 3 >= -a.pad && px + a.bs + 4 <= a.w - 1 + a.pad &&
-           py + a.bs + 4 <= a.h - 1 + a.pad;
+    return px - 3 >= -a.pad && py - 3 >= -a.pad && px + BS + 4 <= a.w - 1 + a.pad &&
+           py + BS + 4 <= a.h - 1 + a.pad;
 }
 
 // A reference sample with its coordinates kept inside the padded plane
@@ -85,277 +92,351 @@ __device__ __forceinline__ uint16_t ref_at(const MctfArgs &a, int x, int y)
     return a.ref[(intptr_t)y * a.rs + x];
 }
 
-__device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long k)
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v)
 {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kHalfMirror = 0x141, kRor4 = 0x124, kRor8 = 0x128;
+
+// Lowest value of the wave, in every lane: 16-lane rows by DPP, then the four rows as scalars.
+__device__ __forceinline__ uint32_t wave_min(uint32_t v)
+{
+    v = min(v, dpp<kXor1>(v));
+    v = min(v, dpp<kXor2>(v));
+    v = min(v, dpp<kRor4>(v));
+    v = min(v, dpp<kRor8>(v));
+    const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), r1 = (uint32_t)__builtin_amdgcn_readlane((int)v, 16),
+                   r2 = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), r3 = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    return min(min(r0, r1), min(r2, r3));
+}
+
+// Sum over aligned groups of 8 or 16 lanes, in every lane of the group.
+template <int G>
+__device__ __forceinline__ uint32_t row_sum(uint32_t v)
+{
+    static_assert(G == 8 || G == 16, "lanes of a DPP row");
+    v += dpp<kXor1>(v);
+    v += dpp<kXor2>(v);
+    v += dpp<kHalfMirror>(v);                    // quads are uniform by now
+    if constexpr (G == 16) v += dpp<kRor8>(v);
+    return v;
+}
+
+// The sample pair at p (any sample alignment).  Reads only dwords that hold one of the two samples.
+__device__ __forceinline__ uint32_t load_pair(const uint16_t *p)
+{
+    const uint32_t odd = (uint32_t)((uintptr_t)p >> 1) & 1;
+    const gdword *g = (const gdword *)((uintptr_t)p & ~(uintptr_t)3);
+    return align16(g[odd], g[0], odd << 4);
+}
+
+// Stages the window of 2 wd x rows samples at picture position (px, py); wd <= kWinDw.
+template <int BS>
+__device__ __forceinline__ void stage_window(const MctfArgs &a, MctfLds<BS> &L, int px, int py, int wd, int rows)
+{
+    const int lane = threadIdx.x, c = lane & (kWinDw - 1), r0 = lane / kWinDw;
+    constexpr int STEP = 64 / kWinDw, N = kWinRows / STEP;
+    __syncthreads();
+    if (px >= -a.pad && py >= -a.pad && px + 2 * wd <= a.w + a.pad && py + rows <= a.h + a.pad) {
+        const uint16_t *g = a.ref + (intptr_t)(py + r0) * a.rs + px + 2 * c;
+        uint32_t v[N];
 #pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-        const unsigned long long o = (unsigned long long)__shfl_xor((long long)k, m, 64);
-        k = o < k ? o : k;
+        for (int k = 0; k < N; k++) {
+            if (c < wd && r0 + k * STEP < rows) v[k] = load_pair(g);
+            g += STEP * a.rs;
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            if (c < wd && r0 + k * STEP < rows) L.win[(r0 + k * STEP) * kWinPitch + c] = v[k];
+    } else if (c < wd) {
+        for (int r = r0; r < rows; r += STEP)
+            L.win[r * kWinPitch + c] = pack16(ref_at(a, px + 2 * c, py + r), ref_at(a, px + 2 * c + 1, py + r));
     }
-    return k;
+    __syncthreads();
 }
 
 // SSD of the block (staged in L.blk) against the prediction at MV (mx, my),
 // computed by the whole wave; UINT32_MAX when the position is not costed.
-__device__ uint32_t mctf_candidate(const MctfArgs &a, MctfLds &L, int x, int y, int mx, int my)
+template <int BS>
+__device__ __forceinline__ uint32_t mctf_candidate(const MctfArgs &a, MctfLds<BS> &L, int x, int y, int mx, int my)
 {
-    if (!mctf_valid(a, x, y, mx, my)) return 0xFFFFFFFFu;
-    const int lane = threadIdx.x, bs = a.bs, ww = bs + 7;
-    const int px = x + (mx >> 4) - 3, py = y + (my >> 4) - 3;
+    if (!mctf_valid<BS>(a, x, y, mx, my)) return 0xFFFFFFFFu;
+    const int lane = threadIdx.x;
     const int8_t *hf = taps_for<8>(mx & 15, 0), *vf = taps_for<8>(my & 15, 0);
-    __syncthreads();
-    for (int i = lane; i < ww * ww; i += 64) {
-        const int r = i / ww, c = i - r * ww;
-        L.win[r * 32 + c] = ref_at(a, px + c, py + r);
-    }
-    __syncthreads();
-    for (int i = lane; i < ww * bs; i += 64) {
-        const int r = i / bs, c = i - r * bs;
-        L.tmp[r * kMctfMaxBs + c] = (int16_t)hpass<8>(&L.win[r * 32 + c], hf);
-    }
+    stage_window(a, L, x + (mx >> 4) - 3, y + (my >> 4) - 3, (BS + 8) / 2, BS + 7);
+    const uint16_t *w = reinterpret_cast<const uint16_t *>(L.win), *blk = reinterpret_cast<const uint16_t *>(L.blk);
+    for (int i = lane; i < (BS + 7) * BS; i += 64)
+        L.tmp[i] = (int16_t)hpass<8>(&w[i / BS * 2 * kWinPitch + i % BS], hf);
     __syncthreads();
     uint32_t e = 0;
-    for (int i = lane; i < bs * bs; i += 64) {
-        const int r = i / bs, c = i - r * bs;
+    for (int i = lane; i < BS * BS; i += 64) {
         int s = 0;
 #pragma unroll
-        for (int k = 0; k < 8; k++) s += (int)vf[k] * (int)L.tmp[(r + k) * kMctfMaxBs + c];
-        const int d = (int)L.blk[r * kMctfMaxBs + c] - vfinal_pix(s);
+        for (int k = 0; k < 8; k++) s += (int)vf[k] * (int)L.tmp[i + k * BS];
+        const int d = (int)blk[i] - vfinal_pix(s);
         e += (uint32_t)(d * d);
     }
     return (uint32_t)group_sum<64>((int)e);
 }
 
-// FRAC: the finest level's fractional rounds (a separate instantiation, so the
-// integer levels keep the register budget of their own code).
 // SSD of the staged block against the window at (dx, dy) on packed pairs: the
 // window pairs realigned by one sample for odd dx (alignbit by 16 dx & 16; an
-// even dx also reads the dword past its last pair, inside the LDS struct, and
-// shifts it out), each pair difference squared and summed by one v_dot2.
+// even dx also reads the dword past its last pair, inside the window's pitch,
+// and shifts it out), each pair difference squared and summed by one v_dot2.
 template <int BS>
-__device__ __forceinline__ uint32_t int_ssd(const MctfLds &L, int dx, int dy)
+__device__ __forceinline__ uint32_t int_ssd(const MctfLds<BS> &L, int dx, int dy)
 {
-    const uint32_t *w32 = reinterpret_cast<const uint32_t *>(L.win) + (dx >> 1);
-    const uint32_t *b32 = reinterpret_cast<const uint32_t *>(L.blk);
+    const uint32_t *w = L.win + dy * kWinPitch + (dx >> 1), *b = L.blk;
     const uint32_t sh = (uint32_t)(dx & 1) << 4;
     int e = 0;
 #pragma unroll 4
     for (int r = 0; r < BS; r++) {
-        const uint32_t *wr = w32 + (dy + r) * 16, *br = b32 + r * (kMctfMaxBs / 2);
 #pragma unroll
         for (int j = 0; j < BS / 2; j++) {
-            const v2s d = as_v2s(br[j]) - as_v2s(align16(wr[j + 1], wr[j], sh));
+            const v2s d = as_v2s(b[r * (BS / 2) + j]) - as_v2s(align16(w[r * kWinPitch + j + 1], w[r * kWinPitch + j], sh));
             e = dot2(as_u32(d), as_u32(d), e);
         }
     }
     return (uint32_t)e;
 }
 
-template <bool FRAC>
-__global__ void __launch_bounds__(64) k_mctf_level(MctfArgs a)
+// One fractional round: the 7x7 positions around (ox, oy), step sixteenths
+// apart, from the window staged at (x0, y0) (picture coordinates).  Lane
+// (i, c) = (lane / 8, lane % 8) takes horizontal offset i and column c (and
+// c + 8 of a 16-wide block): it filters its column once into packed row pairs
+// in registers, and from these forms the prediction at all seven vertical
+// offsets, whose taps and first rows are the same in every lane.  So no
+// first-pass value goes through LDS, and 56 lanes of 64 work (a lane per
+// position leaves 49, each of which reads every first-pass value again).
+// Lane (i, j) ends with position (j, i)'s SSD.  Taps and offsets are scaled as
+// in pack_mid16 and clip_hi16.
+template <int BS>
+__device__ __forceinline__ uint32_t frac_round(const MctfLds<BS> &L, int ox, int oy, int step, int rx, int ry)
 {
-    __shared__ MctfLds L;
-    const int lane = threadIdx.x, bs = a.bs;
-    const int bx = (int)blockIdx.x % a.nbx, by = (int)blockIdx.x / a.nbx;
-    const int x = bx * bs, y = by * bs;
-    for (int i = lane; i < bs * bs; i += 64) {
-        const int r = i / bs, c = i - r * bs;
-        L.blk[r * kMctfMaxBs + c] = a.cur[(intptr_t)(y + r) * a.cs + x + c];
+    const int lane = threadIdx.x, i = min(lane >> 3, 6), c = lane & 7;
+    const int mx = ox + (i - 3) * step;
+    const int col = (mx >> 4) - 3 - rx + c, top = (oy - 3 * step) >> 4;
+    const bool odd = col & 1;
+    uint32_t T[5];                                    // tap pairs against the dwords from the one with the first tap
+    {
+        const int8_t *hf = c_luma[0][mx & 15];
+        uint32_t A[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) A[j] = pack16(64 * hf[2 * j], 64 * hf[2 * j + 1]);
+        T[0] = odd ? A[0] << 16 : A[0];
+#pragma unroll
+        for (int j = 1; j < 4; j++) T[j] = odd ? align16(A[j], A[j - 1], 16) : A[j];
+        T[4] = odd ? A[3] >> 16 : 0;
     }
-    __syncthreads();
+    const uint16_t *blk = reinterpret_cast<const uint16_t *>(L.blk);
+    uint32_t mine = 0;
+#pragma unroll 1
+    for (int h = 0; h < BS / 8; h++) {
+        const uint32_t *q = L.win + (top - 3 - ry) * kWinPitch + (col >> 1) + 4 * h;
+        uint32_t P[BS + 8], cur[BS / 2];              // P[r]: first-pass rows r and r + 1
+#pragma unroll
+        for (int r = 0; r < BS; r += 2) cur[r / 2] = pack16(blk[r * BS + 8 * h + c], blk[(r + 1) * BS + 8 * h + c]);
+        int last = 0;
+#pragma unroll
+        for (int r = 0; r <= BS + 8; r++) {
+            int u = dot2_first(q[r * kWinPitch], T[0], kHRound64);
+#pragma unroll
+            for (int j = 1; j < 5; j++) u = dot2(q[r * kWinPitch + j], T[j], u);
+            if (r) P[r - 1] = pack_mid16(last, u);
+            last = u;
+            if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // no more than four rows' reads in flight: registers
+        }
+        int at = top;                                 // integer row of P[0]'s first tap, 3 above
+#pragma unroll 1                                    // one copy of the shift and of the second pass: registers
+        for (int j = 0; j < 7; j++) {
+            const int my = oy + (j - 3) * step;
+            if ((my >> 4) != at) {                    // uniform, at most twice a round
+#pragma unroll
+                for (int r = 0; r < BS + 7; r++) P[r] = P[r + 1];
+                at++;
+                asm volatile("");                     // stays a branch: as selects it would cost every offset
+            }
+            const int8_t *vf = c_luma[0][my & 15];
+            uint32_t V[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) V[k] = ((uint32_t)(64 * vf[2 * k]) & 0xFFFF) | (uint32_t)(64 * vf[2 * k + 1]) << 16;   // scalars
+            int acc = 0;
+#pragma unroll
+            for (int r = 0; r < BS; r += 2) {
+                int s0 = dot2_first(P[r], V[0], 0), s1 = dot2_first(P[r + 1], V[0], 0);
+#pragma unroll
+                for (int k = 1; k < 4; k++) {
+                    s0 = dot2(P[r + 2 * k], V[k], s0);
+                    s1 = dot2(P[r + 1 + 2 * k], V[k], s1);
+                }
+                const v2s d = as_v2s(cur[r / 2]) - as_v2s(pack_hi16(clip_hi16(s0), clip_hi16(s1)));
+                acc = dot2(as_u32(d), as_u32(d), acc);
+            }
+            const uint32_t sum = row_sum<8>((uint32_t)acc);
+            mine += c == j ? sum : 0;
+        }
+    }
+    return mine;
+}
+
+// FRAC: the finest level's fractional rounds (a separate instantiation, so the
+// integer levels keep the register budget of their own code).
+template <int BS, bool FRAC>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(FRAC && BS == 16 ? 4 : FRAC ? 6 : 8)))
+k_mctf_level(MctfArgs a)
+{
+    __shared__ MctfLds<BS> L;
+    const int lane = threadIdx.x;
+    const int by = (int)blockIdx.x / a.nbx, bx = (int)blockIdx.x - by * a.nbx;
+    const int x = bx * BS, y = by * BS;
+    constexpr int CPR = 64 / BS, NR = (10 + CPR - 1) / CPR;   // candidates at once, rounds of them
+    const int row = lane % BS;
+    {
+        constexpr int N = (BS * BS / 2 + 63) / 64;
+        uint32_t v[N];
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const int i = lane + 64 * k, r = i / (BS / 2), c = i % (BS / 2);
+            if (i < BS * BS / 2) v[k] = load_pair(a.cur + (intptr_t)(y + r) * a.cs + x + 2 * c);
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++)
+            if (lane + 64 * k < BS * BS / 2) L.blk[lane + 64 * k] = v[k];
+    }
     uint32_t best = 0xFFFFFFFFu;
     int bmx = 0, bmy = 0;
     // candidates: the 3x3 lower-level MVs (rows then columns), then zero
     if (a.lower) {
-        int cxs[10], cys[10];
-        bool has[10], allInt = true;
+        int cx[NR], cy[NR];                                   // the lane's candidate of each round
+        bool has[NR], allInt = true;
 #pragma unroll
-        for (int k = 0; k < 10; k++) {
-            int cx = 0, cy = 0;
-            has[k] = true;
-            if (k < 9) {
-                const int tx = bx / 2 + k % 3 - 1, ty = by / 2 + k / 3 - 1;
-                has[k] = tx >= 0 && ty >= 0 && tx < a.lowerBw && ty < a.lowerBh;
-                if (has[k]) {
-                    const int2 m = a.lower[(intptr_t)ty * a.lowerBw + tx];
-                    cx = m.x * a.factor;
-                    cy = m.y * a.factor;
-                }
+        for (int t = 0; t < NR; t++) {
+            const int k = t * CPR + lane / BS, ky = (k * 11) >> 5, kx = k - 3 * ky;   // k / 3 for k < 16
+            const int tx = bx / 2 + kx - 1, ty = by / 2 + ky - 1;
+            cx[t] = cy[t] = 0;
+            has[t] = k == 9 || (k < 9 && tx >= 0 && ty >= 0 && tx < a.lowerBw && ty < a.lowerBh);
+            if (has[t] && k < 9) {
+                const int2 m = a.lower[(intptr_t)ty * a.lowerBw + tx];
+                cx[t] = m.x * a.factor;
+                cy[t] = m.y * a.factor;
             }
-            cxs[k] = cx;
-            cys[k] = cy;
-            allInt = allInt && (!has[k] || ((cx | cy) & 15) == 0);
+            allInt = allInt && ((cx[t] | cy[t]) & 15) == 0;
         }
-        if (allInt) {
+        __syncthreads();
+        if (__all(allInt)) {
             // integer positions (the lower levels' MVs, scaled, always are): the prediction is the
-            // reference itself, so every lane loads its samples of all ten positions at once and
-            // the SSDs need no staging
-            constexpr int SPL = kMctfMaxBs * kMctfMaxBs / 64;
-            bool ok[10];
-            uint16_t v[10][SPL];
+            // reference itself; a lane takes one row of one candidate, all loads before the first use.
+            // A costed position has 3 samples of margin, so the dwords around its rows are in the plane.
+            uint32_t D[NR][BS / 2 + 1], sh[NR], e[NR], lo = 0xFFFFFFFFu;
 #pragma unroll
-            for (int k = 0; k < 10; k++) {
-                ok[k] = has[k] && mctf_valid(a, x, y, cxs[k], cys[k]);
-                const uint16_t *rp = a.ref + (intptr_t)(y + (cys[k] >> 4)) * a.rs + x + (cxs[k] >> 4);
+            for (int t = 0; t < NR; t++) {
+                has[t] = has[t] && mctf_valid<BS>(a, x, y, cx[t], cy[t]);
+                if (has[t]) {
+                    const uint16_t *p = a.ref + (intptr_t)(y + (cy[t] >> 4) + row) * a.rs + x + (cx[t] >> 4);
+                    const gdword *g = (const gdword *)((uintptr_t)p & ~(uintptr_t)3);
+                    sh[t] = ((uint32_t)(uintptr_t)p & 2) << 3;
 #pragma unroll
-                for (int t = 0; t < SPL; t++) {
-                    const int i = lane + 64 * t, r = i / bs, c = i - r * bs;
-                    v[k][t] = (ok[k] && i < bs * bs) ? rp[(intptr_t)r * a.rs + c] : (uint16_t)0;
+                    for (int j = 0; j <= BS / 2; j++) D[t][j] = g[j];
                 }
             }
 #pragma unroll
-            for (int k = 0; k < 10; k++) {
-                int e = 0;
+            for (int t = 0; t < NR; t++) {
+                int s = 0;
 #pragma unroll
-                for (int t = 0; t < SPL; t++) {
-                    const int i = lane + 64 * t, r = i / bs, c = i - r * bs;
-                    if (i < bs * bs) {
-                        const int d = (int)L.blk[r * kMctfMaxBs + c] - (int)v[k][t];
-                        e += d * d;
-                    }
+                for (int j = 0; j < BS / 2; j++) {
+                    const v2s d = as_v2s(L.blk[row * (BS / 2) + j]) - as_v2s(align16(D[t][j + 1], D[t][j], sh[t]));
+                    s = dot2(as_u32(d), as_u32(d), s);
                 }
-                e = group_sum<64>(e);
-                if (ok[k] && (uint32_t)e < best) {
-                    best = (uint32_t)e;
-                    bmx = cxs[k];
-                    bmy = cys[k];
+                e[t] = row_sum<BS>((uint32_t)s);
+                if (!has[t]) e[t] = 0xFFFFFFFFu;
+                lo = min(lo, e[t]);
+            }
+            best = wave_min(lo);
+            if (best != 0xFFFFFFFFu) {
+                // the first candidate with it
+                bool found = false;
+#pragma unroll
+                for (int t = 0; t < NR; t++) {
+                    const unsigned long long m = __ballot(e[t] == best);
+                    if (m && !found) {
+                        found = true;
+                        const int l = __builtin_ctzll(m);
+                        bmx = __builtin_amdgcn_readlane(cx[t], l);
+                        bmy = __builtin_amdgcn_readlane(cy[t], l);
+                    }
                 }
             }
         } else {
+#pragma unroll 1
             for (int k = 0; k < 10; k++) {
-                if (!has[k]) continue;
-                const uint32_t e = mctf_candidate(a, L, x, y, cxs[k], cys[k]);
+                int sx = cx[0], sy = cy[0];
+                bool sh = has[0];
+#pragma unroll
+                for (int t = 1; t < NR; t++)
+                    if (k / CPR == t) {
+                        sx = cx[t];
+                        sy = cy[t];
+                        sh = has[t];
+                    }
+                const int l = k % CPR * BS;
+                if (!__builtin_amdgcn_readlane((int)sh, l)) continue;
+                sx = __builtin_amdgcn_readlane(sx, l);
+                sy = __builtin_amdgcn_readlane(sy, l);
+                const uint32_t e = (uint32_t)uniform((int)mctf_candidate(a, L, x, y, sx, sy));
                 if (e < best) {
                     best = e;
-                    bmx = cxs[k];
-                    bmy = cys[k];
+                    bmx = sx;
+                    bmy = sy;
                 }
             }
         }
     }
-    // integer search +/-range around the best (C division: toward zero)
-    {
-        const int R = a.range, ix = bmx / 16, iy = bmy / 16, ww = 2 * R + bs;
-        __syncthreads();
-        for (int i = lane; i < ww * ww; i += 64) {
-            const int r = i / ww, c = i - r * ww;
-            L.win[r * 32 + c] = ref_at(a, x + ix - R + c, y + iy - R + r);
+    // integer search +/-range around the best (C division: toward zero); with range 0 around an
+    // integer MV that was costed there is nothing new to cost
+    if (a.range > 0 || best == 0xFFFFFFFFu || ((bmx | bmy) & 15)) {
+        const int R = a.range, ix = bmx / 16, iy = bmy / 16, n1 = 2 * R + 1;
+        stage_window(a, L, x + ix - R, y + iy - R, R + BS / 2, 2 * R + BS);
+        uint32_t lo = 0xFFFFFFFFu, lp = 0xFFFFFFFFu;
+        for (int p = lane; p < n1 * n1; p += 64) {
+            const int dy = (p * a.rcp) >> 16, dx = p - dy * n1;
+            if (!mctf_valid<BS>(a, x, y, 16 * (ix - R + dx), 16 * (iy - R + dy))) continue;
+            const uint32_t e = int_ssd(L, dx, dy);
+            if (e < lo) {
+                lo = e;
+                lp = (uint32_t)p;
+            }
         }
-        __syncthreads();
-        const int n = (2 * R + 1) * (2 * R + 1);
-        unsigned long long k = ~0ull;
-        for (int p = lane; p < n; p += 64) {
-            const int dy = p / (2 * R + 1), dx = p - dy * (2 * R + 1);
-            if (!mctf_valid(a, x, y, 16 * (ix - R + dx), 16 * (iy - R + dy))) continue;
-            const uint32_t e = bs == 16 ? int_ssd<16>(L, dx, dy) : int_ssd<8>(L, dx, dy);
-            const unsigned long long kk = ((unsigned long long)e << 32) | (uint32_t)p;
-            k = kk < k ? kk : k;
-        }
-        k = wave_min_u64(k);
-        if (k != ~0ull && (uint32_t)(k >> 32) < best) {
-            const int p = (int)(uint32_t)k, dy = p / (2 * R + 1), dx = p - dy * (2 * R + 1);
-            best = (uint32_t)(k >> 32);
+        const uint32_t m = wave_min(lo);
+        if (m < best) {
+            const int p = (int)wave_min(lo == m ? lp : 0xFFFFFFFFu), dy = (p * a.rcp) >> 16, dx = p - dy * n1;
+            best = m;
             bmx = 16 * (ix - R + dx);
             bmy = 16 * (iy - R + dy);
         }
     }
     // fractional rounds: 7x7 at quarter-pel steps, then 7x7 at 1/16 pel
     if constexpr (FRAC) {
-        __shared__ uint32_t hp[7][kMctfFracPairs][kMctfFracBs];
-        const int x0 = ((bmx - 15) >> 4) - 3, y0 = ((bmy - 15) >> 4) - 3;   // window covering both rounds
-        const int ww = ((bmx + 15) >> 4) - ((bmx - 15) >> 4) + bs + 7;
-        const int wh = ((bmy + 15) >> 4) - ((bmy - 15) >> 4) + bs + 7;
-        __syncthreads();
-        for (int i = lane; i < ww * wh; i += 64) {
-            const int r = i / ww, c = i - r * ww;
-            L.win[r * 32 + c] = ref_at(a, x + x0 + c, y + y0 + r);
-        }
-        __syncthreads();
+        const int rx = ((bmx - 15) >> 4) - 3, ry = ((bmy - 15) >> 4) - 3;   // window covering both rounds
+        stage_window(a, L, x + rx, y + ry, (((bmx + 15) >> 4) - ((bmx - 15) >> 4) + BS + 8) / 2,
+                     ((bmy + 15) >> 4) - ((bmy - 15) >> 4) + BS + 7);
+#pragma unroll 1
         for (int step = 4; step >= 1; step -= 3) {
-            const int ox = bmx, oy = bmy;
-            unsigned long long k = ~0ull;
-            if (bs == kMctfFracBs) {
-                // the first pass of each of the 7 horizontal offsets, once for the 7 positions
-                // that share it: rows from the highest position's first tap row (spread <= 2)
-                const int rb = ((oy - 3 * step) >> 4) - 3 - y0;
-                const int nr = ((oy + 3 * step) >> 4) - 3 - y0 - rb + bs + 7;
-                __syncthreads();                      // earlier readers of hp are done
-                for (int t = lane; t < 7 * nr * bs; t += 64) {
-                    const int i = t / (nr * bs), rc = t - i * (nr * bs), r = rc / bs, c = rc - r * bs;
-                    const int mx = ox + (i - 3) * step;
-                    const int cx = (mx >> 4) - 3 - x0;
-                    const int u = hpass<8>(&L.win[(rb + r) * 32 + cx + c], taps_for<8>(mx & 15, 0));
-                    uint16_t *h = reinterpret_cast<uint16_t *>(&hp[i][0][0]);
-                    if (r < kMctfFracPairs) h[2 * (r * kMctfFracBs + c)] = (uint16_t)u;             // pair (r, r + 1)
-                    if (r >= 1) h[2 * ((r - 1) * kMctfFracBs + c) + 1] = (uint16_t)u;               // pair (r - 1, r)
-                }
-                __syncthreads();
-                if (lane < 49) {
-                    const int i = lane % 7, mx = ox + (i - 3) * step, my = oy + (lane / 7 - 3) * step;
-                    if (mctf_valid(a, x, y, mx, my)) {
-                        // second pass with the taps x 64 and the rounding offset x 64: clamped to
-                        // [0, (1023 << 16) | 0xFFFF], the upper half of the sum is the clipped sample,
-                        // and two columns' samples pack into one dword for a packed difference
-                        const int8_t *vf = taps_for<8>(my & 15, 0);
-                        uint32_t vt[4];
-#pragma unroll
-                        for (int j = 0; j < 4; j++) vt[j] = pack16(64 * vf[2 * j], 64 * vf[2 * j + 1]);
-                        const int r0 = (my >> 4) - 3 - y0 - rb;      // the position's first tap row in hp
-                        const uint32_t *b32 = reinterpret_cast<const uint32_t *>(L.blk);
-                        int e = 0;
-#pragma unroll
-                        for (int r = 0; r < kMctfFracBs; r++)
-#pragma unroll
-                            for (int c = 0; c < kMctfFracBs; c += 2) {
-                                int s0 = dot2_first(hp[i][r0 + r][c], vt[0], kVOffset << 6);
-                                int s1 = dot2_first(hp[i][r0 + r][c + 1], vt[0], kVOffset << 6);
-#pragma unroll
-                                for (int j = 1; j < 4; j++) {
-                                    s0 = dot2(hp[i][r0 + r + 2 * j][c], vt[j], s0);
-                                    s1 = dot2(hp[i][r0 + r + 2 * j][c + 1], vt[j], s1);
-                                }
-                                const v2s d = as_v2s(b32[(r * kMctfMaxBs + c) >> 1]) -
-                                              as_v2s(pack_hi16(clip_hi16(s0), clip_hi16(s1)));
-                                e = dot2(as_u32(d), as_u32(d), e);
-                            }
-                        k = ((unsigned long long)(uint32_t)e << 32) | (uint32_t)lane;
-                    }
-                }
-            } else if (lane < 49) {
-                const int mx = ox + (lane % 7 - 3) * step, my = oy + (lane / 7 - 3) * step;
-                if (mctf_valid(a, x, y, mx, my)) {
-                    const int8_t *hf = taps_for<8>(mx & 15, 0), *vf = taps_for<8>(my & 15, 0);
-                    const int cx = (mx >> 4) - 3 - x0, cy = (my >> 4) - 3 - y0;   // window offset of the first tap
-                    uint32_t e = 0;
-                    for (int c = 0; c < bs; c++) {
-                        int t[kMctfMaxBs + 7];
-#pragma unroll
-                        for (int r = 0; r < kMctfMaxBs + 7; r++)
-                            if (r < bs + 7) t[r] = hpass<8>(&L.win[(cy + r) * 32 + cx + c], hf);
-                        for (int r = 0; r < bs; r++) {
-                            int s = 0;
-#pragma unroll
-                            for (int j = 0; j < 8; j++) s += (int)vf[j] * t[r + j];
-                            const int d = (int)L.blk[r * kMctfMaxBs + c] - vfinal_pix(s);
-                            e += (uint32_t)(d * d);
-                        }
-                    }
-                    k = ((unsigned long long)e << 32) | (uint32_t)lane;
-                }
-            }
-            k = wave_min_u64(k);
-            if (k != ~0ull && (uint32_t)(k >> 32) < best) {
-                const int p = (int)(uint32_t)k;
-                best = (uint32_t)(k >> 32);
-                bmx = ox + (p % 7 - 3) * step;
-                bmy = oy + (p / 7 - 3) * step;
+            const int ox = bmx, oy = bmy, i = lane >> 3, j = lane & 7;
+            const uint32_t f = frac_round(L, ox, oy, step, rx, ry);
+            const bool ok = i < 7 && j < 7 && mctf_valid<BS>(a, x, y, ox + (i - 3) * step, oy + (j - 3) * step);
+            const uint32_t e = ok ? f : 0xFFFFFFFFu, m = wave_min(e);
+            if (m < best) {
+                const int p = (int)wave_min(e == m ? (uint32_t)(7 * j + i) : 0xFFFFFFFFu), pj = (p * 37) >> 8;   // p / 7
+                best = m;
+                bmx = ox + (p - 7 * pj - 3) * step;
+                bmy = oy + (pj - 3) * step;
             }
         }
     }
     if (lane == 0) {
-        const intptr_t b = (intptr_t)by * a.nbx + bx;
-        a.mv[b] = make_int2(bmx, bmy);
-        a.err[b] = best;
+        a.mv[blockIdx.x] = make_int2(bmx, bmy);
+        a.err[blockIdx.x] = best;
     }
 }
 
@@ -393,9 +474,8 @@ int32_t level_launch(hipStream_t st, const xg_plane *cur, const xg_plane *ref, i
     a.w = cur->width;
     a.h = cur->height;
     a.pad = ref->pad;
-    a.bs = bs;
     a.range = range;
-    a.frac = frac;
+    a.rcp = (65536 + 2 * range) / (2 * range + 1);
     a.factor = factor;
     a.lower = (const int2 *)lower;
     a.lowerBw = lowerBw;
@@ -405,8 +485,13 @@ int32_t level_launch(hipStream_t st, const xg_plane *cur, const xg_plane *ref, i
     a.nbx = cur->width / bs;
     const int n = a.nbx * (cur->height / bs);
     if (n <= 0) return XG_OK;
-    if (frac) k_mctf_level<true><<<n, 64, 0, st>>>(a);
-    else k_mctf_level<false><<<n, 64, 0, st>>>(a);
+    if (bs == 8) {
+        if (frac) k_mctf_level<8, true><<<n, 64, 0, st>>>(a);
+        else k_mctf_level<8, false><<<n, 64, 0, st>>>(a);
+    } else {
+        if (frac) k_mctf_level<16, true><<<n, 64, 0, st>>>(a);
+        else k_mctf_level<16, false><<<n, 64, 0, st>>>(a);
+    }
     return XG_HIP(hipGetLastError()) ? XG_OK : XG_ERR_HIP;
 }
 
