@@ -21,7 +21,7 @@ constexpr int kVOffset = (1 << (kVShift - 1)) + (8192 << 6);
 // includes this header.  [fi][phase][tap]: fi 0 default, 1 with the
 // alternative half-pel filter at phase 8, 2 the 4x4-affine variant
 // (h266_core/source/h266_luma_mc.c:27-70, selection rule :117-128).
-static __constant__ int8_t c_luma[3][16][8] = {
+static __constant__ constexpr int8_t c_luma[3][16][8] = {
     {{0, 0, 0, 64, 0, 0, 0, 0}, {0, 1, -3, 63, 4, -2, 1, 0}, {-1, 2, -5, 62, 8, -3, 1, 0},
      {-1, 3, -8, 60, 13, -4, 1, 0}, {-1, 4, -10, 58, 17, -5, 1, 0}, {-1, 4, -11, 52, 26, -8, 3, -1},
      {-1, 3, -9, 47, 31, -10, 4, -1}, {-1, 4, -11, 45, 34, -10, 4, -1}, {-1, 4, -11, 40, 40, -11, 4, -1},
@@ -42,7 +42,7 @@ static __constant__ int8_t c_luma[3][16][8] = {
      {0, 1, -2, 4, 63, -3, 1, 0}}};
 
 // h266_core/source/h266_chroma_mc.c:26-60
-static __constant__ int8_t c_chroma[32][4] = {
+static __constant__ constexpr int8_t c_chroma[32][4] = {
     {0, 64, 0, 0}, {-1, 63, 2, 0}, {-2, 62, 4, 0}, {-2, 60, 7, -1}, {-2, 58, 10, -2},
     {-3, 57, 12, -2}, {-4, 56, 14, -2}, {-4, 55, 15, -2}, {-4, 54, 16, -2}, {-5, 53, 18, -2},
     {-6, 52, 20, -2}, {-6, 49, 24, -3}, {-6, 46, 28, -4}, {-5, 44, 29, -4}, {-4, 42, 30, -4},
@@ -104,6 +104,25 @@ __device__ __forceinline__ int group_sum(int v)
     if constexpr (G >= 32) v += shfl_xor<16>(v);
     if constexpr (G >= 64) v += shfl_xor<32>(v);
     return v;
+}
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kHalfMirror = 0x141, kRor4 = 0x124, kRor8 = 0x128;
+
+// Lowest value of the wave, in every lane: 16-lane rows by DPP, then the four rows as scalars.
+__device__ __forceinline__ uint32_t wave_min(uint32_t v)
+{
+    v = min(v, dpp<kXor1>(v));
+    v = min(v, dpp<kXor2>(v));
+    v = min(v, dpp<kRor4>(v));
+    v = min(v, dpp<kRor8>(v));
+    const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), r1 = (uint32_t)__builtin_amdgcn_readlane((int)v, 16),
+                   r2 = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), r3 = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+    return min(min(r0, r1), min(r2, r3));
 }
 
 // One butterfly stage of a Walsh-Hadamard transform across lanes: the lane

@@ -92,25 +92,6 @@ __device__ __forceinline__ uint16_t ref_at(const MctfArgs &a, int x, int y)
     return a.ref[(intptr_t)y * a.rs + x];
 }
 
-template <int CTRL>
-__device__ __forceinline__ uint32_t dpp(uint32_t v)
-{
-    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
-}
-constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kHalfMirror = 0x141, kRor4 = 0x124, kRor8 = 0x128;
-
-// Lowest value of the wave, in every lane: 16-lane rows by DPP, then the four rows as scalars.
-__device__ __forceinline__ uint32_t wave_min(uint32_t v)
-{
-    v = min(v, dpp<kXor1>(v));
-    v = min(v, dpp<kXor2>(v));
-    v = min(v, dpp<kRor4>(v));
-    v = min(v, dpp<kRor8>(v));
-    const uint32_t r0 = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), r1 = (uint32_t)__builtin_amdgcn_readlane((int)v, 16),
-                   r2 = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), r3 = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
-    return min(min(r0, r1), min(r2, r3));
-}
-
 // Sum over aligned groups of 8 or 16 lanes, in every lane of the group.
 template <int G>
 __device__ __forceinline__ uint32_t row_sum(uint32_t v)

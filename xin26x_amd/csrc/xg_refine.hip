@@ -60,16 +60,10 @@ constexpr int kNumShapes = 25;     // (lgW-2)*5 + (lgH-2), W, H in 4..64
 constexpr int kPicSlots = kSessionPicSlots;
 constexpr int kRegions = 8;        // picture bands of the batched form: at most one per XCD of the MI355X
 
-struct RefineArgs {
+// A list (its blocks, tasks, outputs) and what all lists of a launch share.
+struct RefineArgs : RefineList {
     const xg_picture *pics;
-    const xg_block *blocks;
-    const int2 *tasks;             // x: block index, y: c0 | (count << 16)
-    int taskBegin, taskEnd;        // this launch's task range
-    const int *wgBegin;            // batched mode: task range [wgBegin[g], wgBegin[g+1]) of workgroup g
-    uint32_t *candCost;
-    xg_block_result *best;
-    unsigned long long *bestKey;   // per block: min over tasks of (cost << 32 | cand); all-ones when idle
-    int *done;                     // per block: candidates costed so far; 0 when idle
+    int taskBegin, taskEnd;        // this launch's task range (plain form)
     int ncand;
     int offMinX, offMaxX, offMinY, offMaxY;
     uint32_t lambda;
@@ -78,8 +72,6 @@ struct RefineArgs {
     const int16_t *off;            // device: offx[XG_MAX_CAND] then offy[XG_MAX_CAND]
     int doMc;                      // 0: costs only (tile timing), no block completion or MC
     const xg_picture *predTab;     // per picture slot: prediction planes (unpadded) the MC writes
-    int2 *mvField;                 // when set: the winner's MV is also written to every 4x4 unit
-    int mvStride;                  //   of the block in this field (units per row)
 };
 
 // CU MV window in 1/16 pel (h266_enc_init.c:1462-1465, int16 as stored there).
@@ -96,23 +88,50 @@ __device__ __forceinline__ MvWin mv_window(const xg_block &B, int fw, int fh, in
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return min(max(v, lo), hi); }
 
-// Task, block, list and picture descriptors are the same for every lane, but
-// the kernel also stores to global memory, so they are loaded into vector
-// registers.  Read back through readfirstlane they live in scalar registers,
-// and so does every address and loop bound derived from them.
+// Task, block, list and picture descriptors are the same for every lane, and
+// nothing the kernel stores: read through the constant address space they are
+// scalar loads into scalar registers, and so is every address and loop bound
+// derived from them.
 template <class T>
 __device__ __forceinline__ T uniform_load(const T *p)
 {
     static_assert(sizeof(T) % 4 == 0, "descriptor of whole dwords");
     constexpr int N = sizeof(T) / 4;
+    const __attribute__((address_space(4))) uint32_t *q = (const __attribute__((address_space(4))) uint32_t *)(uintptr_t)p;
     uint32_t w[N];
-    __builtin_memcpy(w, p, sizeof(T));
 #pragma unroll
-    for (int k = 0; k < N; k++) w[k] = (uint32_t)__builtin_amdgcn_readfirstlane((int)w[k]);
+    for (int k = 0; k < N; k++) w[k] = q[k];
     T out;
     __builtin_memcpy(&out, w, sizeof(T));
     return out;
 }
+
+// Arguments, lists and picture descriptors, read field by field where they
+// are used: held as a whole in scalar registers they made these spill (about
+// 200 lane writes and reads a task).  fresh() hides a pointer's history, so
+// that fields are read again instead of kept across it.
+template <class T>
+using ConstPtr = const __attribute__((address_space(4))) T *;
+typedef ConstPtr<xg_picture> PicPtr;
+typedef ConstPtr<RefineArgs> ArgPtr;
+typedef ConstPtr<RefineList> ListPtr;
+template <class P>
+__device__ __forceinline__ P fresh(P p)
+{
+    asm volatile("" : "+s"(p));
+    return p;
+}
+// The lane, with its history hidden: what a stage derives from it is computed
+// there, and not for every block shape ahead of the task loop.
+__device__ __forceinline__ int lane_here()
+{
+    int l = (int)threadIdx.x;
+    asm volatile("" : "+v"(l));
+    return l;
+}
+__device__ __forceinline__ PicPtr pic_ptr(const xg_picture *p) { return (PicPtr)(uintptr_t)p; }
+// The launch's arguments (every kernel's first parameter is RefineArgs).
+__device__ __forceinline__ ArgPtr args_ptr() { return (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr(); }
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
@@ -229,20 +248,33 @@ struct RefineLds {
 // odd (D[0] holds the sample left of it), s0 = D.B and s1 = D.A'.  The
 // vertical pass uses the first TAPS / 2 pairs of A.
 template <int TAPS>
-__device__ __forceinline__ uint32_t tap_row(const int8_t *c, int row, int j)
+constexpr uint32_t tap_row(const int8_t *c, int row, int j)
 {
     constexpr int H = TAPS / 2;
-    if (row == 0) return j < H ? pack16(64 * c[2 * j], 64 * c[2 * j + 1]) : 0u;
-    if (row == 1) return pack16(j == 0 ? 0 : 64 * c[2 * j - 1], j == H ? 0 : 64 * c[2 * j]);
-    return j == 0 ? 0u : pack16(64 * c[2 * j - 2], 64 * c[2 * j - 1]);
+    const int lo = row == 0 ? (j < H ? 2 * j : -1) : row == 1 ? 2 * j - 1 : 2 * j - 2, hi = lo + 1;
+    const int l = lo >= 0 && lo < TAPS ? 64 * c[lo] : 0, h = hi >= 0 && hi < TAPS && !(row == 0 && j == H) ? 64 * c[hi] : 0;
+    return ((uint32_t)l & 0xFFFFu) | (uint32_t)h << 16;
 }
+// The tables as every workgroup copies them (computing them from the taps took
+// about 500 vector instructions a workgroup).
+struct TapTables {
+    uint32_t l[16 * 15], c[32 * 9];
+};
+constexpr TapTables tap_tables()
+{
+    TapTables t{};
+    for (int i = 0; i < 16 * 15; i++) t.l[i] = tap_row<8>(c_luma[0][i / 15], (i % 15) / 5, i % 5);
+    for (int i = 0; i < 32 * 9; i++) t.c[i] = tap_row<4>(c_chroma[i / 9], (i % 9) / 3, i % 3);
+    return t;
+}
+static __constant__ TapTables c_taps = tap_tables();
 
-__device__ __forceinline__ void lds_init(RefineLds &L, const RefineArgs &a)
+__device__ __forceinline__ void lds_init(RefineLds &L, ArgPtr a)
 {
     const int lane = threadIdx.x;
-    for (int i = lane; i < 16 * 15; i += 64) L.tapL[i] = tap_row<8>(c_luma[0][i / 15], (i % 15) / 5, i % 5);
-    for (int i = lane; i < 32 * 9; i += 64) L.tapC[i] = tap_row<4>(c_chroma[i / 9], (i % 9) / 3, i % 3);
-    for (int i = lane; i < 2 * XG_MAX_CAND; i += 64) L.off[i] = a.off[i];
+    for (int i = lane; i < 16 * 15; i += 64) L.tapL[i] = c_taps.l[i];
+    for (int i = lane; i < 32 * 9; i += 64) L.tapC[i] = c_taps.c[i];
+    for (int i = lane; i < 2 * XG_MAX_CAND; i += 64) L.off[i] = a->off[i];
     __syncthreads();
 }
 
@@ -502,7 +534,7 @@ __device__ __forceinline__ void luma_task(const xg_block &B, const MvWin &mw, co
                                           uint32_t *csum)
 {
     constexpr int LN = W / 2, CP = 64 / LN;
-    const int lane = threadIdx.x, m = lane & (LN - 1), u = lane / LN;
+    const int lane = lane_here(), m = lane & (LN - 1), u = (unsigned)lane / LN;
     for (int base = 0; base < nc; base += CP) {
         const int ci = base + u;
         const int c = c0 + min(ci, nc - 1);
@@ -524,7 +556,7 @@ __device__ __forceinline__ void chroma_task(const xg_block &B, const MvWin &mw, 
                                             int oy, int c0, int nc, uint32_t *csum)
 {
     constexpr int LN = WC / 2 > 0 ? WC / 2 : 1, UP = 64 / LN;
-    const int lane = threadIdx.x, m = lane & (LN - 1), u = lane / LN;
+    const int lane = lane_here(), m = lane & (LN - 1), u = (unsigned)lane / LN;
     for (int base = 0; base < 2 * nc; base += UP) {
         const int ui = base + u;
         const int ci = ui >> 1, pl = ui & 1;
@@ -540,47 +572,45 @@ __device__ __forceinline__ void chroma_task(const xg_block &B, const MvWin &mw, 
     }
 }
 
-// Dword pointer to sample (x, y) of a plane; x even.
-__device__ __forceinline__ const gdword *plane_dw(const xg_plane &pl, int x, int y)
-{
-    return (const gdword *)(pl.data + (intptr_t)y * pl.stride + x);
-}
-
 // Global -> LDS copy plan of one plane's window: `rows` rows of `wd` dwords
-// (wd <= 64) from s (row pitch sp dwords) to d (row pitch dp dwords).  Lane
-// (c, r0) = (lane % wd, lane / wd) copies column c of rows r0, r0 + per, ...
-// (per = 64 / wd rows at a time).  Loads go in batches of 8 per lane, all
-// issued before the batch's first store, and a lane loads only its own rows.
+// (wd <= 32) from column x (even) and row y of the plane to d (row pitch dp
+// dwords).  Lane (r0, c) = (lane >> lg, lane & (1 << lg) - 1) copies column c
+// of rows r0, r0 + step, ..., lg the smallest of 3, 4, 5 that spans a row.  A
+// lane's byte offset stays the same; the base moves by scalar additions.
 struct StagePlan {
-    const gdword *s;     // the lane's first source dword
+    const char *s;       // base of the rows of one step (uniform)
+    intptr_t sstep;      // bytes to the next (uniform)
+    uint32_t soff;       // the lane's byte offset
     uint32_t *d;         // its first LDS dword
-    intptr_t sstep;      // source dwords from one of its rows to the next
-    int dstep;           // LDS dwords likewise
-    int n;               // its rows
-    int batches;         // batches of the lanes with the most rows (wave-uniform)
+    int dstep;           // LDS dwords from one of its rows to the next
+    int step;            // rows at once (uniform)
+    int left;            // rows from the lane's first on, none past the columns
+    int batches;         // batches of 8 steps (uniform)
 };
 
-__device__ __forceinline__ StagePlan stage_plan(uint32_t *d, int dp, const gdword *s, intptr_t sp, int rows, int wd)
+__device__ __forceinline__ StagePlan stage_plan(uint32_t *d, int dp, PicPtr pic, int plane, int x, int y, int rows, int wd)
 {
-    const int per = 64 / wd, c = (int)threadIdx.x % wd, r0 = (int)threadIdx.x / wd;
+    const int lane = lane_here(), lg = wd <= 8 ? 3 : wd <= 16 ? 4 : 5, c = lane & ((1 << lg) - 1), r0 = lane >> lg;
     StagePlan P;
-    P.s = s + (intptr_t)r0 * sp + c;
+    P.step = 64 >> lg;
+    const intptr_t stride = pic->plane[plane].stride;
+    P.s = (const char *)(pic->plane[plane].data + (intptr_t)y * stride + x);
+    P.sstep = (intptr_t)P.step * stride * 2;
+    P.soff = (uint32_t)r0 * (uint32_t)(stride * 2) + 4 * (uint32_t)c;
     P.d = d + r0 * dp + c;
-    P.sstep = (intptr_t)per * sp;
-    P.dstep = per * dp;
-    P.n = r0 < per && r0 < rows ? (rows - r0 + per - 1) / per : 0;
-    P.batches = ((rows + per - 1) / per + 7) / 8;
+    P.dstep = P.step * dp;
+    P.left = c < wd ? rows - r0 : 0;
+    P.batches = (rows + 8 * P.step - 1) >> (9 - lg);
     return P;
 }
 
 __device__ __forceinline__ void stage_load(const StagePlan &P, int k, uint32_t *v)
 {
-    const gdword *g = P.s + (intptr_t)(8 * k) * P.sstep;
+    const char *g = P.s + (intptr_t)(8 * k) * P.sstep;
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        if (8 * k + j < P.n) v[j] = *g;
+        if ((8 * k + j) * P.step < P.left) v[j] = *(const gdword *)(g + P.soff);
         g += P.sstep;
-        asm volatile("" : "+v"(g));              // one 64-bit add per row, no offsets held per row
     }
 }
 
@@ -588,47 +618,69 @@ __device__ __forceinline__ void stage_store(const StagePlan &P, int k, const uin
 {
 #pragma unroll
     for (int j = 0; j < 8; j++)
-        if (8 * k + j < P.n) P.d[(8 * k + j) * P.dstep] = v[j];
+        if ((8 * k + j) * P.step < P.left) P.d[(8 * k + j) * P.dstep] = v[j];
 }
 
-// Motion compensation of one plane from its LDS window: lanes [lane0,
-// lane0 + nlanes) split the W x H block into row groups of W / 2 lanes; each
-// lane forms columns 2m, 2m+1 of its rows and stores them as one dword.
+// Motion compensation of one plane from its LDS window: the caller's 2^lgN
+// lanes split the W x H block (powers of two) into row groups of W / 2 lanes;
+// lane lid of them forms columns 2m, 2m+1 of its rows, with the arithmetic of
+// interp_satd_pass, and stores them as one dword.
 template <int TAPS>
-__device__ __forceinline__ void mc_pass(const uint32_t *win, int ls, int wx, int wy, const uint32_t *hp, int fy, int W,
-                                        int H, uint16_t *dst, intptr_t ds, int lane0, int nlanes)
+__device__ __forceinline__ void mc_pass(const uint32_t *win, int ls, int wx, int wy, const uint32_t *hp,
+                                        const uint32_t *vp, int W, int H, uint16_t *dst, intptr_t ds, int lid, int lgN)
 {
-    const int lid = (int)threadIdx.x - lane0;
-    const int LN = W > 2 ? W >> 1 : 1;
-    const int groups = min(nlanes / LN, H);
-    const int m = lid & (LN - 1), g = lid / LN;
-    if (lid < 0 || lid >= nlanes || g >= groups) return;
-    const int rows = H / groups, y0 = g * rows;
-    int vc[TAPS];
-    const int8_t *cv = taps_for<TAPS>(fy, 0);
-#pragma unroll
-    for (int j = 0; j < TAPS; j++) vc[j] = cv[j];
-    int t0[TAPS], t1[TAPS];
-    const int base = (wy + y0) * ls + wx + 2 * m;
+    const int lgL = 30 - __builtin_clz((unsigned)W), lgH = 31 - __builtin_clz((unsigned)H);   // lanes a row, rows
+    const int lgG = min(lgN - lgL, lgH), rows = H >> lgG;
+    const int m = lid & ((1 << lgL) - 1), g = lid >> lgL, y0 = g * rows;
+    if (g >> lgG) return;
     HTaps<TAPS> ht;
+    const int base = (wy + y0) * ls + wx + 2 * m;
     ht.load(hp, base & 1);
+    uint32_t vt[TAPS / 2];
 #pragma unroll
-    for (int k = 0; k < TAPS - 1; k++) hrow2<TAPS>(win, base + k * ls, ht, t0[k], t1[k]);
+    for (int j = 0; j < TAPS / 2; j++) vt[j] = vp[j];
+    const uint32_t *q = win + (base >> 1);
+    uint32_t P0[TAPS - 1], P1[TAPS - 1];            // first-pass rows k and k + 1 of the two columns
+    int l0 = 0, l1 = 0;
+#pragma unroll
+    for (int k = 0; k < TAPS; k++) {
+        HRow<TAPS> h;
+        int b0, b1;
+        h.fetch(q);
+        q += ls >> 1;
+        h.sums(ht, b0, b1);
+        if (k) {
+            P0[k - 1] = pack_mid16(l0, b0);
+            P1[k - 1] = pack_mid16(l1, b1);
+        }
+        l0 = b0;
+        l1 = b1;
+    }
     uint16_t *o = dst + (intptr_t)y0 * ds + 2 * m;
-    for (int y = 0; y < rows; y++) {
-        hrow2<TAPS>(win, base + (y + TAPS - 1) * ls, ht, t0[TAPS - 1], t1[TAPS - 1]);
-        int s0 = 0, s1 = 0;                         // offset-free second pass (kHRound)
+    for (int y = 0;;) {
+        int s0 = dot2_first(P0[0], vt[0], 0), s1 = dot2_first(P1[0], vt[0], 0);
 #pragma unroll
-        for (int j = 0; j < TAPS; j++) {
-            s0 += vc[j] * t0[j];
-            s1 += vc[j] * t1[j];
+        for (int j = 1; j < TAPS / 2; j++) {
+            s0 = dot2(P0[2 * j], vt[j], s0);
+            s1 = dot2(P1[2 * j], vt[j], s1);
         }
-        *reinterpret_cast<uint32_t *>(o + (intptr_t)y * ds) = pack16(clip_pix(s0 >> kVShift), clip_pix(s1 >> kVShift));
+        *reinterpret_cast<uint32_t *>(o) = pack_hi16(clip_hi16(s0), clip_hi16(s1));
+        if (++y >= rows) break;
+        o += ds;
+        HRow<TAPS> h;
+        int b0, b1;
+        h.fetch(q);
+        q += ls >> 1;
+        h.sums(ht, b0, b1);
 #pragma unroll
-        for (int k = 0; k < TAPS - 1; k++) {
-            t0[k] = t0[k + 1];
-            t1[k] = t1[k + 1];
+        for (int k = 0; k < TAPS - 2; k++) {
+            P0[k] = P0[k + 1];
+            P1[k] = P1[k + 1];
         }
+        P0[TAPS - 2] = pack_mid16(l0, b0);
+        P1[TAPS - 2] = pack_mid16(l1, b1);
+        l0 = b0;
+        l1 = b1;
     }
 }
 
@@ -640,13 +692,13 @@ struct SubWin {
     int wx0, wy0, cx0, cy0;
 };
 
-__device__ __forceinline__ SubWin stage_sub(const RefineArgs &a, const xg_block &B, const MvWin &mw,
-                                            const xg_picture &R, int sx, int sy, int sw, int sh, RefineLds &L)
+__device__ __forceinline__ SubWin stage_sub(ArgPtr a, const xg_block &B, const MvWin &mw,
+                                            PicPtr R, int sx, int sy, int sw, int sh, RefineLds &L)
 {
-    const int qx0 = (sx << 4) + clampi(B.mvx + a.offMinX, mw.mnx, mw.mxx);
-    const int qx1 = (sx << 4) + clampi(B.mvx + a.offMaxX, mw.mnx, mw.mxx);
-    const int qy0 = (sy << 4) + clampi(B.mvy + a.offMinY, mw.mny, mw.mxy);
-    const int qy1 = (sy << 4) + clampi(B.mvy + a.offMaxY, mw.mny, mw.mxy);
+    const int qx0 = (sx << 4) + clampi(B.mvx + a->offMinX, mw.mnx, mw.mxx);
+    const int qx1 = (sx << 4) + clampi(B.mvx + a->offMaxX, mw.mnx, mw.mxx);
+    const int qy0 = (sy << 4) + clampi(B.mvy + a->offMinY, mw.mny, mw.mxy);
+    const int qy1 = (sy << 4) + clampi(B.mvy + a->offMaxY, mw.mny, mw.mxy);
     SubWin w;
     w.wx0 = ((qx0 >> 4) - 3) & ~1;
     w.wy0 = (qy0 >> 4) - 3;
@@ -654,12 +706,9 @@ __device__ __forceinline__ SubWin stage_sub(const RefineArgs &a, const xg_block 
     w.cx0 = ((qx0 >> 5) - 1) & ~1;
     w.cy0 = (qy0 >> 5) - 1;
     const int CWW = (qx1 >> 5) + (sw >> 1) + 2 - w.cx0, CHH = (qy1 >> 5) - (qy0 >> 5) + (sh >> 1) + 3;
-    const StagePlan pl = stage_plan(L.luma, kLumaLW / 2, plane_dw(R.plane[0], w.wx0, w.wy0), R.plane[0].stride >> 1,
-                                    HH, (WW + 1) >> 1);
-    const StagePlan pu = stage_plan(L.cb, kChromaLW / 2, plane_dw(R.plane[1], w.cx0, w.cy0), R.plane[1].stride >> 1,
-                                    CHH, (CWW + 1) >> 1);
-    const StagePlan pv = stage_plan(L.cr, kChromaLW / 2, plane_dw(R.plane[2], w.cx0, w.cy0), R.plane[2].stride >> 1,
-                                    CHH, (CWW + 1) >> 1);
+    const StagePlan pl = stage_plan(L.luma, kLumaLW / 2, R, 0, w.wx0, w.wy0, HH, (WW + 1) >> 1);
+    const StagePlan pu = stage_plan(L.cb, kChromaLW / 2, R, 1, w.cx0, w.cy0, CHH, (CWW + 1) >> 1);
+    const StagePlan pv = stage_plan(L.cr, kChromaLW / 2, R, 2, w.cx0, w.cy0, CHH, (CWW + 1) >> 1);
     const int nb = max(pl.batches, pu.batches);
     for (int k = 0; k < nb; k++) {
         uint32_t vl[8], vu[8], vv[8];
@@ -678,26 +727,26 @@ __device__ __forceinline__ SubWin stage_sub(const RefineArgs &a, const xg_block 
 }
 
 // Luma + chroma prediction of one sub-block of the winner from the staged windows.
-__device__ __forceinline__ void mc_sub(const RefineArgs &a, const xg_block &B, int mvx, int mvy, int sx, int sy,
+__device__ __forceinline__ void mc_sub(ArgPtr a, const xg_block &B, int mvx, int mvy, int sx, int sy,
                                        int sw, int sh, const SubWin &w, const RefineLds &L)
 {
-    const xg_picture PT = uniform_load(&a.predTab[B.pic]);
-    const xg_plane &P0 = PT.plane[0], &P1 = PT.plane[1], &P2 = PT.plane[2];
+    const PicPtr PT = fresh(pic_ptr(&a->predTab[B.pic]));
     const int rx = (sx << 4) + mvx, ry = (sy << 4) + mvy;   // the sub-block's reference position
-    mc_pass<8>(L.luma, kLumaLW, (rx >> 4) - 3 - w.wx0, (ry >> 4) - 3 - w.wy0, L.tapL + 15 * (rx & 15), ry & 15, sw, sh,
-               P0.data + (intptr_t)sy * P0.stride + sx, P0.stride, 0, 64);
+    mc_pass<8>(L.luma, kLumaLW, (rx >> 4) - 3 - w.wx0, (ry >> 4) - 3 - w.wy0, L.tapL + 15 * (rx & 15),
+               L.tapL + 15 * (ry & 15), sw, sh, PT->plane[0].data + (intptr_t)sy * PT->plane[0].stride + sx, PT->plane[0].stride, lane_here(), 6);
+    // chroma: half the wave a plane
     const int wc = sw >> 1, hc = sh >> 1, ox = (rx >> 5) - 1 - w.cx0, oy = (ry >> 5) - 1 - w.cy0;
-    const uint32_t *hc4 = L.tapC + 9 * (rx & 31);
-    mc_pass<4>(L.cb, kChromaLW, ox, oy, hc4, ry & 31, wc, hc,
-               P1.data + (intptr_t)(sy >> 1) * P1.stride + (sx >> 1), P1.stride, 0, 64);
-    mc_pass<4>(L.cr, kChromaLW, ox, oy, hc4, ry & 31, wc, hc,
-               P2.data + (intptr_t)(sy >> 1) * P2.stride + (sx >> 1), P2.stride, 0, 64);
+    const int lane = lane_here();
+    const bool cr = lane >= 32;
+    const intptr_t ds = cr ? PT->plane[2].stride : PT->plane[1].stride;
+    mc_pass<4>(cr ? L.cr : L.cb, kChromaLW, ox, oy, L.tapC + 9 * (rx & 31), L.tapC + 9 * (ry & 31), wc, hc,
+               (cr ? PT->plane[2].data : PT->plane[1].data) + (intptr_t)(sy >> 1) * ds + (sx >> 1), ds, lane & 31, 5);
 }
 
 // Best-candidate record and luma + chroma prediction of block b.  A block of
 // one sub-block predicts from the windows its task staged; a larger block
 // stages each sub-block again (they hold every candidate's footprint).
-__device__ __forceinline__ void mc_block(const RefineArgs &a, int b, const xg_block &B, const MvWin &mw,
+__device__ __forceinline__ void mc_block(ArgPtr a, ListPtr l, int b, const xg_block &B, const MvWin &mw,
                                          unsigned long long key, RefineLds &L, const SubWin &last)
 {
     const int lane = threadIdx.x;
@@ -710,37 +759,42 @@ __device__ __forceinline__ void mc_block(const RefineArgs &a, int b, const xg_bl
         r.mvy = mvy;
         r.cost = (uint32_t)(key >> 32);
         r.cand = c;
-        a.best[b] = r;
+        l->best[b] = r;
     }
-    if (a.mvField) {
-        const int uw = B.w >> 2, nu = uw * (B.h >> 2);
-        int2 *f = a.mvField + (intptr_t)(B.y >> 2) * a.mvStride + (B.x >> 2);
-        for (int u = lane; u < nu; u += 64) f[(intptr_t)(u / uw) * a.mvStride + u % uw] = make_int2(mvx, mvy);
+    if (l->mvField) {
+        const int lgU = 29 - __builtin_clz((unsigned)B.w), nu = (B.h >> 2) << lgU;
+        int2 *f = l->mvField + (intptr_t)(B.y >> 2) * l->mvStride + (B.x >> 2);
+        for (int u = lane; u < nu; u += 64)
+            f[(intptr_t)(u >> lgU) * l->mvStride + (u & ((1 << lgU) - 1))] = make_int2(mvx, mvy);
     }
     const int sw = min(B.w, kSub), sh = min(B.h, kSub);
     if (sw == B.w && sh == B.h) {
         mc_sub(a, B, mvx, mvy, B.x, B.y, sw, sh, last, L);
         return;
     }
-    const xg_picture R = uniform_load(&a.pics[B.ref]);
     for (int sy = B.y; sy < B.y + B.h; sy += sh)
         for (int sx = B.x; sx < B.x + B.w; sx += sw) {
             __syncthreads();
-            const SubWin w = stage_sub(a, B, mw, R, sx, sy, sw, sh, L);
+            const SubWin w = stage_sub(a, B, mw, fresh(pic_ptr(&a->pics[B.ref])), sx, sy, sw, sh, L);
             __syncthreads();
             mc_sub(a, B, mvx, mvy, sx, sy, sw, sh, w, L);
         }
 }
 
-__device__ __forceinline__ void refine_one(const RefineArgs &a, int2 tk, const xg_block &B, RefineLds &L)
+// Bound by VALU issue.  1920x1080, 32 candidates, 18,600 blocks: 48.3 M vector
+// instructions, which take 79 us to issue; 86 us a launch with several in
+// flight, 126 alone (62.2 M, 107 and 151 before).  About 30 M are the filters
+// and transforms; the rest, once as large as these, is what a task does beside
+// them: descriptors and windows addressed with scalars (a division-free copy
+// plan), tap tables copied instead of computed, the winner's prediction on the
+// packed filters with both chroma planes at once, and nothing computed ahead
+// of the task loop for shapes a task does not have (lane_here, fresh).
+__device__ __forceinline__ void refine_one(ArgPtr a, ListPtr l, int2 tk, const xg_block &B, RefineLds &L)
 {
-    const int lane = threadIdx.x;
+    const int lane = lane_here();
     const int b = tk.x, c0 = tk.y & 0xFFFF, nc = tk.y >> 16;
-    const xg_picture P = uniform_load(&a.pics[B.pic]);
-    const xg_picture R = uniform_load(&a.pics[B.ref]);
-    const MvWin mw = mv_window(B, P.plane[0].width, P.plane[0].height, a.ctuSize);
-
-    const intptr_t cs = P.plane[0].stride, ccs = P.plane[1].stride;
+    const PicPtr pics = pic_ptr(a->pics);
+    const MvWin mw = mv_window(B, pics[B.pic].plane[0].width, pics[B.pic].plane[0].height, a->ctuSize);
     L.csum[lane] = 0;
     uint32_t *csum = L.csum;
     const int sw = min(B.w, kSub), sh = min(B.h, kSub);
@@ -748,9 +802,11 @@ __device__ __forceinline__ void refine_one(const RefineArgs &a, int2 tk, const x
     for (int sy = B.y; sy < B.y + B.h; sy += sh)
         for (int sx = B.x; sx < B.x + B.w; sx += sw) {
             __syncthreads();                           // the previous sub-block's readers are done
-            w = stage_sub(a, B, mw, R, sx, sy, sw, sh, L);
+            w = stage_sub(fresh(a), B, mw, fresh(pics + B.ref), sx, sy, sw, sh, L);
             __syncthreads();
-            const uint16_t *cur = P.plane[0].data + (intptr_t)sy * cs + sx;
+            PicPtr P = fresh(pics + B.pic);
+            const intptr_t cs = P->plane[0].stride;
+            const uint16_t *cur = P->plane[0].data + (intptr_t)sy * cs + sx;
             const int ox = sx - B.x, oy = sy - B.y;     // sub-block offset inside the block
             const bool t4 = sw == 4 || sh == 4;
             switch (sw) {
@@ -764,9 +820,10 @@ __device__ __forceinline__ void refine_one(const RefineArgs &a, int2 tk, const x
             }
             __syncthreads();
 
-            if (a.useChroma) {
-                const intptr_t co = (intptr_t)(sy >> 1) * ccs + (sx >> 1);
-                const uint16_t *cu = P.plane[1].data + co, *cv = P.plane[2].data + co;
+            if (fresh(a)->useChroma) {
+                P = fresh(P);
+                const intptr_t ccs = P->plane[1].stride, co = (intptr_t)(sy >> 1) * ccs + (sx >> 1);
+                const uint16_t *cu = P->plane[1].data + co, *cv = P->plane[2].data + co;
                 const int wc = sw >> 1, hc = sh >> 1;
                 const int tc = (wc % 8 == 0 && hc % 8 == 0) ? 8 : (wc % 4 == 0 && hc % 4 == 0) ? 4 : 2;
                 const int cx0 = w.cx0, cy0 = w.cy0;
@@ -786,57 +843,64 @@ __device__ __forceinline__ void refine_one(const RefineArgs &a, int2 tk, const x
         }
 
     // ---- costs, task-local best, block completion ----
-    unsigned long long key = ~0ull;
+    a = fresh(a);
+    l = fresh(l);
+    uint32_t cost = 0xFFFFFFFFu;
     if (lane < nc) {
         const int c = c0 + lane;
         const int mvx = clampi(B.mvx + L.off[c], mw.mnx, mw.mxx);
         const int mvy = clampi(B.mvy + L.off[XG_MAX_CAND + c], mw.mny, mw.mxy);
         const uint32_t bits = eg_bits(mvx - B.mvpx) + eg_bits(mvy - B.mvpy);
-        const uint32_t cost = (csum[lane] << 8) + bits * a.lambda;
-        a.candCost[(size_t)b * a.ncand + c] = cost;
-        key = ((unsigned long long)cost << 32) | (uint32_t)c;
+        cost = (csum[lane] << 8) + bits * a->lambda;
+        l->candCost[(size_t)b * a->ncand + c] = cost;
     }
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) {
-        const unsigned long long o = (unsigned long long)__shfl_xor((long long)key, m, 64);
-        key = o < key ? o : key;
-    }
+    const uint32_t lo = wave_min(cost);
+    unsigned long long key = ((unsigned long long)lo << 32) |
+                             (uint32_t)(c0 + __builtin_ctzll(__ballot(lane < nc && cost == lo)));
     if (lane == 0) {
         int last = 0;
-        if (!a.doMc) {
+        if (!a->doMc) {
             last = 0;
-        } else if (nc == a.ncand) {
+        } else if (nc == a->ncand) {
             last = 1;                                // the task covers the whole block
         } else {
-            atomicMin(&a.bestKey[b], key);
+            atomicMin(&l->bestKey[b], key);
             __threadfence();
-            last = atomicAdd(&a.done[b], nc) + nc == a.ncand;
+            last = atomicAdd(&l->done[b], nc) + nc == a->ncand;
             if (last) {
                 __threadfence();
-                key = atomicExch(&a.bestKey[b], ~0ull);   // read and reset for the next launch
-                atomicExch(&a.done[b], 0);
+                key = atomicExch(&l->bestKey[b], ~0ull);   // read and reset for the next launch
+                atomicExch(&l->done[b], 0);
             }
         }
         L.last = last;
         L.key = key;
     }
     __syncthreads();
-    if (uniform(L.last)) mc_block(a, b, B, mw, L.key, L, w);
+    if (uniform(L.last)) mc_block(fresh(a), fresh(l), b, B, mw, L.key, L, w);
     __syncthreads();
 }
 
 // Batched form: a persistent grid; workgroup g runs the tasks the host
 // assigned to it (balanced by estimated cost, heaviest first), so the launch
 // takes no atomics to schedule and leaves no state behind.
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_refine_persistent(RefineArgs a)
+__device__ __forceinline__ void refine_tasks(ArgPtr a, ListPtr l, int g, RefineLds &L)
+{
+    ConstPtr<int> wg = (ConstPtr<int>)(uintptr_t)l->wgBegin;
+    const int e = wg[g + 1];
+    for (int t = wg[g]; t < e; t++) {
+        l = fresh(l);
+        const int2 tk = uniform_load(&l->tasks[t]);
+        refine_one(fresh(a), l, tk, uniform_load(&l->blocks[tk.x]), L);
+    }
+}
+
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_refine_persistent(RefineArgs)
 {
     __shared__ RefineLds L;
+    const ArgPtr a = args_ptr();
     lds_init(L, a);
-    const int e = uniform(a.wgBegin[blockIdx.x + 1]);
-    for (int t = uniform(a.wgBegin[blockIdx.x]); t < e; t++) {
-        const int2 tk = uniform_load(&a.tasks[t]);
-        refine_one(a, tk, uniform_load(&a.blocks[tk.x]), L);
-    }
+    refine_tasks(a, (ListPtr)a, (int)blockIdx.x, L);
 }
 
 // Multi-list form (serving): one persistent grid over the frames of several
@@ -844,39 +908,29 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_
 // and outputs; workgroup g runs, list after list, the tasks of virtual
 // workgroup (g + rot) mod grid, so small lists are spread over the grid.
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
-k_refine_multi(RefineArgs base, const RefineList *__restrict__ lists, int nLists, int grid)
+k_refine_multi(RefineArgs, const RefineList *__restrict__ lists, int nLists, int grid)
 {
     __shared__ RefineLds L;
-    lds_init(L, base);
-    for (int l = 0; l < nLists; l++) {
-        const RefineList R = uniform_load(&lists[l]);
-        RefineArgs a = base;
-        a.blocks = R.blocks;
-        a.candCost = R.candCost;
-        a.best = R.best;
-        a.bestKey = R.bestKey;
-        a.done = R.done;
-        a.mvField = R.mvField;
-        a.mvStride = R.mvStride;
-        int v = (int)blockIdx.x + R.rot;
+    const ArgPtr a = args_ptr();
+    lds_init(L, a);
+    for (int i = 0; i < nLists; i++) {
+        const ListPtr l = (ListPtr)(uintptr_t)lists + i;
+        int v = (int)blockIdx.x + l->rot;
         if (v >= grid) v -= grid;
-        const int e = uniform(R.wgBegin[v + 1]);
-        for (int t = uniform(R.wgBegin[v]); t < e; t++) {
-            const int2 tk = uniform_load(&R.tasks[t]);
-            refine_one(a, tk, uniform_load(&R.blocks[tk.x]), L);
-        }
+        refine_tasks(a, l, v, L);
     }
 }
 
 // Plain form: one launch per block shape, one workgroup per task.
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_refine_shape(RefineArgs a)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) k_refine_shape(RefineArgs)
 {
     __shared__ RefineLds L;
+    const ArgPtr a = args_ptr();
     lds_init(L, a);
-    const int t = a.taskBegin + (int)blockIdx.x;
-    if (t < a.taskEnd) {
-        const int2 tk = uniform_load(&a.tasks[t]);
-        refine_one(a, tk, uniform_load(&a.blocks[tk.x]), L);
+    const int t = a->taskBegin + (int)blockIdx.x;
+    if (t < a->taskEnd) {
+        const int2 tk = uniform_load(&a->tasks[t]);
+        refine_one(a, (ListPtr)a, tk, uniform_load(&a->blocks[tk.x]), L);
     }
 }
 
