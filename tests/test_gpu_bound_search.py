@@ -133,3 +133,68 @@ def test_frame_search(oracle, kind, size, bs, rng, ctu, lam, shift):
     assert np.array_equal(g[:, 0], emx) and np.array_equal(g[:, 1], emy)
     assert np.array_equal(cost.cpu().numpy().view(np.uint32), ec)
     assert np.array_equal(sad.cpu().numpy().view(np.uint32), es)
+
+
+@pytest.mark.parametrize("kind,rng,ctu,lam,n", [
+    ("texture", 16, 64, 1024, 4400), ("texture", 32, 48, 1024, 4000), ("texture", 16, 64, 1024, 3999),
+    ("texture", 15, 64, 1024, 4000), ("texture", 16, 64, (1 << 21) + 1, 4000), ("half", 21, 64, 1024, 4100),
+    ("flat", 16, 7, 0, 4000), ("extreme", 24, 64, 1024, 4000), ("extreme", 16, 64, 1 << 21, 4000),
+    ("periodic", 19, 64, 0, 4000), ("constant", 16, 31, 0, 4000)])
+def test_block_search(oracle, kind, rng, ctu, lam, n):
+    """Session blocks of every shape, large ones listed over several launches, on both sides of the rule."""
+    from tests.oracle_lib import OrMe
+    from xin26x_amd.device import blocks_to_struct
+    lib = capi.load()
+    h, w, pad = 136, 200, 96
+    cur, ref, _ = content(kind, h, w)
+    half = lambda p: np.ascontiguousarray(p[::2, ::2])
+    pics = [DevicePicture([p, half(p), half(p)], pad) for p in (cur, ref)]
+    pred = DevicePicture.empty(w, h)
+    r = np.random.default_rng(n + rng)
+    sides, p = (4, 8, 16, 32, 64), (0.2, 0.3, 0.25, 0.15, 0.1)
+    blocks = []
+    for _ in range(n):
+        bw, bh = (int(v) for v in r.choice(sides, 2, p=p))
+        x, y = int(r.integers(0, (w - bw) // 4 + 1)) * 4, int(r.integers(0, (h - bh) // 4 + 1)) * 4
+        blocks.append((x, y, bw, bh, 0, 0, int(r.integers(-600, 601)), int(r.integers(-600, 601))))
+    s = ctypes.c_void_p()
+    assert lib.xg_session_create(ctypes.byref(s), n) == 0
+    try:
+        for k in (0, 1):
+            assert lib.xg_session_set_picture(s, k, pics[k].ref()) == 0
+        barr = blocks_to_struct(blocks)
+        assert lib.xg_session_set_blocks(s, barr.ctypes.data, n) == 0
+        assert lib.xg_search_blocks(s, rng, lam, ctu) == 0
+        cfg = refine_cfg([(0, 0)], wl.LAMBDA_REFINE, ctu)
+        assert lib.xg_refine_frac(s, ctypes.byref(cfg), pred.ref(), capi.MODE_BATCHED) == 0
+        best = np.zeros(n * 4, np.int32)
+        assert lib.xg_session_read(s, None, best.ctypes.data) == 0
+    finally:
+        lib.xg_session_destroy(s)
+    got = best.reshape(n, 4)[:, :2]
+    refp = np.ascontiguousarray(np.pad(ref, pad, mode="edge"))
+    rs, m = w + 2 * pad, ctu + 8
+
+    def check(i):
+        x, y, bw, bh, _, _, mvpx, mvpy = blocks[i]
+        o = OrMe()
+        o.width, o.height = bw, bh
+        o.minMvX, o.minMvY, o.maxMvX, o.maxMvY = -x - m, -y - m, w + m - bw - x, h + m - bh - y
+        # the search centre kept inside the window, as the block search keeps it
+        o.predMvX, o.predMvY = mvpx >> 2, mvpy >> 2
+        o.searchWidth = o.searchHeight = rng
+        o.sadLambda = lam
+        o.input = cur.ctypes.data + 2 * (y * w + x)
+        o.inputStride = w
+        o.ref = refp.ctypes.data + 2 * ((y + pad) * rs + x + pad)
+        o.refStride = rs
+        oracle.or_MotionEstFull(ctypes.byref(o))
+        return (got[i, 0], got[i, 1]) == (4 * o.bestMvX, 4 * o.bestMvY)
+
+    # predictors whose centre lies outside the window are not the oracle's form
+    inside = [i for i, (x, y, bw, bh, _, _, px, py) in enumerate(blocks)
+              if -x - m <= ((px >> 2) + 2) >> 2 <= w + m - bw - x and -y - m <= ((py >> 2) + 2) >> 2 <= h + m - bh - y]
+    with ThreadPoolExecutor(8) as ex:
+        bad = [i for i, ok in zip(inside, ex.map(check, inside)) if not ok]
+    assert not bad, [blocks[i] for i in bad[:5]]
+    assert len(inside) > n // 2

@@ -234,6 +234,14 @@ __device__ __forceinline__ uint32_t align16(uint32_t hi, uint32_t lo, uint32_t s
     return __builtin_amdgcn_alignbit(hi, lo, sh);
 }
 
+// The sample pair at p (any sample alignment).  Reads only dwords that hold one of the two samples.
+__device__ __forceinline__ uint32_t load_pair(const uint16_t *p)
+{
+    const uint32_t odd = (uint32_t)((uintptr_t)p >> 1) & 1;
+    const gdword *g = (const gdword *)((uintptr_t)p & ~(uintptr_t)3);
+    return align16(g[odd], g[0], odd << 4);
+}
+
 // Block-reduce helper for one workgroup of 256 threads.
 __device__ __forceinline__ uint32_t block_sum256(uint32_t v)
 {

@@ -104,14 +104,6 @@ __device__ __forceinline__ uint32_t row_sum(uint32_t v)
     return v;
 }
 
-// The sample pair at p (any sample alignment).  Reads only dwords that hold one of the two samples.
-__device__ __forceinline__ uint32_t load_pair(const uint16_t *p)
-{
-    const uint32_t odd = (uint32_t)((uintptr_t)p >> 1) & 1;
-    const gdword *g = (const gdword *)((uintptr_t)p & ~(uintptr_t)3);
-    return align16(g[odd], g[0], odd << 4);
-}
-
 // Stages the window of 2 wd x rows samples at picture position (px, py); wd <= kWinDw.
 template <int BS>
 __device__ __forceinline__ void stage_window(const MctfArgs &a, MctfLds<BS> &L, int px, int py, int wd, int rows)

@@ -908,6 +908,18 @@ __global__ void __launch_bounds__(256) k_subpel_one(const uint16_t *greg, int rs
     }
 }
 
+// The bounded form of the block search from range 16 and 4,000 blocks on.  With
+// all its launches (predictors, search, refinement), several calls in flight:
+// 1280x720 (8,300 blocks) range 16: 166 -> 114 us, range 24: 281 -> 159, range 12:
+// no gain; 960x540 (4,600) range 16: 115 -> 83; 640x360 (2,100) range 16: no gain,
+// and 416x240 (900) 43 -> 53.  With noise of +-64, where most candidates are
+// listed, 1280x720 range 16 takes as long either way.
+constexpr int kBlkMinRange = 16, kBlkMinBlocks = 4000;
+static bool bound_blocks_rule(int n, int range, uint32_t lambda)
+{
+    return n >= kBlkMinBlocks && range >= kBlkMinRange && lambda <= kSeaLambda;
+}
+
 // Dynamic LDS of the per-call searches.
 constexpr size_t kCallLds = 60 * 1024;         // (a 16-byte round-up more at most)
 
@@ -953,6 +965,13 @@ __device__ __forceinline__ void search_block(const xg_picture *pics, xg_block &B
     B.mvy = 16 * (y0 + i / nx);
 }
 
+// Session blocks that k_search_blocks_bound takes; the others' windows are too
+// large for its one wave (bound_blocks_rule).
+__host__ __device__ __forceinline__ bool bound_block(int w, int h, int range)
+{
+    return (w + 2 * range) * (h + 2 * range) <= (16 + 2 * range) * (32 + 2 * range);
+}
+
 // Integer search of every session block around its predictor; the result is
 // written back as the block's base MV.
 __global__ void __launch_bounds__(1024) k_search_blocks(const xg_picture *pics, xg_block *blocks, int range,
@@ -964,6 +983,318 @@ __global__ void __launch_bounds__(1024) k_search_blocks(const xg_picture *pics, 
     if (threadIdx.x == 0) {
         blocks[b].mvx = B.mvx;
         blocks[b].mvy = B.mvy;
+    }
+}
+
+// The same for listed blocks, those that the bounded form leaves.
+constexpr int kRestMax = 480;                    // of a launch: the list travels with its arguments
+struct RestList {
+    int b[kRestMax];
+};
+__global__ void __launch_bounds__(1024) k_search_blocks_rest(const xg_picture *pics, xg_block *blocks, int range,
+                                                             uint32_t lambda, int ctu, int ws, RestList rest)
+{
+    const int b = rest.b[blockIdx.x];
+    xg_block B = blocks[b];
+    search_block(pics, B, range, lambda, ctu, ws);
+    if (threadIdx.x == 0) {
+        blocks[b].mvx = B.mvx;
+        blocks[b].mvy = B.mvy;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Session blocks by bounds (xg_sea.hpp), a workgroup of two waves a block
+//
+// The window, staged so that candidate (0, 0) is column 0 of row 0, and the sums
+// of 4x4 samples at each of its positions, lie in LDS.  (1) Each lane takes the
+// lowest bound of its share of the candidates, and the 128 of them are costed, a
+// lane each: their lowest cost limits the rest.  (2) Every candidate whose
+// bound is within the limit goes to its wave's list, which is costed 64 at a
+// time, a lane each, and may lower the wave's limit.  A lane that costs a whole candidate needs no
+// reduction, and flat content, where every candidate is listed, is searched at
+// the cost of the exhaustive form.  Up to three waves' worth of candidates are
+// costed without bounds.
+//
+// 1280x720, 8,300 blocks, range 16: 124 us exhaustively; 68 us here, 21 M vector
+// instructions (35 us to issue) at 3 waves a SIMD, which is what 13 KB of window
+// and sums a block leave, and 20 us for the 2 % that go by the list.  Two waves a
+// block: one took 87 us.
+// ---------------------------------------------------------------------------
+constexpr int kBlkDirect = 192;                  // candidates costed without bounds at most
+constexpr int kBlkWaves = 2, kBlkWg = 64 * kBlkWaves;
+constexpr int kBlkList = 192;                    // of a wave: under 64 when a step adds up to 128
+
+struct BlkLds {
+    int wp, sums, cur, csum, rates, list, bytes; // window pitch; dword offsets; all in bytes
+};
+__host__ __device__ __forceinline__ BlkLds blk_lds(int w, int h, int range)
+{
+    const int n = 2 * range + 1, rows = n + h;   // a row more than the candidates reach
+    BlkLds l;
+    l.wp = ((n + w) / 2 + 2) | 1;
+    l.sums = rows * l.wp;
+    l.cur = 2 * l.sums;
+    l.csum = l.cur + w * h / 2;
+    l.rates = l.csum + (h / 4) * (w < 8 ? 1 : w / 8);
+    l.list = l.rates + 2 * (n + 2);
+    l.bytes = 4 * l.list + 2 * kBlkList * kBlkWaves;
+    return l;
+}
+
+// SAD of the candidate at (cx, cy) of the window, by one lane.
+template <int W>
+__device__ __forceinline__ uint32_t lane_sad(const uint32_t *win, int wp, const uint32_t *cur, int h, int cx, int cy)
+{
+    constexpr int CH = W < 16 ? W / 2 : 8;       // dwords of a row at once
+    const uint32_t sh = (uint32_t)(cx & 1) << 4;
+    uint32_t e = 0;
+    const uint32_t *w = win + cy * wp + (cx >> 1);
+#pragma unroll 1
+    for (int i = 0; i < h; i++, w += wp, cur += W / 2)
+#pragma unroll
+        for (int k = 0; k < W / 2; k += CH) {
+            uint32_t D[CH + 1];
+#pragma unroll
+            for (int j = 0; j <= CH; j++) D[j] = w[k + j];
+#pragma unroll
+            for (int j = 0; j < CH; j++) e = sad2(align16(D[j + 1], D[j], sh), cur[k + j], e);
+        }
+    return e;
+}
+
+// Bounds of candidates 2 j and 2 j + 1 of a row (q: their dword of the sums) of a
+// block W wide with hs rows of sub-blocks, added to l and h.  C: the block's sums,
+// a packed pair of adjacent sub-blocks a dword (W = 4: one in the lower half).
+template <int W>
+__device__ __forceinline__ void lane_bounds(const uint32_t *q, int pitch, const uint32_t *C, int hs, uint32_t &l, uint32_t &h)
+{
+#pragma unroll 1
+    for (int i = 0; i < hs; i++, q += 4 * pitch) {
+        if constexpr (W == 4) {
+            const uint32_t u = q[0], c = C[i];
+            l = sad2(u & 0xFFFFu, c, l);
+            h = sad2(u >> 16, c, h);
+        } else {
+#pragma unroll
+            for (int k = 0; k < W / 8; k++) {
+                const uint32_t u = q[4 * k], v = q[4 * k + 2], c = C[i * (W / 8) + k];
+                l = sad2(__builtin_amdgcn_perm(v, u, 0x05040100u), c, l);
+                h = sad2(__builtin_amdgcn_perm(v, u, 0x07060302u), c, h);
+            }
+        }
+    }
+}
+
+struct BlkWin {
+    int x0, y0, nx, ny, pmx, pmy, h;
+    uint32_t lambda;
+};
+
+template <int W>
+__device__ __forceinline__ unsigned long long bound_search(uint32_t *lds, const BlkLds &o, const BlkWin &v, uint32_t *limits)
+{
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));               // nothing computed ahead for the other widths: registers
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wp = o.wp, nx = v.nx, ny = v.ny, hs = v.h / 4;
+    const uint32_t *win = lds, *S = lds + o.sums, *cur = lds + o.cur, *C = lds + o.csum, *bxq = lds + o.rates + 1,
+                   *byq = bxq + nx + 1;
+    uint16_t *list = reinterpret_cast<uint16_t *>(lds + o.list) + wave * kBlkList;
+    unsigned long long best = ~0ull;             // the lane's lowest (cost, position)
+    auto cost = [&](int pos) {
+        const int cx = pos & 255, cy = pos >> 8;
+        const uint32_t e = lane_sad<W>(win, wp, cur, v.h, cx, cy);
+        const uint32_t k = (e << 8) + (eg_bits(4 * (v.x0 + cx) - v.pmx) + eg_bits(4 * (v.y0 + cy) - v.pmy)) * v.lambda;
+        const unsigned long long q = ((unsigned long long)k << 32) | (uint32_t)pos;
+        best = q < best ? q : best;
+    };
+    if (nx * ny <= kBlkDirect) {
+        const uint32_t rcp = (65536u + (uint32_t)nx - 1) / (uint32_t)nx;
+        for (int i = tid; i < nx * ny; i += kBlkWg) {
+            const int cy = (int)(((uint32_t)i * rcp) >> 16);
+            cost(cy << 8 | (i - cy * nx));
+        }
+    } else {
+        const int nc = (nx + 1) >> 1, items = ny * nc;
+        const uint32_t rcp = (65536u + (uint32_t)nc - 1) / (uint32_t)nc;
+        const int dr = (int)(((uint32_t)kBlkWg * rcp) >> 16), dj = kBlkWg - dr * nc;
+        const int r0 = (int)(((uint32_t)tid * rcp) >> 16), j0 = tid - r0 * nc;
+        uint32_t key = 0xFFFFFFFFu;
+        int kpos = 0;
+        for (int i = tid, r = r0, j = j0; i < items; i += kBlkWg) {
+            uint32_t l = byq[r] + bxq[2 * j], h = byq[r] + bxq[2 * j + 1];
+            lane_bounds<W>(S + r * wp + j, wp, C, hs, l, h);
+            const uint32_t k = min(l, h);
+            kpos = k < key ? r << 8 | (2 * j + (h < l)) : kpos;
+            key = min(key, k);
+            r += dr;
+            j += dj;
+            if (j >= nc) {
+                j -= nc;
+                r++;
+            }
+        }
+        cost(kpos);                              // lanes without an item cost candidate 0
+        uint32_t limit = wave_min((uint32_t)(best >> 32)) >> 8;
+        if (lane == 0) limits[wave] = limit;
+        __syncthreads();
+        limit = min(limits[0], limits[1]);
+        int n = 0;
+        auto flush = [&]() {                     // cost the first 64 of the list, keep the others
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int rest = n - 64;
+            const uint16_t a = list[64 + lane], b = list[128 + lane];
+            if (lane < n) cost(list[lane]);
+            limit = min(limit, wave_min((uint32_t)(best >> 32)) >> 8);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            if (lane < rest) list[lane] = a;
+            if (lane + 64 < rest) list[64 + lane] = b;
+            n = max(rest, 0);
+        };
+        for (int i0 = 64 * wave, r = r0, j = j0; i0 < items; i0 += kBlkWg) {
+            const bool in = i0 + lane < items;
+            uint32_t l = kSeaOver, h = kSeaOver;
+            if (in) {
+                l = byq[r] + bxq[2 * j];
+                h = byq[r] + bxq[2 * j + 1];
+                lane_bounds<W>(S + r * wp + j, wp, C, hs, l, h);
+            }
+            auto push = [&](uint32_t q, int pos) {
+                const bool ok = q <= limit;
+                const unsigned long long m = __ballot(ok);
+                const int at = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+                if (ok) list[at] = (uint16_t)pos;
+                n += __popcll(m);
+            };
+            push(l, r << 8 | 2 * j);
+            push(h, r << 8 | (2 * j + 1));
+            while (n >= 64) flush();
+            r += dr;
+            j += dj;
+            if (j >= nc) {
+                j -= nc;
+                r++;
+            }
+        }
+        if (n) flush();
+    }
+    const uint32_t lo = wave_min((uint32_t)(best >> 32));
+    const uint32_t pos = wave_min((uint32_t)(best >> 32) == lo ? (uint32_t)best : 0xFFFFFFFFu);
+    return ((unsigned long long)lo << 32) | pos;
+}
+
+__global__ void __launch_bounds__(kBlkWg) __attribute__((amdgpu_waves_per_eu(6))) k_search_blocks_bound(const xg_picture *pics, xg_block *blocks, int range,
+                                                            uint32_t lambda, int ctu)
+{
+    extern __shared__ uint32_t smem32[];
+    __shared__ uint32_t limits[kBlkWaves];
+    __shared__ unsigned long long found[kBlkWaves];
+    const int tid = threadIdx.x;
+    const xg_block &B = blocks[blockIdx.x];
+    const int bw = B.w, bh = B.h;
+    if (!bound_block(bw, bh, range)) return;
+    const xg_picture &P = pics[B.pic], &Rf = pics[B.ref];
+    const int fw = P.plane[0].width, fh = P.plane[0].height;
+    const int mnx = (int16_t)(-B.x - ctu - 8), mny = (int16_t)(-B.y - ctu - 8);
+    const int mxx = (int16_t)(fw + (ctu - bw + 8) - B.x), mxy = (int16_t)(fh + (ctu - bh + 8) - B.y);
+    const int cx = min(max(((B.mvpx >> 2) + 2) >> 2, mnx), mxx), cy = min(max(((B.mvpy >> 2) + 2) >> 2, mny), mxy);
+    BlkWin v;
+    v.x0 = max(cx - range, mnx);
+    v.y0 = max(cy - range, mny);
+    v.nx = min(cx + range, mxx) - v.x0 + 1;
+    v.ny = min(cy + range, mxy) - v.y0 + 1;
+    v.pmx = B.mvpx >> 2;
+    v.pmy = B.mvpy >> 2;
+    v.h = bh;
+    v.lambda = lambda;
+    const BlkLds o = blk_lds(bw, bh, range);
+    const int rows = v.ny + bh - 1, wd = (v.nx + bw) >> 1, wp = o.wp;     // the window: rows of wd dwords
+    // window and current block (its rows are dword aligned)
+    {
+        const int lg = wd <= 16 ? 4 : 5, c = tid & ((1 << lg) - 1), r0 = tid >> lg, step = kBlkWg >> lg;
+        const intptr_t rs = Rf.plane[0].stride;
+        const uint16_t *g = Rf.plane[0].data + (intptr_t)(B.y + v.y0 + r0) * rs + B.x + v.x0;
+        for (int cc = c; cc < wd; cc += 1 << lg) {
+            const uint16_t *p = g + 2 * cc;
+            uint32_t *d = smem32 + r0 * wp + cc;
+            for (int r = r0; r < rows; r += 4 * step) {
+                uint32_t w[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (r + k * step < rows) w[k] = load_pair(p + (intptr_t)(k * step) * rs);
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    if (r + k * step < rows) d[k * step * wp] = w[k];
+                p += (intptr_t)(4 * step) * rs;
+                d += 4 * step * wp;
+            }
+        }
+        const int lw = 30 - __builtin_clz((unsigned)bw);                  // dwords of a block row, log2
+        const intptr_t cs = P.plane[0].stride;
+        const uint16_t *q = P.plane[0].data + (intptr_t)B.y * cs + B.x;
+        for (int i = tid; i < bh << lw; i += kBlkWg)
+            smem32[o.cur + i] = *(const gdword *)(q + (intptr_t)(i >> lw) * cs + 2 * (i & ((1 << lw) - 1)));
+    }
+    // shares of the rate: columns -1 .. nx (over any limit outside), then rows
+    uint32_t *rates = smem32 + o.rates;
+    for (int i = tid; i < v.nx + 2 + v.ny; i += kBlkWg) {
+        const int k = i - 1, m = k <= v.nx ? 4 * (v.x0 + k) - v.pmx : 4 * (v.y0 + i - v.nx - 2) - v.pmy;
+        rates[i] = i == 0 || k == v.nx ? kSeaOver : (eg_bits(m) * lambda) >> 8;
+    }
+    __syncthreads();
+    if (v.nx * v.ny > kBlkDirect) {
+        // sums of 4x4 samples: a column pair and a run of rows a lane, sliding
+        const uint32_t *win = smem32;
+        uint32_t *S = smem32 + o.sums;
+        const int nj = (v.nx + bw - 2) >> 1, ns = rows - 3;               // column pairs that hold a candidate's sum
+        const int runs = max(1, (int)((uint32_t)kBlkWg / (uint32_t)nj)), len = (ns + runs - 1) / runs;
+        for (int i = tid; i < runs * nj; i += kBlkWg) {
+            const int run = i / nj, j = i - run * nj, y0 = run * len, y1 = min(ns, y0 + len);
+            auto hsum = [&](int r) {
+                const uint32_t *w = win + r * wp + j;
+                const uint32_t a = w[0], b = w[1], c = w[2];
+                return as_v2s(a) + as_v2s(align16(b, a, 16)) + as_v2s(b) + as_v2s(align16(c, b, 16));
+            };
+            if (y0 < y1) {
+                v2s h0 = hsum(y0), h1 = hsum(y0 + 1), h2 = hsum(y0 + 2);
+                for (int r = y0; r < y1; r++) {
+                    const v2s h3 = hsum(r + 3);
+                    S[r * wp + j] = as_u32(h0 + h1 + h2 + h3);
+                    h0 = h1;
+                    h1 = h2;
+                    h2 = h3;
+                }
+            }
+        }
+        // the block's own sums
+        const int lp = bw < 8 ? 0 : 28 - __builtin_clz((unsigned)bw);     // pairs of sub-blocks a row, log2
+        for (int i = tid; i < (bh / 4) << lp; i += kBlkWg) {
+            const uint32_t *q = smem32 + o.cur + 4 * (i >> lp) * (bw / 2) + 4 * (i & ((1 << lp) - 1));
+            uint32_t a = 0, b = 0;
+#pragma unroll
+            for (int r = 0; r < 4; r++, q += bw / 2) {
+                a = sad2(q[0], 0, sad2(q[1], 0, a));
+                if (bw >= 8) b = sad2(q[2], 0, sad2(q[3], 0, b));
+            }
+            smem32[o.csum + i] = a | b << 16;
+        }
+        __syncthreads();
+    }
+    unsigned long long k;
+    switch (bw) {
+    case 4: k = bound_search<4>(smem32, o, v, limits); break;
+    case 8: k = bound_search<8>(smem32, o, v, limits); break;
+    case 16: k = bound_search<16>(smem32, o, v, limits); break;
+    case 32: k = bound_search<32>(smem32, o, v, limits); break;
+    default: k = bound_search<64>(smem32, o, v, limits); break;
+    }
+    if ((tid & 63) == 0) found[tid >> 6] = k;
+    __syncthreads();
+    if (tid == 0) {
+        k = min(found[0], found[1]);
+        blocks[blockIdx.x].mvx = 16 * (v.x0 + (int)((uint32_t)k & 255));
+        blocks[blockIdx.x].mvy = 16 * (v.y0 + (int)((uint32_t)k >> 8));
     }
 }
 
@@ -1105,7 +1436,7 @@ int32_t xg_search_blocks(xg_session *s, int32_t range, uint32_t sadLambda, int32
         return XG_ERR_ARG;
     }
     if (v.nblocks == 0) return XG_OK;
-    int maxw = 0, maxh = 0;
+    int maxw = 0, maxh = 0, restw = 0, resth = 0, boundLds = 0;      // rest: those k_search_blocks_bound leaves
     for (int i = 0; i < v.nblocks; i++) {
         const xg_block &B = v.hBlocks[i];
         if (B.pic >= kSessionPicSlots || B.ref >= kSessionPicSlots || !v.picSet[B.pic] || !v.picSet[B.ref]) {
@@ -1128,6 +1459,12 @@ int32_t xg_search_blocks(xg_session *s, int32_t range, uint32_t sadLambda, int32
         }
         maxw = std::max(maxw, (int)B.w);
         maxh = std::max(maxh, (int)B.h);
+        if (bound_block(B.w, B.h, range)) {
+            boundLds = std::max(boundLds, blk_lds(B.w, B.h, range).bytes);
+        } else {
+            restw = std::max(restw, (int)B.w);
+            resth = std::max(resth, (int)B.h);
+        }
     }
     const int ws = packed_ws(2 * range + 1, maxw);
     const size_t lds = ((size_t)(2 * range + maxh) * ws + (size_t)maxw * maxh) * 2 + 16;
@@ -1135,10 +1472,30 @@ int32_t xg_search_blocks(xg_session *s, int32_t range, uint32_t sadLambda, int32
         set_error(XG_ERR_ARG, "xg_search_blocks: window exceeds the LDS budget");
         return XG_ERR_ARG;
     }
+    const bool bounded = bound_blocks_rule(v.nblocks, range, sadLambda);
     int ev[2];
     const bool timed = session_timer_begin(s, 3, ev);
-    k_search_blocks<<<v.nblocks, packed_threads(2 * range + 1), lds, v.stream>>>(v.dPics, v.dBlocks, range,
-                                                                                sadLambda, ctuSize, ws);
+    const int threads = packed_threads(2 * range + 1);
+    if (!bounded) {
+        k_search_blocks<<<v.nblocks, threads, lds, v.stream>>>(v.dPics, v.dBlocks, range, sadLambda, ctuSize, ws);
+    } else {
+        if (restw) {
+            const int wsr = packed_ws(2 * range + 1, restw);
+            const size_t ldsr = ((size_t)(2 * range + resth) * wsr + (size_t)restw * resth) * 2 + 16;
+            RestList l;
+            for (int i = 0, k = 0; i < v.nblocks; i++) {
+                if (!bound_block(v.hBlocks[i].w, v.hBlocks[i].h, range)) l.b[k++] = i;
+                if (k == kRestMax || (k && i == v.nblocks - 1)) {
+                    k_search_blocks_rest<<<k, threads, ldsr, v.stream>>>(v.dPics, v.dBlocks, range, sadLambda, ctuSize,
+                                                                         wsr, l);
+                    k = 0;
+                }
+            }
+        }
+        if (boundLds)
+            k_search_blocks_bound<<<v.nblocks, kBlkWg, (size_t)boundLds, v.stream>>>(v.dPics, v.dBlocks, range, sadLambda,
+                                                                                   ctuSize);
+    }
     if (timed) session_timer_end(s, 3, ev);
     return XG_HIP(hipGetLastError()) ? XG_OK : XG_ERR_HIP;
 }
