@@ -125,6 +125,20 @@ __device__ __forceinline__ uint32_t wave_min(uint32_t v)
     return min(min(r0, r1), min(r2, r3));
 }
 
+// Sum over aligned groups of 8 or 16 lanes, in every lane of the group.
+template <int G>
+__device__ __forceinline__ uint32_t row_sum(uint32_t v)
+{
+    static_assert(G == 8 || G == 16, "lanes of a DPP row");
+    v += dpp<kXor1>(v);
+    v += dpp<kXor2>(v);
+    v += dpp<kHalfMirror>(v);                    // quads are uniform by now
+    if constexpr (G == 16) v += dpp<kRor8>(v);
+    return v;
+}
+
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // One butterfly stage of a Walsh-Hadamard transform across lanes: the lane
 // with bit M clear keeps a + b, the partner keeps a - b.
 template <int M>

@@ -44,8 +44,6 @@ namespace xg {
 constexpr int kMctfMaxRange = 8;
 constexpr int kMctfMaxBs = 16;
 
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
 struct MctfArgs {
     const uint16_t *cur;
     intptr_t cs;
@@ -90,18 +88,6 @@ __device__ __forceinline__ uint16_t ref_at(const MctfArgs &a, int x, int y)
     x = min(max(x, -a.pad), a.w - 1 + a.pad);
     y = min(max(y, -a.pad), a.h - 1 + a.pad);
     return a.ref[(intptr_t)y * a.rs + x];
-}
-
-// Sum over aligned groups of 8 or 16 lanes, in every lane of the group.
-template <int G>
-__device__ __forceinline__ uint32_t row_sum(uint32_t v)
-{
-    static_assert(G == 8 || G == 16, "lanes of a DPP row");
-    v += dpp<kXor1>(v);
-    v += dpp<kXor2>(v);
-    v += dpp<kHalfMirror>(v);                    // quads are uniform by now
-    if constexpr (G == 16) v += dpp<kRor8>(v);
-    return v;
 }
 
 // Stages the window of 2 wd x rows samples at picture position (px, py); wd <= kWinDw.

@@ -333,25 +333,6 @@ __device__ __forceinline__ uint32_t row_sad(const xg_plane &R, int rx, int ry, c
     return acc;
 }
 
-// Sum over the 16 lanes of a row of the wavefront.
-__device__ __forceinline__ uint32_t sum16(uint32_t v)
-{
-    v += (uint32_t)shfl_xor<1>((int)v);
-    v += (uint32_t)shfl_xor<2>((int)v);
-    v += (uint32_t)shfl_xor<4>((int)v);
-    v += (uint32_t)shfl_xor<8>((int)v);
-    return v;
-}
-
-// Sum over aligned groups of 8 lanes.
-__device__ __forceinline__ uint32_t sum8(uint32_t v)
-{
-    v += (uint32_t)shfl_xor<1>((int)v);
-    v += (uint32_t)shfl_xor<2>((int)v);
-    v += (uint32_t)shfl_xor<4>((int)v);
-    return v;
-}
-
 __device__ __forceinline__ uint32_t cost_q(uint32_t sad, int mvqx, int mvqy, int px, int py, uint32_t lambda)
 {
     return (sad << 8) + (eg_bits(mvqx - px) + eg_bits(mvqy - py)) * lambda;
@@ -367,7 +348,7 @@ __device__ __forceinline__ uint32_t cost_row16(const xg_plane &RP, int x, int y,
                                                uint32_t lambda)
 {
     const int row = threadIdx.x & 15;
-    const uint32_t s = sum16(row_sad(RP, x + mx, y + my + row, c));
+    const uint32_t s = row_sum<16>(row_sad(RP, x + mx, y + my + row, c));
     return cost_q(s, 4 * mx, 4 * my, 0, 0, lambda);
 }
 
@@ -676,35 +657,44 @@ __global__ void __launch_bounds__(256) k_pipe_left(PipeArgs a, int per)
     if (lane == 0) a.found[id].best = best;
 }
 
-__global__ void __launch_bounds__(64) k_pipe_dia(PipeArgs a)
+// Bound by VALU issue.  3840x2160, two references, 64,800 waves: 375 -> 209 us,
+// 2,990 -> 1,500 vector instructions a wave (159 us to issue).
+// What is the same in every lane (predictor, candidate list, the search's position
+// and its decisions) is kept in scalars; a 16-lane group costs its own position
+// and no other; and the rings filter a column at one of the three horizontal
+// offsets a lane (48 of 64), once, into packed row pairs in registers, from which
+// the three vertical offsets are formed with scalar taps.
+__global__ void __launch_bounds__(64) k_pipe_dia(PipeArgs a, int per)
 {
-    const int b = blockIdx.x >> 1, r = blockIdx.x & 1;
-    const int bx = b % a.nbx, by = b / a.nbx, x = bx * kPB, y = by * kPB;
+    const int id = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (id >= 2 * a.nb) return;
+    const int b = id >> 1, r = id & 1;
+    const int by = b / a.nbx, bx = b - by * a.nbx, x = bx * kPB, y = by * kPB;
     const IWin w = int_window(x, y, a.fw, a.fh, a.ctu);
     const xg_plane &RP = a.pics[r ? a.refSlot1 : a.refSlot0].plane[0];
     const xg_plane &CP = a.pics[a.curSlot].plane[0];
     const int lane = threadIdx.x, grp = lane >> 4, row = lane & 15;
 
-    // predictor and start candidates (every lane computes the same list)
+    // predictor and start candidates
     int nqx[4], nqy[4];
     {
         const int nbi[4] = {b, bx > 0 ? b - 1 : -1, by > 0 ? b - a.nbx : -1,
                             (by > 0 && bx + 1 < a.nbx) ? b - a.nbx + 1 : -1};
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            const unsigned long long f = a.found[max(nbi[k], 0) * 2 + r].best;
+            const unsigned long long f = (uint32_t)uniform((int)(uint32_t)a.found[max(nbi[k], 0) * 2 + r].best);
             nqx[k] = nbi[k] < 0 ? 0 : 4 * pos_x(f);
             nqy[k] = nbi[k] < 0 ? 0 : 4 * pos_y(f);
         }
         if (lane == 0) {
-            a.fullMv[(b * 2 + r) * 2] = (int16_t)(nqx[0] >> 2);
-            a.fullMv[(b * 2 + r) * 2 + 1] = (int16_t)(nqy[0] >> 2);
+            a.fullMv[id * 2] = (int16_t)(nqx[0] >> 2);
+            a.fullMv[id * 2 + 1] = (int16_t)(nqy[0] >> 2);
         }
     }
     const int px = (int16_t)median3(nqx[1], nqx[2], nqx[3]), py = (int16_t)median3(nqy[1], nqy[2], nqy[3]);
-    int cx[6], cy[6], nc = 1;
-    cx[0] = 0;
-    cy[0] = 0;
+    int cx[8], cy[8], nc = 1;
+#pragma unroll
+    for (int j = 0; j < 8; j++) cx[j] = cy[j] = 0;
 #pragma unroll
     for (int i = 0; i < 5; i++) {
         const int vx = i == 0 ? px : nqx[i - 1], vy = i == 0 ? py : nqy[i - 1];
@@ -729,44 +719,30 @@ __global__ void __launch_bounds__(64) k_pipe_dia(PipeArgs a)
 #pragma unroll
         for (int j = 0; j < 8; j++) c[j] = cp[j];
     }
-    // cost of up to 4 integer positions at once (group g = lane / 16 takes position g)
-    auto eval4 = [&](const int *mx, const int *my, const bool *ok, uint32_t *cost, uint32_t *sads) {
-        const int g = grp;
+    // costs of the four groups' integer positions; UINT32_MAX where a group has none
+    auto eval4 = [&](int mx, int my, bool ok, uint32_t *cost) {
         uint32_t s = 0;
-        if (ok[0] | ok[1] | ok[2] | ok[3]) {
-            const int gx = g == 0 ? mx[0] : g == 1 ? mx[1] : g == 2 ? mx[2] : mx[3];
-            const int gy = g == 0 ? my[0] : g == 1 ? my[1] : g == 2 ? my[2] : my[3];
-            const bool gok = g == 0 ? ok[0] : g == 1 ? ok[1] : g == 2 ? ok[2] : ok[3];
-            if (gok) s = row_sad(RP, x + gx, y + gy + row, c);
-            s = sum16(s);
-        }
+        if (ok) s = row_sad(RP, x + mx, y + my + row, c);
+        s = row_sum<16>(s);
+        const uint32_t k = ok ? cost_q(s, 4 * mx, 4 * my, px, py, a.lambda) : 0xFFFFFFFFu;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            sads[k] = (uint32_t)__shfl((int)s, 16 * k, 64);
-            cost[k] = ok[k] ? cost_q(sads[k], 4 * mx[k], 4 * my[k], px, py, a.lambda) : 0xFFFFFFFFu;
-        }
+        for (int g = 0; g < 4; g++) cost[g] = (uint32_t)__builtin_amdgcn_readlane((int)k, 16 * g);
     };
     // start candidates in list order (clipped to the MV window), strict <
     uint32_t best = 0xFFFFFFFFu;
     int bmx = 0, bmy = 0;
-    for (int base = 0; base < nc; base += 4) {
+#pragma unroll
+    for (int base = 0; base < 8; base += 4) {
+        if (base >= nc) break;
+        uint32_t cost[4];
         int mx[4], my[4];
-        bool ok[4];
-        uint32_t cost[4], sads[4];
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            int ix = 0, iy = 0;
-#pragma unroll
-            for (int j = 0; j < 6; j++)
-                if (j == base + k) {
-                    ix = cx[j];
-                    iy = cy[j];
-                }
-            mx[k] = min(max(ix, w.mnx), w.mxx);
-            my[k] = min(max(iy, w.mny), w.mxy);
-            ok[k] = base + k < nc;
+            mx[k] = min(max(cx[base + k], w.mnx), w.mxx);
+            my[k] = min(max(cy[base + k], w.mny), w.mxy);
         }
-        eval4(mx, my, ok, cost, sads);
+        eval4(grp == 0 ? mx[0] : grp == 1 ? mx[1] : grp == 2 ? mx[2] : mx[3],
+              grp == 0 ? my[0] : grp == 1 ? my[1] : grp == 2 ? my[2] : my[3], base + grp < nc, cost);
 #pragma unroll
         for (int k = 0; k < 4; k++)
             if (cost[k] < best) {
@@ -776,133 +752,131 @@ __global__ void __launch_bounds__(64) k_pipe_dia(PipeArgs a)
             }
     }
     // small diamond L, R, T, B around the best, inside the window and +/-range of the rounded predictor
-    const int ccx = (px + 2) >> 2, ccy = (py + 2) >> 2;
-    for (int step = 0; step < 2 * a.range; step++) {
-        const int dxs[4] = {-1, 1, 0, 0}, dys[4] = {0, 0, -1, 1};
-        int mx[4], my[4];
-        bool ok[4];
-        uint32_t cost[4], sads[4];
+    {
+        const int ccx = (px + 2) >> 2, ccy = (py + 2) >> 2;
+        const int lx = max(w.mnx, ccx - a.range), hx = min(w.mxx, ccx + a.range);
+        const int ly = max(w.mny, ccy - a.range), hy = min(w.mxy, ccy + a.range);
+        const int gx = (grp == 1) - (grp == 0), gy = (grp == 3) - (grp == 2);
+        for (int step = 0; step < 2 * a.range; step++) {
+            const int mx = bmx + gx, my = bmy + gy;
+            uint32_t cost[4];
+            eval4(mx, my, mx >= lx && mx <= hx && my >= ly && my <= hy, cost);
+            uint32_t nb = best;
+            int win = -1;
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            mx[k] = bmx + dxs[k];
-            my[k] = bmy + dys[k];
-            ok[k] = mx[k] >= w.mnx && mx[k] <= w.mxx && my[k] >= w.mny && my[k] <= w.mxy &&
-                    mx[k] >= ccx - a.range && mx[k] <= ccx + a.range && my[k] >= ccy - a.range &&
-                    my[k] <= ccy + a.range;
+            for (int k = 0; k < 4; k++)
+                if (cost[k] < nb) {
+                    nb = cost[k];
+                    win = k;
+                }
+            if (win < 0) break;
+            bmx += (win == 1) - (win == 0);
+            bmy += (win == 3) - (win == 2);
+            best = nb;
         }
-        eval4(mx, my, ok, cost, sads);
-        uint32_t nb = best;
-        int nx = bmx, ny = bmy;
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            if (cost[k] < nb) {
-                nb = cost[k];
-                nx = mx[k];
-                ny = my[k];
-            }
-        if (nx == bmx && ny == bmy) break;
-        bmx = nx;
-        bmy = ny;
-        best = nb;
     }
     if (lane == 0) {
-        a.predMv[(b * 2 + r) * 2] = (int16_t)px;
-        a.predMv[(b * 2 + r) * 2 + 1] = (int16_t)py;
-        a.intMv[(b * 2 + r) * 2] = (int16_t)bmx;
-        a.intMv[(b * 2 + r) * 2 + 1] = (int16_t)bmy;
-        a.intCost[b * 2 + r] = best;
+        a.predMv[id * 2] = (int16_t)px;
+        a.predMv[id * 2 + 1] = (int16_t)py;
+        a.intMv[id * 2] = (int16_t)bmx;
+        a.intMv[id * 2 + 1] = (int16_t)bmy;
+        a.intCost[id] = best;
     }
 
-    // half- then quarter-pel rings (L, R, T, B, TL, TR, BL, BR), 8-tap SAD, strict <;
-    // lane = candidate * 8 + m: columns 2m, 2m+1 of candidate lane / 8
+    // half- then quarter-pel rings (L, R, T, B, TL, TR, BL, BR), 8-tap SAD, strict <:
+    // lane (i, col) = (lane / 16, lane % 16) takes horizontal offset i - 1 and column col;
+    // taps and offsets are scaled as in pack_mid16 and clip_hi16
     int qx = bmx * 4, qy = bmy * 4;
-    if (bmx < w.mnx || bmx > w.mxx || bmy < w.mny || bmy > w.mxy) {   // cannot happen: kept for the reference's guard
-        if (lane == 0) {
-            a.qMv[(b * 2 + r) * 2] = (int16_t)qx;
-            a.qMv[(b * 2 + r) * 2 + 1] = (int16_t)qy;
-            a.qCost[b * 2 + r] = best;
-        }
-        return;
-    }
-    const int cand = lane >> 3, m = lane & 7;
-    const int ringx[8] = {-1, 1, 0, 0, -1, 1, -1, 1}, ringy[8] = {0, 0, -1, 1, -1, -1, 1, 1};
-    uint32_t cw[16];
+    const bool inside = bmx >= w.mnx && bmx <= w.mxx && bmy >= w.mny && bmy <= w.mxy;   // always: the reference's guard
+    const int i = min(grp, 2), col = row;
+    uint32_t cv[kPB / 2];                            // the column's rows in pairs
     {
-        const uint32_t *cp = reinterpret_cast<const uint32_t *>(CP.data + (intptr_t)y * CP.stride + x + 2 * m);
+        const gword *cp = (const gword *)(CP.data + (intptr_t)y * CP.stride + x + col);
 #pragma unroll
-        for (int i = 0; i < 16; i++) cw[i] = cp[(intptr_t)i * (CP.stride >> 1)];
+        for (int k = 0; k < kPB / 2; k++) cv[k] = pack16(cp[(intptr_t)(2 * k) * CP.stride], cp[(intptr_t)(2 * k + 1) * CP.stride]);
     }
-    for (int pass = 0; pass < 2; pass++) {
-        const int step = pass == 0 ? 2 : 1;
-        int rx = ringx[0], ry = ringy[0];
-#pragma unroll
-        for (int k = 1; k < 8; k++)
-            if (k == cand) {
-                rx = ringx[k];
-                ry = ringy[k];
-            }
-        const int tx = qx + rx * step, ty = qy + ry * step;          // quarter pel
-        const int m16x = tx * 4, m16y = ty * 4;
-        const int fx = m16x & 15, fy = m16y & 15;
-        uint32_t hp[4];
-        int vc[8];
+#pragma unroll 1
+    for (int step = inside ? 2 : 0; step > 0; step--) {
+        const int m16x = 4 * (qx + (i - 1) * step);
+        const int top = (4 * (qy - step)) >> 4, spread = ((4 * (qy + step)) >> 4) - top;    // 0 or 1
+        const uint16_t *p = RP.data + (intptr_t)(y + top - 3) * RP.stride + x + col + (m16x >> 4) - 3;
+        const bool odd = (uintptr_t)p & 2;               // in every row: strides are even
+        const gdword *q = (const gdword *)((uintptr_t)p & ~(uintptr_t)3);
+        const intptr_t rsw = RP.stride >> 1;
+        uint32_t T[5];                                   // tap pairs against the dwords from the one with the first tap
         {
-            const int8_t *ch = taps_for<8>(fx, 0), *cv = taps_for<8>(fy, 0);
+            const int8_t *hf = c_luma[0][m16x & 15];
+            uint32_t A[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++)
-                hp[j] = pack16(ch[2 * j], ch[2 * j + 1]);
+            for (int j = 0; j < 4; j++) A[j] = pack16(64 * hf[2 * j], 64 * hf[2 * j + 1]);
+            T[0] = odd ? A[0] << 16 : A[0];
 #pragma unroll
-            for (int j = 0; j < 8; j++) vc[j] = cv[j];
+            for (int j = 1; j < 4; j++) T[j] = odd ? align16(A[j], A[j - 1], 16) : A[j];
+            T[4] = odd ? A[3] >> 16 : 0;
         }
-        // first tap of column 2m at row 0: (x + 2m + (m16x >> 4) - 3, y + (m16y >> 4) - 3)
-        const int sx = x + 2 * m + (m16x >> 4) - 3, sy = y + (m16y >> 4) - 3;
-        int t0[kPB + 7], t1[kPB + 7];
-        uint32_t sad = 0;
+        uint32_t P[kPB + 7];                             // P[k]: first-pass rows k and k + 1
+        int last = 0;
 #pragma unroll
-        for (int i = 0; i < kPB + 7; i++) {
-            const uint16_t *p = RP.data + (intptr_t)(sy + i) * RP.stride + sx;
-            const uint32_t *q = reinterpret_cast<const uint32_t *>(reinterpret_cast<uintptr_t>(p) & ~(uintptr_t)3);
-            const uint32_t sh = (uint32_t)(reinterpret_cast<uintptr_t>(p) & 2) << 3;
-            uint32_t D[6], E[5];
+        for (int k = 0; k < kPB + 8; k++) {
+            uint32_t D[5];
 #pragma unroll
-            for (int j = 0; j < 6; j++) D[j] = q[j];
+            for (int j = 0; j < 5; j++) D[j] = q[j];
+            if (k + 1 < kPB + 7 || spread) q += rsw;     // the last row again when the offsets share their rows
+            int u = dot2_first(D[0], T[0], kHRound64);
 #pragma unroll
-            for (int j = 0; j < 5; j++) E[j] = align16(D[j + 1], D[j], sh);
-            int s0 = kHOffset, s1 = kHOffset;
+            for (int j = 1; j < 5; j++) u = dot2(D[j], T[j], u);
+            if (k) P[k - 1] = pack_mid16(last, u);
+            last = u;
+            if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // no more than four rows' loads in flight: registers
+        }
+        int at = top;
+        uint32_t mine = 0;
+#pragma unroll 1
+        for (int j = 0; j < 3; j++) {
+            const int my = 4 * (qy + (j - 1) * step);
+            if ((my >> 4) != at) {                       // uniform, at most once
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                s0 = dot2(E[j], hp[j], s0);
-                s1 = dot2(align16(E[j + 1], E[j], 16), hp[j], s1);
+                for (int k = 0; k < kPB + 6; k++) P[k] = P[k + 1];
+                at++;
+                asm volatile("");                        // stays a branch
             }
-            t0[i] = s0 >> kHShift;
-            t1[i] = s1 >> kHShift;
-            if (i >= 7) {
-                int v0 = kVOffset, v1 = kVOffset;
+            const int8_t *vf = c_luma[0][my & 15];
+            uint32_t V[4];
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    v0 += vc[j] * t0[i - 7 + j];
-                    v1 += vc[j] * t1[i - 7 + j];
+            for (int k = 0; k < 4; k++) V[k] = ((uint32_t)(64 * vf[2 * k]) & 0xFFFF) | (uint32_t)(64 * vf[2 * k + 1]) << 16;
+            uint32_t sad = 0;
+#pragma unroll
+            for (int k = 0; k < kPB; k += 2) {
+                int s0 = dot2_first(P[k], V[0], 0), s1 = dot2_first(P[k + 1], V[0], 0);
+#pragma unroll
+                for (int m = 1; m < 4; m++) {
+                    s0 = dot2(P[k + 2 * m], V[m], s0);
+                    s1 = dot2(P[k + 1 + 2 * m], V[m], s1);
                 }
-                sad = sad2(pack16(clip_pix(v0 >> kVShift), clip_pix(v1 >> kVShift)), cw[i - 7], sad);
+                sad = sad2(pack_hi16(clip_hi16(s0), clip_hi16(s1)), cv[k / 2], sad);
             }
+            sad = row_sum<16>(sad);
+            mine = col == j ? sad : mine;
         }
-        sad = sum8(sad);
-        const uint32_t cost = cost_q(sad, tx, ty, px, py, a.lambda);
-        // earliest candidate among the strictly better ones
-        unsigned long long key = ((unsigned long long)cost << 32) | (uint32_t)cand;
-#pragma unroll
-        for (int mm = 8; mm < 64; mm <<= 1) key = min_u64(key, (unsigned long long)__shfl_xor((long long)key, mm, 64));
-        if ((uint32_t)(key >> 32) < best) {
-            best = (uint32_t)(key >> 32);
-            const int kk = (int)(uint32_t)key;
-            qx = qx + ringx[kk] * step;
-            qy = qy + ringy[kk] * step;
+        // lane (i, j): the position at offsets (i - 1, j - 1); its place in the ring's order
+        const int dx = i - 1, dy = col - 1;
+        const bool ok = grp < 3 && col < 3 && (dx | dy);
+        const uint32_t cost = ok ? cost_q(mine, qx + dx * step, qy + dy * step, px, py, a.lambda) : 0xFFFFFFFFu;
+        const int order = dy == 0 ? (dx > 0) : dx == 0 ? 2 + (dy > 0) : 4 + 2 * (dy > 0) + (dx > 0);
+        const uint32_t lo = wave_min(cost);
+        if (lo < best) {
+            best = lo;
+            const int o = (int)wave_min(cost == lo ? (uint32_t)order : 8u);
+            const int wx = o == 2 || o == 3 ? 0 : (o & 1) ? 1 : -1;
+            const int wy = o < 2 ? 0 : o == 2 || o == 4 || o == 5 ? -1 : 1;
+            qx += wx * step;
+            qy += wy * step;
         }
     }
     if (lane == 0) {
-        a.qMv[(b * 2 + r) * 2] = (int16_t)qx;
-        a.qMv[(b * 2 + r) * 2 + 1] = (int16_t)qy;
-        a.qCost[b * 2 + r] = best;
+        a.qMv[id * 2] = (int16_t)qx;
+        a.qMv[id * 2 + 1] = (int16_t)qy;
+        a.qCost[id] = best;
     }
 }
 
@@ -1027,7 +1001,8 @@ static bool enqueue_pipe(const PipeState *p, hipStream_t st, xg_session *s, bool
         k_pipe_full<kPipeQuads, false><<<2 * p->nb, 256, 0, st>>>(p->args);
     }
     if (t3) session_timer_end(s, 3, ev);
-    k_pipe_dia<<<2 * p->nb, 64, 0, st>>>(p->args);
+    const int perDia = (2 * p->nb + 7) / 8;
+    k_pipe_dia<<<8 * perDia, 64, 0, st>>>(p->args, perDia);
     k_pipe_select<<<(p->nb + 255) / 256, 256, 0, st>>>(p->args);
     return XG_HIP(hipGetLastError()) && refine_enqueue_prepared(s);
 }

@@ -133,8 +133,6 @@ __device__ __forceinline__ PicPtr pic_ptr(const xg_picture *p) { return (PicPtr)
 // The launch's arguments (every kernel's first parameter is RefineArgs).
 __device__ __forceinline__ ArgPtr args_ptr() { return (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr(); }
 
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
 // ---------------------------------------------------------------------------
 // Interpolation + SATD of one plane for a pass of candidates, two adjacent
 // columns per lane.
