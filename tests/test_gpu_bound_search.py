@@ -88,6 +88,56 @@ def test_pipeline_full_search(oracle, kind, rng, ctu, lam):
         lib.xg_session_destroy(s)
 
 
+def test_pipeline_graph_follows_the_references(oracle):
+    """Reference pictures that change from frame to frame, other buffers and strides among them: every replay
+    searches the pictures it was given, and the graph is captured once.  A call that only changes its pictures
+    takes the time of one that does not, and not of one that changes the rate weight, which is captured again."""
+    import time
+    lib = capi.load()
+    h, w, lam = 496, 848, 1024
+    planes = content("texture", h, w)
+    planes.append(np.ascontiguousarray(planes[1][::-1]))
+    half = lambda p: np.ascontiguousarray(p[::2, ::2])
+    pads = (152, 152, 96, 120)
+    pics = [DevicePicture([p, half(p), half(p)], pad) for p, pad in zip(planes, pads)]
+    pred = DevicePicture.empty(w, h)
+    nb = (w // 16) * (h // 16)
+    exp = {k: oracle_search(oracle, planes[0], planes[k], 16, 16, 24, lam, 64, 152)[:2] for k in (1, 2, 3)}
+    s = ctypes.c_void_p()
+    assert lib.xg_session_create(ctypes.byref(s), nb) == 0
+    try:
+        cfg = capi.XgPipelineCfg()
+        cfg.range, cfg.ctuSize = 24, 64
+        cfg.refine = refine_cfg([(0, 0)], wl.LAMBDA_REFINE)
+
+        def call(a, b, weight):
+            assert lib.xg_session_sync(s) == 0
+            cfg.sadLambda = weight
+            t = time.perf_counter()
+            assert lib.xg_me_pipeline(s, ctypes.byref(cfg), pics[0].ref(), pics[a].ref(), pics[b].ref(), pred.ref(),
+                                      capi.MODE_GRAPH) == 0
+            return time.perf_counter() - t
+
+        for k in range(6):
+            a, b = 1 + k % 3, 1 + (k + 1) % 3
+            call(a, b, lam)
+            full = np.zeros((nb, 2, 2), np.int16)
+            assert lib.xg_me_pipeline_read(s, full.ctypes.data, None, None, None, None, None) == 0
+            for r, e in enumerate((exp[a], exp[b])):
+                assert np.array_equal(full[:, r, 0], e[0] >> 2) and np.array_equal(full[:, r, 1], e[1] >> 2), (k, r)
+        same, other, again = [], [], []
+        for k in range(60):
+            call(1, 2, lam)
+            same.append(call(1, 2, lam))
+            other.append(call(1 + k % 2, 3, lam))
+            again.append(call(1, 2, lam + 1))
+        same, other, again = (1e6 * float(np.median(v)) for v in (same, other, again))
+        print(f"host us a call: same references {same:.1f}, others {other:.1f}, captured again {again:.1f}", flush=True)
+        assert other - same < 0.5 * (again - same)
+    finally:
+        lib.xg_session_destroy(s)
+
+
 @pytest.mark.parametrize("kind,size,bs,rng,ctu,lam,shift", [
     ("texture", (560, 816), 16, 16, 64, 1024, 0), ("texture", (489, 485), 8, 24, 64, 1024, 1),
     ("texture", (713, 709), 16, 32, 32, 0, 1), ("texture", (480, 480), 8, 48, 48, 500, 0),

@@ -50,13 +50,12 @@ constexpr int kPipeQuads = 3;                              // candidate quads pe
 constexpr int kPipeWinW = 2 * kPipeMaxRange + kPB + 4 * kPipeQuads + 2;   // 158
 constexpr int kPipeWinH = 2 * kPipeMaxRange + kPB + 1;    // 145: a two-row item may read one row past the window
 
-// Box sums of a plane over positions x0 .. x0 + w - 1, y0 .. y0 + h - 1: the
-// sum of the 8x8 (s8) and of the 4x4 samples (s4) from (x, y), at
+// Box sums of a reference plane over positions x0 .. x0 + w - 1, y0 .. y0 + h - 1:
+// the sum of the 8x8 (s8) and of the 4x4 samples (s4) from (x, y), at
 // [(y - y0) * stride + (x - x0)].  x0, w and stride even, rows of whole dwords.
-// 10-bit samples keep 8x8 sums (at most 65,472) in 16 bits.
+// 10-bit samples keep 8x8 sums (at most 65,472) in 16 bits.  The plane itself is
+// read through the device picture table, so a captured launch follows the pictures.
 struct SeaPlane {
-    const uint16_t *src;           // sample (0, 0) of the plane
-    intptr_t rs;                   // its stride (even)
     uint16_t *s8, *s4;
     int stride;                    // sums per row
     int x0, y0, w, h;              // covered positions; the samples read end at x0 + w + 8, y0 + h + 7
@@ -64,6 +63,8 @@ struct SeaPlane {
 
 struct SeaPlanes {
     SeaPlane p[2];
+    const xg_picture *pics;
+    int slot[2];                   // the planes' pictures (even stride, dword aligned: xg_session_set_picture)
 };
 
 // Both sums, two columns per thread, kBoxRows rows by sliding sums: row sums of
@@ -79,8 +80,10 @@ __global__ void __launch_bounds__(256) k_box_sums(SeaPlanes pl, int *zero)
     if (zero && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0) *zero = 0;
     const int j = (int)(blockIdx.x * blockDim.x + threadIdx.x), r0 = (int)blockIdx.y * kBoxRows;
     if (2 * j >= P.w) return;
-    const gdword *q = (const gdword *)(P.src + (intptr_t)P.y0 * P.rs + P.x0 + 2 * j);
-    const int sp = (int)(P.rs >> 1), op = P.stride >> 1, last = P.h - 1 + 7;
+    const xg_plane &R = pl.pics[pl.slot[blockIdx.z]].plane[0];
+    const intptr_t rs = R.stride;
+    const gdword *q = (const gdword *)(R.data + (intptr_t)P.y0 * rs + P.x0 + 2 * j);
+    const int sp = (int)(rs >> 1), op = P.stride >> 1, last = P.h - 1 + 7;
     uint32_t *o8 = reinterpret_cast<uint32_t *>(P.s8) + j, *o4 = reinterpret_cast<uint32_t *>(P.s4) + j;
     v2s va = {0, 0}, vb = {0, 0}, ra[4], rb[4], t[4];
 #pragma unroll
@@ -111,13 +114,11 @@ __global__ void __launch_bounds__(256) k_box_sums(SeaPlanes pl, int *zero)
     }
 }
 
-// One launch over n (1 or 2) planes of one size.
-inline void box_sums_enqueue(hipStream_t st, const SeaPlane *p, int n, int *zero)
+// One launch over both references.
+inline void box_sums_enqueue(hipStream_t st, const SeaPlanes &a, int *zero)
 {
-    SeaPlanes a;
-    a.p[0] = p[0];
-    a.p[1] = p[n - 1];
-    k_box_sums<<<dim3((p[0].w / 2 + 255) / 256, (p[0].h + kBoxRows - 1) / kBoxRows, n), 256, 0, st>>>(a, zero);
+    const SeaPlane &p = a.p[0];
+    k_box_sums<<<dim3((p.w / 2 + 255) / 256, (p.h + kBoxRows - 1) / kBoxRows, 2), 256, 0, st>>>(a, zero);
 }
 
 // The full search of a block and reference: the lowest (cost << 32 | position)
@@ -959,7 +960,7 @@ constexpr int kBoundBlocks = 1600;
 
 // Sum planes of both references over every position the searches read, and
 // the list of the exhaustive search.
-static bool sums_prepare(PipeState *p, const xg_plane &r0, const xg_plane &r1, int range, int ctu, hipStream_t st)
+static bool sums_prepare(PipeState *p, int range, int ctu, hipStream_t st)
 {
     const int reach = std::min(range, ctu + 8), left = (reach + 1) & ~1;
     // 4x4 sums to position + 12 of the last candidate; the 8x8 ones (to + 8, + 9 by pairs) fill the same box
@@ -975,11 +976,8 @@ static bool sums_prepare(PipeState *p, const xg_plane &r0, const xg_plane &r1, i
         p->sumsCap = need;
     }
     if (!p->denseGrid) p->denseGrid = resident_slots((const void *)k_pipe_full<kPipeQuads, true>, 256);
-    for (int k = 0; k < 2; k++) {
-        const xg_plane &R = k ? r1 : r0;
-        p->args.sums[k] = {R.data, R.stride, p->dSums + 2 * k * one, p->dSums + (2 * k + 1) * one, stride,
-                           -left, -left, w, h};
-    }
+    for (int k = 0; k < 2; k++)
+        p->args.sums[k] = {p->dSums + 2 * k * one, p->dSums + (2 * k + 1) * one, stride, -left, -left, w, h};
     p->args.dense = p->dDense;
     p->args.left = p->dLeft;
     return true;
@@ -992,7 +990,8 @@ static bool enqueue_pipe(const PipeState *p, hipStream_t st, xg_session *s, bool
     if (p->bounded) {
         const int nby = p->nb / p->args.nbx;
         const int per = (2 * ((p->args.nbx + kBoundB - 1) / kBoundB) * ((nby + kBoundB - 1) / kBoundB) + 7) / 8;
-        box_sums_enqueue(st, p->args.sums, 2, p->args.dense);
+        const PipeArgs &A = p->args;
+        box_sums_enqueue(st, {{A.sums[0], A.sums[1]}, A.pics, {A.refSlot0, A.refSlot1}}, A.dense);
         k_pipe_bound<<<8 * per, 64 * kBoundWaves, 0, st>>>(p->args, per);
         const int perLeft = ((2 * p->nb + 3) / 4 + 7) / 8;
         k_pipe_left<<<8 * perLeft, 256, 0, st>>>(p->args, perLeft);
@@ -1109,7 +1108,7 @@ int32_t xg_me_pipeline(xg_session *s, const xg_pipeline_cfg *cfg, const xg_pictu
     A.found = p->dFound;
     A.left = nullptr;
     p->bounded = cfg->sadLambda <= kBoundLambda && nb >= kBoundBlocks;
-    if (p->bounded && !sums_prepare(p, ref0->plane[0], ref1->plane[0], cfg->range, cfg->ctuSize, v.stream))
+    if (p->bounded && !sums_prepare(p, cfg->range, cfg->ctuSize, v.stream))
         return XG_ERR_NOMEM;
     int ev[2];
     const bool timed = session_timer_begin(s, 4, ev);
@@ -1125,10 +1124,7 @@ int32_t xg_me_pipeline(xg_session *s, const xg_pipeline_cfg *cfg, const xg_pictu
     key = hmix(key, (uint64_t)(uintptr_t)p->dMv);
     key = hmix(key, (uint64_t)(uintptr_t)p->dCost);
     if (p->bounded)
-        for (const SeaPlane &S : A.sums) {
-            key = hmix(hmix(key, (uint64_t)(uintptr_t)S.src), (uint64_t)S.rs);
-            key = hmix(key, (uint64_t)(uintptr_t)S.s8);
-        }
+        for (const SeaPlane &S : A.sums) key = hmix(key, (uint64_t)(uintptr_t)S.s8);
     key = hmix(hmix(hmix(key, (uint64_t)(uintptr_t)A.dense), (uint64_t)(uintptr_t)A.found), (uint64_t)(uintptr_t)A.left);
     // the captured refinement launch: grid, task lists, tile table, per-block state
     key = hmix(key, refine_prepared_key(s));
