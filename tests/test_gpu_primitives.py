@@ -295,3 +295,42 @@ def test_func_table(lib):
     assert lib.Xg266FuncInit(ctypes.byref(t), 0) == 0
     assert t.pfXinComputeDist[3] == addr("Xg266ComputeSad")
     assert t.pfXinComputeAvgDist[4] == addr("Xg266ComputeAvgSad")
+
+
+def _us(call, n=40, reps=7):
+    """Median time of a call in us, warmed up."""
+    import time
+    t = []
+    for k in range(reps + 1):
+        t0 = time.perf_counter()
+        for _ in range(n):
+            call()
+        t.append((time.perf_counter() - t0) / n * 1e6)
+    return float(np.median(t[1:]))
+
+
+def test_sad_sizes_past_whole_vectors(lib, oracle):
+    """Sample counts around multiples of 8 samples and of the workgroup's loads, several references a call."""
+    rng = np.random.default_rng(14)
+    a, b = rand_pixels(rng, (140, 290)), rand_pixels(rng, (140, 290))
+    for w, h in ((1, 1), (7, 1), (1, 9), (3, 5), (17, 13), (5, 51), (127, 127), (128, 127), (121, 17), (16, 128), (127, 16),
+                 (41, 50)):
+        ra = [b.ctypes.data + 2 * (k * 290 + 3 * k + 1) for k in range(8)]
+        out = np.zeros(8, np.uint32)
+        lib.Xg266ComputeSadx8(ptr(a, 5), 290, ctypes.cast((ctypes.c_void_p * 8)(*ra), ctypes.c_void_p), 290, w, h, ptr(out))
+        assert out.tolist() == [oracle.or_ComputeSad(ptr(a, 5), 290, ctypes.c_void_p(r), 290, w, h) for r in ra], (w, h)
+        lib.Xg266ComputeSad(ptr(a, 5), 290, ctypes.c_void_p(ra[1]), 290, w, h, ptr(out))
+        assert out[0] == oracle.or_ComputeSad(ptr(a, 5), 290, ctypes.c_void_p(ra[1]), 290, w, h), (w, h)
+
+
+def test_sad_takes_no_longer_than_by_copies(lib):
+    """The SAD slot, which reads its operands over the bus, against the averaged SAD slot, which copies three blocks
+    to device memory and runs two kernels: the large blocks, where a load at a time would show."""
+    rng = np.random.default_rng(15)
+    a, b = rand_pixels(rng, (128, 128)), rand_pixels(rng, (130, 128))
+    out = np.zeros(1, np.uint32)
+    for w, h in ((64, 64), (127, 127), (128, 128)):
+        one = _us(lambda: lib.Xg266ComputeSad(ptr(a), 128, ptr(b), 128, w, h, ptr(out)))
+        avg = _us(lambda: lib.Xg266ComputeAvgSad(ptr(a), 128, ptr(b), ptr(b, 128), 128, w, h, ptr(out)))
+        print(f"{w}x{h}: SAD {one:.1f} us, averaged {avg:.1f} us", flush=True)
+        assert one < 1.2 * avg, (w, h)

@@ -23,6 +23,7 @@
 
 #include "xg_device.hpp"
 #include "xg_runtime.hpp"
+#include "xg_sea.hpp"
 #include "xg_trmatrix.hpp"
 
 namespace xg {
@@ -123,14 +124,43 @@ __global__ void k_bipred(const int16_t *__restrict__ a, const int16_t *__restric
 }
 
 // SAD of packed reference blocks (one every refPitch samples) against one
-// packed input block; one workgroup per reference block.
+// packed input block; one workgroup per reference block.  Blocks start at 16-byte
+// boundaries and are readable to a multiple of 8 samples.  Bound by the round
+// trips over the bus where they lie in mapped host memory: 16 bytes a load, all
+// of a block's loads (8 of each at 128x128) issued before the first use.  A call,
+// a sample a load -> here: 64x64 33 -> 16 us, 128x128 87 -> 20, eight references of
+// 128x128 99 -> 29 (with copies to device memory instead: 24, 50 and 57).
 __global__ void __launch_bounds__(256) k_sad(const uint16_t *__restrict__ in,
                                              const uint16_t *__restrict__ refs, int npix, int refPitch,
                                              uint32_t *__restrict__ out)
 {
-    const uint16_t *r = refs + (size_t)blockIdx.x * refPitch;
+    constexpr int N = 8;
+    const uint4 *a = reinterpret_cast<const uint4 *>(in);
+    const uint4 *b = reinterpret_cast<const uint4 *>(refs + (size_t)blockIdx.x * refPitch);
+    const int nq = (npix + 7) >> 3;
     uint32_t s = 0;
-    for (int i = threadIdx.x; i < npix; i += 256) s += (uint32_t)abs((int)in[i] - (int)r[i]);
+    for (int i0 = threadIdx.x; i0 < nq; i0 += N * 256) {
+        uint4 x[N], y[N];
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const int i = i0 + 256 * k;
+            if (i < nq) {
+                x[k] = a[i];
+                y[k] = b[i];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const int left = npix - 8 * (i0 + 256 * k);          // samples from this vector's first on
+            if (left <= 0) continue;
+            const uint32_t u[4] = {x[k].x, x[k].y, x[k].z, x[k].w}, v[4] = {y[k].x, y[k].y, y[k].z, y[k].w};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t m = left >= 2 * j + 2 ? ~0u : left == 2 * j + 1 ? 0xFFFFu : 0u;
+                s = sad2(u[j] & m, v[j] & m, s);
+            }
+        }
+    }
     s = block_sum256(s);
     if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
