@@ -334,3 +334,30 @@ def test_sad_takes_no_longer_than_by_copies(lib):
         avg = _us(lambda: lib.Xg266ComputeAvgSad(ptr(a), 128, ptr(b), ptr(b, 128), 128, w, h, ptr(out)))
         print(f"{w}x{h}: SAD {one:.1f} us, averaged {avg:.1f} us", flush=True)
         assert one < 1.2 * avg, (w, h)
+
+
+def test_satd_sizes_of_two_by_two_tiles(lib, oracle):
+    """Sizes that are no multiple of 4: tile counts around the workgroup's loads, the largest, extreme samples."""
+    rng = np.random.default_rng(16)
+    a, b = rand_pixels(rng, (128, 140)), rand_pixels(rng, (128, 140))
+    e, f = ((rng.integers(0, 2, (128, 140)) * 1023).astype(np.uint16) for _ in range(2))
+    for p, q in ((a, b), (e, f)):
+        for w, h in ((2, 128), (128, 2), (6, 10), (30, 34), (32, 34), (34, 30), (62, 66), (90, 92), (92, 90), (90, 90),
+                     (126, 126), (128, 126), (126, 128)):
+            out = np.zeros(1, np.uint32)
+            lib.Xg266ComputeSatd(ptr(p, 3), 140, ptr(q, 8), 140, w, h, ptr(out))
+            assert int(out[0]) == oracle.or_ComputeSatd(ptr(p, 3), 140, ptr(q, 8), 140, w, h), (w, h)
+            lib.Xg266ComputeAvgSatd(ptr(p, 3), 140, ptr(q, 8), ptr(q, 8), 140, w, h, ptr(out))
+            assert int(out[0]) == oracle.or_ComputeSatd(ptr(p, 3), 140, ptr(q, 8), 140, w, h), (w, h)
+
+
+def test_satd_takes_no_longer_than_by_copies(lib):
+    """As for SAD: the SATD slot against the averaged SATD slot, which copies."""
+    rng = np.random.default_rng(17)
+    a, b = rand_pixels(rng, (128, 128)), rand_pixels(rng, (130, 128))
+    out = np.zeros(1, np.uint32)
+    for w, h in ((64, 64), (126, 126), (124, 124), (128, 128)):
+        one = _us(lambda: lib.Xg266ComputeSatd(ptr(a), 128, ptr(b), 128, w, h, ptr(out)))
+        avg = _us(lambda: lib.Xg266ComputeAvgSatd(ptr(a), 128, ptr(b), ptr(b, 128), 128, w, h, ptr(out)))
+        print(f"{w}x{h}: SATD {one:.1f} us, averaged {avg:.1f} us", flush=True)
+        assert one < 1.1 * avg, (w, h)

@@ -205,15 +205,10 @@ __global__ void __launch_bounds__(64) k_qiq(const int32_t *__restrict__ t, int32
     if (g == 0) *map = m;
 }
 
-// SATD of a packed w x h block pair; one thread per Hadamard tile.
+// SATD of an N x N tile of differences, normalised.
 template <int N>
-__device__ uint32_t tile_satd_serial(const uint16_t *a, const uint16_t *b, int stride)
+__device__ __forceinline__ uint32_t tile_satd_of(int (&d)[N * N])
 {
-    int d[N * N];
-#pragma unroll
-    for (int y = 0; y < N; y++)
-#pragma unroll
-        for (int x = 0; x < N; x++) d[y * N + x] = (int)a[y * stride + x] - (int)b[y * stride + x];
 #pragma unroll
     for (int y = 0; y < N; y++) wht_reg<N>(d + y * N);
 #pragma unroll
@@ -233,6 +228,56 @@ __device__ uint32_t tile_satd_serial(const uint16_t *a, const uint16_t *b, int s
     return s;
 }
 
+template <int N>
+__device__ uint32_t tile_satd_serial(const uint16_t *a, const uint16_t *b, int stride)
+{
+    int d[N * N];
+#pragma unroll
+    for (int y = 0; y < N; y++)
+#pragma unroll
+        for (int x = 0; x < N; x++) d[y * N + x] = (int)a[y * stride + x] - (int)b[y * stride + x];
+    return tile_satd_of<N>(d);
+}
+
+// SATD of the 2x2 tiles of a block pair (w even, dword aligned): a tile is a
+// dword of two rows of each, and a thread loads eight tiles before the first use.
+// Over the bus a tile at a time pays a round trip each; 126x126 has 16 a thread:
+// 54 -> 21 us a call (40 with copies to device memory).
+__device__ __forceinline__ uint32_t satd_2x2(const uint16_t *a, const uint16_t *b, int w, int tiles)
+{
+    constexpr int N = 8;
+    const uint32_t *pa = reinterpret_cast<const uint32_t *>(a), *pb = reinterpret_cast<const uint32_t *>(b);
+    const int tw = w >> 1;
+    uint32_t s = 0;
+    for (int t0 = threadIdx.x; t0 < tiles; t0 += N * 256) {
+        uint32_t x[N][2], y[N][2];
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            const int t = t0 + 256 * k;
+            if (t < tiles) {
+                const int o = t / tw * w + t % tw;               // the tile's upper row, in dwords
+                x[k][0] = pa[o];
+                x[k][1] = pa[o + tw];
+                y[k][0] = pb[o];
+                y[k][1] = pb[o + tw];
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+            if (t0 + 256 * k >= tiles) continue;
+            int d[4];
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                d[2 * r] = (int)(x[k][r] & 0xFFFF) - (int)(y[k][r] & 0xFFFF);
+                d[2 * r + 1] = (int)(x[k][r] >> 16) - (int)(y[k][r] >> 16);
+            }
+            s += tile_satd_of<2>(d);
+        }
+    }
+    return s;
+}
+
+// SATD of a packed w x h block pair; one thread per Hadamard tile.
 __global__ void __launch_bounds__(256) k_satd(const uint16_t *__restrict__ a,
                                               const uint16_t *__restrict__ b, int w, int h,
                                               uint32_t *__restrict__ out)
@@ -240,11 +285,14 @@ __global__ void __launch_bounds__(256) k_satd(const uint16_t *__restrict__ a,
     const int n = (w % 8 == 0 && h % 8 == 0) ? 8 : (w % 4 == 0 && h % 4 == 0) ? 4 : 2;
     const int tw = w / n, tiles = tw * (h / n);
     uint32_t s = 0;
-    for (int t = threadIdx.x; t < tiles; t += 256) {
-        const int off = (t / tw) * n * w + (t % tw) * n;
-        if (n == 8) s += tile_satd_serial<8>(a + off, b + off, w);
-        else if (n == 4) s += tile_satd_serial<4>(a + off, b + off, w);
-        else s += tile_satd_serial<2>(a + off, b + off, w);
+    if (n == 2) {
+        s = satd_2x2(a, b, w, tiles);
+    } else {
+        for (int t = threadIdx.x; t < tiles; t += 256) {
+            const int off = (t / tw) * n * w + (t % tw) * n;
+            if (n == 8) s += tile_satd_serial<8>(a + off, b + off, w);
+            else s += tile_satd_serial<4>(a + off, b + off, w);
+        }
     }
     s = block_sum256(s);
     if (threadIdx.x == 0) out[0] = s;
