@@ -289,3 +289,48 @@ def test_lookahead_me(oracle, unit, rng_):
                                mv.data_ptr(), cost.data_ptr(), sad.data_ptr()) == capi.XG_ERR_ARG
     lib.xg_clear_error()
     lib.xg_session_destroy(s)
+
+
+@pytest.mark.parametrize("w,h,sw,sh", [(1, 1, 3, 2), (3, 5, 8, 1), (5, 3, 2, 9), (7, 7, 0, 0), (17, 13, 11, 6), (4, 4, 84, 84),
+                                       (16, 16, 104, 60), (127, 33, 4, 5), (128, 96, 5, 3), (64, 127, 9, 2)])
+def test_full_search_staging_sizes(oracle, w, h, sw, sh):
+    """The per-call full search at odd sizes (window and block past whole 16-byte loads), large blocks and the largest
+    window it takes (16x16 at +/-104 x +/-60 is 60 KB of samples); one column more is refused."""
+    lib = capi.load()
+    lib.xg_clear_error()
+    rng, plane, cur = _planes(36)
+    bx, by = 118, 52
+    xm, om = _me_pair(rng, plane, cur, w, h, bx, by, (2, -3), sw, 512, (-180, -130), (180, 130))
+    xm.searchHeight = om.searchHeight = sh
+    lib.Xg26xMotionEstFull(ctypes.byref(xm))
+    oracle.or_MotionEstFull(ctypes.byref(om))
+    assert (xm.bestMv.mvX, xm.bestMv.mvY, xm.bestCost, xm.bestSad) == \
+           (om.bestMvX, om.bestMvY, om.bestCost, om.bestSad)
+    assert lib.xg_last_error() == 0
+    if sw == 104:
+        xm.searchWidth = 105
+        lib.Xg26xMotionEstFull(ctypes.byref(xm))
+        assert lib.xg_last_error() == capi.XG_ERR_ARG
+        lib.xg_clear_error()
+
+
+def test_full_search_stages_as_fast_as_the_diamond():
+    """A one-sample block has next to nothing to cost, so the time of its search is that of its window's staging, which
+    the diamond does for the same window."""
+    import time
+    lib = capi.load()
+    rng, plane, cur = _planes(37)
+    xm, _ = _me_pair(rng, plane, cur, 1, 1, 130, 90, (0, 0), 80, 1024, (-180, -130), (180, 130), [(0, 0)])
+
+    def us(call, n=20):
+        t = []
+        for _ in range(8):
+            t0 = time.perf_counter()
+            for _ in range(n):
+                call(ctypes.byref(xm))
+            t.append((time.perf_counter() - t0) / n * 1e6)
+        return float(np.median(t[1:]))
+
+    full, dia = us(lib.Xg26xMotionEstFull), us(lib.Xg26xMotionEstDia)
+    print(f"1x1 at +/-80: full {full:.1f} us, diamond {dia:.1f} us", flush=True)
+    assert full < 2.5 * dia

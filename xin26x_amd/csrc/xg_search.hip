@@ -41,7 +41,9 @@ __device__ __forceinline__ unsigned long long block_min_u64(unsigned long long v
 
 // One block's full search over window [x0,x1] x [y0,y1] (integer MVs).
 // win: reference samples from (x0, y0) relative to the block, stride ws;
-// cur: the block, stride bw.  Both in LDS.
+// cur: the block, stride bw.  Both in LDS.  STEP: samples whose reads are in flight
+// together (bw is a multiple of it).
+template <int STEP>
 __device__ unsigned long long full_search_core(const uint16_t *win, int ws, const uint16_t *cur, int bw, int bh,
                                                int x0, int x1, int y0, int y1, uint32_t lambda, int pmx, int pmy,
                                                unsigned long long *red)
@@ -54,7 +56,9 @@ __device__ unsigned long long full_search_core(const uint16_t *win, int ws, cons
         uint32_t sad = 0;
         for (int r = 0; r < bh; r++) {
             const uint16_t *wr = w + r * ws, *cr = cur + r * bw;
-            for (int c = 0; c < bw; c++) sad += (uint32_t)abs((int)cr[c] - (int)wr[c]);
+            for (int c = 0; c < bw; c += STEP)
+#pragma unroll
+                for (int k = 0; k < STEP; k++) sad += (uint32_t)abs((int)cr[c + k] - (int)wr[c + k]);
         }
         const int mx = x0 + ox, my = y0 + oy;
         const uint32_t cost = (sad << 8) + (eg_bits(4 * mx - pmx) + eg_bits(4 * my - pmy)) * lambda;
@@ -91,7 +95,7 @@ __global__ void __launch_bounds__(256) k_full_search_frame(FsFrameArgs a)
     const uint16_t *cp = a.cur + (intptr_t)y * a.cs + x;
     for (int i = threadIdx.x; i < a.bw * a.bh; i += blockDim.x) cur[i] = cp[(intptr_t)(i / a.bw) * a.cs + (i % a.bw)];
     __syncthreads();
-    const unsigned long long k = full_search_core(win, ws, cur, a.bw, a.bh, x0, x1, y0, y1, a.lambda, 0, 0, red);
+    const unsigned long long k = full_search_core<1>(win, ws, cur, a.bw, a.bh, x0, x1, y0, y1, a.lambda, 0, 0, red);
     if (threadIdx.x == 0) {
         const int i = (int)(uint32_t)k, nx = x1 - x0 + 1;
         const int mx = x0 + i % nx, my = y0 + i / nx;
@@ -669,32 +673,6 @@ __global__ void __launch_bounds__(256) k_search_bound(SeaFrameArgs a)
     }
 }
 
-// Per-call form: packed window and block already in global memory.
-__global__ void __launch_bounds__(256) k_full_search_one(const uint16_t *gwin, int ws, int wh, const uint16_t *gcur,
-                                                         int bw, int bh, int x0, int x1, int y0, int y1,
-                                                         uint32_t lambda, int pmx, int pmy, uint32_t *out)
-{
-    extern __shared__ uint16_t smem[];
-    __shared__ unsigned long long red[4];
-    uint16_t *win = smem, *cur = smem + ws * wh;
-    for (int i = threadIdx.x; i < ws * wh; i += blockDim.x) win[i] = gwin[i];
-    for (int i = threadIdx.x; i < bw * bh; i += blockDim.x) cur[i] = gcur[i];
-    __syncthreads();
-    const unsigned long long k = full_search_core(win, ws, cur, bw, bh, x0, x1, y0, y1, lambda, pmx, pmy, red);
-    if (threadIdx.x == 0) {
-        const int i = (int)(uint32_t)k, nx = x1 - x0 + 1;
-        const int mx = x0 + i % nx, my = y0 + i / nx;
-        uint32_t sad = 0;
-        const uint16_t *w = win + (my - y0) * ws + (mx - x0);
-        for (int r = 0; r < bh; r++)
-            for (int c = 0; c < bw; c++) sad += (uint32_t)abs((int)cur[r * bw + c] - (int)w[r * ws + c]);
-        out[0] = (uint32_t)mx;
-        out[1] = (uint32_t)my;
-        out[2] = (uint32_t)(k >> 32);
-        out[3] = sad;
-    }
-}
-
 // Region and block (na and nb packed samples, 16-byte aligned, readable to a
 // multiple of 8) into LDS at dst and dst + align8(na), 16 bytes a thread and
 // load, every load of a thread issued before its first store: over the bus each
@@ -717,6 +695,37 @@ __device__ __forceinline__ void stage_packed(uint16_t *dst, const uint16_t *a, i
             const int i = i0 + k * (int)blockDim.x;
             if (i < n) reinterpret_cast<uint4 *>(dst)[i] = v[k];
         }
+    }
+}
+
+// Per-call form: packed window and block, which may be mapped host memory, are
+// read once into LDS.  A sample a load, a round trip per 256 samples: 4x4 at +/-84
+// took 256 us, 16x16 at +/-16 90 (177 and 83 with copies to device memory); with
+// 16-byte loads 146 and 83.  Costing a sample at a time waits for its two reads,
+// and its time moves by 3 % with its place in the code; STEP 4 takes the widths that
+// are multiples of 4 (104 and 59; 64x64 at +/-44 6,142 -> 3,610, 5,943 with copies).
+template <int STEP>
+__global__ void __launch_bounds__(256) k_full_search_one(const uint16_t *gwin, int ws, int wh, const uint16_t *gcur,
+                                                         int bw, int bh, int x0, int x1, int y0, int y1,
+                                                         uint32_t lambda, int pmx, int pmy, uint32_t *out)
+{
+    extern __shared__ __align__(16) uint16_t smem[];
+    __shared__ unsigned long long red[4];
+    const uint16_t *win = smem, *cur = smem + align8(ws * wh);
+    stage_packed(smem, gwin, ws * wh, gcur, bw * bh);
+    __syncthreads();
+    const unsigned long long k = full_search_core<STEP>(win, ws, cur, bw, bh, x0, x1, y0, y1, lambda, pmx, pmy, red);
+    if (threadIdx.x == 0) {
+        const int i = (int)(uint32_t)k, nx = x1 - x0 + 1;
+        const int mx = x0 + i % nx, my = y0 + i / nx;
+        uint32_t sad = 0;
+        const uint16_t *w = win + (my - y0) * ws + (mx - x0);
+        for (int r = 0; r < bh; r++)
+            for (int c = 0; c < bw; c++) sad += (uint32_t)abs((int)cur[r * bw + c] - (int)w[r * ws + c]);
+        out[0] = (uint32_t)mx;
+        out[1] = (uint32_t)my;
+        out[2] = (uint32_t)(k >> 32);
+        out[3] = sad;
     }
 }
 
@@ -921,7 +930,7 @@ static bool bound_blocks_rule(int n, int range, uint32_t lambda)
 }
 
 // Dynamic LDS of the per-call searches.
-constexpr size_t kCallLds = 60 * 1024;         // (a 16-byte round-up more at most)
+constexpr size_t kCallLds = 60 * 1024;         // of samples (two 16-byte round-ups more at most)
 
 static inline int clampi_h(int v, int lo, int hi) { return std::min(std::max(v, lo), hi); }
 
@@ -1319,19 +1328,20 @@ void Xg26xMotionEstFull(xg_me_struct *me)
         return;
     }
     const int ws = x1 - x0 + bw, wh = y1 - y0 + bh;
-    const size_t lds = ((size_t)ws * wh + (size_t)bw * bh) * 2;
-    if (lds > 60 * 1024) {
+    if (((size_t)ws * wh + (size_t)bw * bh) * 2 > kCallLds) {
         set_error(XG_ERR_ARG, "Xg26xMotionEstFull: window %dx%d exceeds the LDS budget", ws, wh);
         return;
     }
+    const size_t lds = ((size_t)align8(ws * wh) + (size_t)align8(bw * bh)) * 2;
     const size_t wB = align_up((size_t)ws * wh * 2, 256), cB = align_up((size_t)bw * bh * 2, 256);
     CallCtx *c = call_ctx(0, wB + cB + 256);
     if (!c) return;
     pack2d(c->host, me->ref + (intptr_t)y0 * me->refStride + x0, me->refStride, ws, wh, 2);
     pack2d(c->host + wB, me->input, me->inputStride, bw, bh, 2);
-    k_full_search_one<<<1, 256, lds, c->stream>>>((uint16_t *)c->view, ws, wh, (uint16_t *)(c->view + wB), bw, bh,
-                                                  x0, x1, y0, y1, me->sadLambda, me->predMv.mvX,
-                                                  me->predMv.mvY, (uint32_t *)(c->view + wB + cB));
+    auto *kernel = bw % 4 == 0 ? &k_full_search_one<4> : &k_full_search_one<1>;
+    kernel<<<1, 256, lds, c->stream>>>((uint16_t *)c->view, ws, wh, (uint16_t *)(c->view + wB), bw, bh, x0, x1, y0, y1,
+                                       me->sadLambda, me->predMv.mvX, me->predMv.mvY,
+                                       (uint32_t *)(c->view + wB + cB));
     if (!XG_HIP(hipGetLastError())) return;
     uint32_t *hout = (uint32_t *)(c->host + wB + cB);
     if (!XG_HIP(hipStreamSynchronize(c->stream))) return;
