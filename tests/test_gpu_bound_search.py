@@ -248,3 +248,94 @@ def test_block_search(oracle, kind, rng, ctu, lam, n):
         bad = [i for i, ok in zip(inside, ex.map(check, inside)) if not ok]
     assert not bad, [blocks[i] for i in bad[:5]]
     assert len(inside) > n // 2
+
+
+def search_session(lib, pics, blocks):
+    """A session over the two pictures with these blocks installed."""
+    from xin26x_amd.device import blocks_to_struct
+    s = ctypes.c_void_p()
+    assert lib.xg_session_create(ctypes.byref(s), len(blocks)) == 0
+    for k in (0, 1):
+        assert lib.xg_session_set_picture(s, k, pics[k].ref()) == 0
+    barr = blocks_to_struct(blocks)
+    assert lib.xg_session_set_blocks(s, barr.ctypes.data, len(blocks)) == 0
+    return s
+
+
+def searched(lib, pics, pred, blocks, rng, lam, ctu):
+    """Best MVs of xg_search_blocks, read back through a refinement of one candidate at offset 0."""
+    s = search_session(lib, pics, blocks)
+    try:
+        assert lib.xg_search_blocks(s, rng, lam, ctu) == 0
+        cfg = refine_cfg([(0, 0)], wl.LAMBDA_REFINE, ctu)
+        assert lib.xg_refine_frac(s, ctypes.byref(cfg), pred.ref(), capi.MODE_BATCHED) == 0
+        best = np.zeros((len(blocks), 4), np.int32)
+        assert lib.xg_session_read(s, None, best.ctypes.data) == 0
+        return best[:, :2]
+    finally:
+        lib.xg_session_destroy(s)
+
+
+@pytest.mark.parametrize("kind,rng,ctu,n,large,reach", [
+    ("texture", 16, 64, 3700, 0.15, 2600), ("half", 24, 16, 6200, 0.5, 1500), ("periodic", 32, 33, 9100, 0.66, 2600),
+    ("texture", 17, 64, 3001, 0.0, 2600), ("flat", 16, 7, 3500, 0.1, 600)])
+def test_block_search_is_that_of_short_lists(kind, rng, ctu, n, large, reach):
+    """A long list of blocks in one call against the same blocks in calls below the rule, which search exhaustively:
+    predictors far outside the window, many or no blocks too large for the bounds, at both ends of the list."""
+    lib = capi.load()
+    h, w, pad = 136, 200, 160
+    cur, ref, _ = content(kind, h, w)
+    half = lambda p: np.ascontiguousarray(p[::2, ::2])
+    pics = [DevicePicture([p, half(p), half(p)], pad) for p in (cur, ref)]
+    pred = DevicePicture.empty(w, h)
+    r = np.random.default_rng(n)
+    small, big = ((4, 4), (8, 8), (16, 8), (16, 16), (4, 32), (32, 16)), ((32, 32), (64, 64), (64, 8), (16, 64))
+    blocks = []
+    for i in range(n):
+        t = big if (r.random() < large or (large and i in (0, n - 1))) else small
+        bw, bh = t[int(r.integers(len(t)))]
+        x, y = int(r.integers(0, (w - bw) // 4 + 1)) * 4, int(r.integers(0, (h - bh) // 4 + 1)) * 4
+        blocks.append((x, y, bw, bh, 0, 0, int(r.integers(-reach, reach + 1)), int(r.integers(-reach, reach + 1))))
+    assert sum((b[2] + 2 * rng) * (b[3] + 2 * rng) <= (16 + 2 * rng) * (32 + 2 * rng) for b in blocks) >= 3000
+    m = ctu + 8
+    outside = sum(not (-x - m <= ((px >> 2) + 2) >> 2 <= w + m - bw - x and -y - m <= ((py >> 2) + 2) >> 2 <= h + m - bh - y)
+                  for x, y, bw, bh, _, _, px, py in blocks)
+    assert outside > n // 20
+    got = searched(lib, pics, pred, blocks, rng, 1024, ctu)
+    exp = np.concatenate([searched(lib, pics, pred, blocks[k:k + 2500], rng, 1024, ctu) for k in range(0, n, 2500)])
+    bad = np.flatnonzero((got != exp).any(1))
+    assert bad.size == 0, [(blocks[i], got[i].tolist(), exp[i].tolist()) for i in bad[:4]]
+
+
+def test_large_blocks_take_one_launch():
+    """Blocks that the bounds do not take: a list of them is searched at once, and takes less time than its thirds in
+    three sessions, which the rule leaves to the exhaustive search for their number."""
+    import time
+    lib = capi.load()
+    h, w, pad = 2160, 3840, 96
+    f = wl.smooth_field(h, w, 5)
+    cur, ref = np.ascontiguousarray(f.astype(np.uint16)), np.ascontiguousarray(np.roll(f, 3, 1).astype(np.uint16))
+    half = lambda p: np.ascontiguousarray(p[::2, ::2])
+    pics = [DevicePicture([p, half(p), half(p)], pad) for p in (cur, ref)]
+    blocks = [(x, y, 32, 32, 0, 0, 0, 0) for y in range(0, h - 31, 32) for x in range(0, w, 32)][:7500]
+    parts = [[search_session(lib, pics, blocks)],
+             [search_session(lib, pics, blocks[k:k + 2500]) for k in range(0, 7500, 2500)]]
+
+    def us(sessions):
+        t = []
+        for _ in range(7):
+            t0 = time.perf_counter()
+            for s in sessions:                                # one after the other, several calls in flight
+                for _ in range(6):
+                    assert lib.xg_search_blocks(s, 16, 1024, 64) == 0
+                assert lib.xg_session_sync(s) == 0
+            t.append((time.perf_counter() - t0) / 6 * 1e6)
+        return float(np.median(t[1:]))
+
+    try:
+        whole, thirds = us(parts[0]), us(parts[1])
+        print(f"7,500 blocks of 32x32: whole {whole:.0f} us, in thirds {thirds:.0f}", flush=True)
+        assert whole < 0.97 * thirds
+    finally:
+        for s in parts[0] + parts[1]:
+            lib.xg_session_destroy(s)

@@ -917,13 +917,17 @@ __global__ void __launch_bounds__(256) k_subpel_one(const uint16_t *greg, int rs
     }
 }
 
-// The bounded form of the block search from range 16 and 4,000 blocks on.  With
-// all its launches (predictors, search, refinement), several calls in flight:
+// The bounded form of the block search from range 16 on, where it can take 3,000
+// blocks (bound_block; the others, whatever their number, take as long either way).
+// With all its launches (predictors, search, refinement), several calls in flight:
 // 1280x720 (8,300 blocks) range 16: 166 -> 114 us, range 24: 281 -> 159, range 12:
 // no gain; 960x540 (4,600) range 16: 115 -> 83; 640x360 (2,100) range 16: no gain,
-// and 416x240 (900) 43 -> 53.  With noise of +-64, where most candidates are
-// listed, 1280x720 range 16 takes as long either way.
-constexpr int kBlkMinRange = 16, kBlkMinBlocks = 4000;
+// and 416x240 (900) 43 -> 53.  The search alone at range 16, exhaustive then this
+// form: 3,000 blocks of 8x8 36 -> 20 us, of 16x16 62 -> 39, with 1,000 of 64x64
+// 263 -> 246; 8,000 of 32x32 stay exhaustive.  With noise of sigma 64, where most
+// candidates are listed, 3,000 blocks take 0.79 to 1.03 of the time, 2,000 up to
+// 1.11 of it and 1,000 up to 1.3: the line.
+constexpr int kBlkMinRange = 16, kBlkMinBlocks = 3000;
 static bool bound_blocks_rule(int n, int range, uint32_t lambda)
 {
     return n >= kBlkMinBlocks && range >= kBlkMinRange && lambda <= kSeaLambda;
@@ -995,15 +999,43 @@ __global__ void __launch_bounds__(1024) k_search_blocks(const xg_picture *pics, 
     }
 }
 
-// The same for listed blocks, those that the bounded form leaves.
-constexpr int kRestMax = 480;                    // of a launch: the list travels with its arguments
-struct RestList {
-    int b[kRestMax];
+// The same for the blocks that the bounded form leaves, in one launch whatever
+// their number: workgroup k takes the k-th.  Their counts by runs of `per` session
+// blocks travel with the arguments, and a workgroup looks its block up in its run.
+// (A launch per 480 listed blocks waits for the last of each: 4,100 blocks of 16x16 and
+// 2,000 of 64x64 at range 16 took 439 us, and take 383; exhaustively 431.)
+constexpr int kRestRuns = 480;
+struct RestRuns {
+    int n, per;                                  // session blocks, of a run
+    int before[kRestRuns];                       // blocks left before the run
 };
-__global__ void __launch_bounds__(1024) k_search_blocks_rest(const xg_picture *pics, xg_block *blocks, int range,
-                                                             uint32_t lambda, int ctu, int ws, RestList rest)
+
+// Session block of the k-th block left, in every lane; -1 where there is none.
+__device__ __forceinline__ int rest_block(const RestRuns &l, const xg_block *blocks, int range, int k)
 {
-    const int b = rest.b[blockIdx.x];
+    int run = 0;
+#pragma unroll 1
+    for (int step = 256; step; step >>= 1)       // the last run with no more than k before it
+        if (run + step < kRestRuns && l.before[run + step] <= k) run += step;
+    int at = k - l.before[run];
+    const int end = min(l.n, (run + 1) * l.per);
+    for (int b0 = run * l.per; b0 < end; b0 += 64) {
+        const int b = b0 + (int)(threadIdx.x & 63);
+        const bool left = b < end && !bound_block(blocks[b].w, blocks[b].h, range);
+        const unsigned long long m = __ballot(left);
+        const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        const unsigned long long hit = __ballot(left && rank == at);
+        if (hit) return b0 + (int)__builtin_ctzll(hit);
+        at -= (int)__popcll(m);
+    }
+    return -1;
+}
+
+__global__ void __launch_bounds__(1024) k_search_blocks_rest(const xg_picture *pics, xg_block *blocks, int range,
+                                                             uint32_t lambda, int ctu, int ws, RestRuns runs)
+{
+    const int b = rest_block(runs, blocks, range, (int)blockIdx.x);
+    if (b < 0) return;
     xg_block B = blocks[b];
     search_block(pics, B, range, lambda, ctu, ws);
     if (threadIdx.x == 0) {
@@ -1446,7 +1478,7 @@ int32_t xg_search_blocks(xg_session *s, int32_t range, uint32_t sadLambda, int32
         return XG_ERR_ARG;
     }
     if (v.nblocks == 0) return XG_OK;
-    int maxw = 0, maxh = 0, restw = 0, resth = 0, boundLds = 0;      // rest: those k_search_blocks_bound leaves
+    int maxw = 0, maxh = 0, rest = 0, restw = 0, resth = 0, boundLds = 0;    // rest: those k_search_blocks_bound leaves
     for (int i = 0; i < v.nblocks; i++) {
         const xg_block &B = v.hBlocks[i];
         if (B.pic >= kSessionPicSlots || B.ref >= kSessionPicSlots || !v.picSet[B.pic] || !v.picSet[B.ref]) {
@@ -1472,6 +1504,7 @@ int32_t xg_search_blocks(xg_session *s, int32_t range, uint32_t sadLambda, int32
         if (bound_block(B.w, B.h, range)) {
             boundLds = std::max(boundLds, blk_lds(B.w, B.h, range).bytes);
         } else {
+            rest++;
             restw = std::max(restw, (int)B.w);
             resth = std::max(resth, (int)B.h);
         }
@@ -1482,29 +1515,28 @@ int32_t xg_search_blocks(xg_session *s, int32_t range, uint32_t sadLambda, int32
         set_error(XG_ERR_ARG, "xg_search_blocks: window exceeds the LDS budget");
         return XG_ERR_ARG;
     }
-    const bool bounded = bound_blocks_rule(v.nblocks, range, sadLambda);
+    const bool bounded = bound_blocks_rule(v.nblocks - rest, range, sadLambda);
     int ev[2];
     const bool timed = session_timer_begin(s, 3, ev);
     const int threads = packed_threads(2 * range + 1);
     if (!bounded) {
         k_search_blocks<<<v.nblocks, threads, lds, v.stream>>>(v.dPics, v.dBlocks, range, sadLambda, ctuSize, ws);
     } else {
-        if (restw) {
+        if (rest) {
             const int wsr = packed_ws(2 * range + 1, restw);
             const size_t ldsr = ((size_t)(2 * range + resth) * wsr + (size_t)restw * resth) * 2 + 16;
-            RestList l;
-            for (int i = 0, k = 0; i < v.nblocks; i++) {
-                if (!bound_block(v.hBlocks[i].w, v.hBlocks[i].h, range)) l.b[k++] = i;
-                if (k == kRestMax || (k && i == v.nblocks - 1)) {
-                    k_search_blocks_rest<<<k, threads, ldsr, v.stream>>>(v.dPics, v.dBlocks, range, sadLambda, ctuSize,
-                                                                         wsr, l);
-                    k = 0;
-                }
+            RestRuns l;
+            l.n = v.nblocks;
+            l.per = (v.nblocks + kRestRuns - 1) / kRestRuns;
+            int left = 0, b = 0;
+            for (int r = 0; r < kRestRuns; r++) {
+                l.before[r] = left;
+                for (const int e = std::min(v.nblocks, (r + 1) * l.per); b < e; b++)
+                    left += !bound_block(v.hBlocks[b].w, v.hBlocks[b].h, range);
             }
+            k_search_blocks_rest<<<rest, threads, ldsr, v.stream>>>(v.dPics, v.dBlocks, range, sadLambda, ctuSize, wsr, l);
         }
-        if (boundLds)
-            k_search_blocks_bound<<<v.nblocks, kBlkWg, (size_t)boundLds, v.stream>>>(v.dPics, v.dBlocks, range, sadLambda,
-                                                                                   ctuSize);
+        k_search_blocks_bound<<<v.nblocks, kBlkWg, (size_t)boundLds, v.stream>>>(v.dPics, v.dBlocks, range, sadLambda, ctuSize);
     }
     if (timed) session_timer_end(s, 3, ev);
     return XG_HIP(hipGetLastError()) ? XG_OK : XG_ERR_HIP;
