@@ -978,8 +978,9 @@ __device__ __forceinline__ void search_block(const xg_picture *pics, xg_block &B
     B.mvy = 16 * (y0 + i / nx);
 }
 
-// Session blocks that k_search_blocks_bound takes; the others' windows are too
-// large for its one wave (bound_blocks_rule).
+// Session blocks that k_search_blocks_bound takes: the others' windows would leave
+// its two waves too few to a CU.  From range 16 on (bound_blocks_rule) no block 64
+// wide is among them, and 32-wide ones up to a height of 16.
 __host__ __device__ __forceinline__ bool bound_block(int w, int h, int range)
 {
     return (w + 2 * range) * (h + 2 * range) <= (16 + 2 * range) * (32 + 2 * range);
@@ -1327,8 +1328,7 @@ __global__ void __launch_bounds__(kBlkWg) __attribute__((amdgpu_waves_per_eu(6))
     case 4: k = bound_search<4>(smem32, o, v, limits); break;
     case 8: k = bound_search<8>(smem32, o, v, limits); break;
     case 16: k = bound_search<16>(smem32, o, v, limits); break;
-    case 32: k = bound_search<32>(smem32, o, v, limits); break;
-    default: k = bound_search<64>(smem32, o, v, limits); break;
+    default: k = bound_search<32>(smem32, o, v, limits); break;      // bound_block: no wider
     }
     if ((tid & 63) == 0) found[tid >> 6] = k;
     __syncthreads();
