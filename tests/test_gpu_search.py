@@ -334,3 +334,28 @@ def test_full_search_stages_as_fast_as_the_diamond():
     full, dia = us(lib.Xg26xMotionEstFull), us(lib.Xg26xMotionEstDia)
     print(f"1x1 at +/-80: full {full:.1f} us, diamond {dia:.1f} us", flush=True)
     assert full < 2.5 * dia
+
+
+@pytest.mark.parametrize("w,h,sw", [(128, 128, 8), (128, 64, 8), (64, 128, 20), (96, 100, 12), (100, 70, 64), (127, 128, 3),
+                                    (64, 64, 64), (64, 64, 6), (8, 8, 78)])
+def test_diamond_and_subpel_of_large_blocks_and_windows(oracle, w, h, sw):
+    """The forms of the per-call diamond and rings on either side of their LDS limit: regions read in place because
+    they do not fit, first passes in several strips (128x128), widths over a wave and no powers of two."""
+    lib = capi.load()
+    lib.xg_clear_error()
+    rng, plane, cur = _planes(38)
+    for k in range(4):
+        bx, by = int(rng.integers(0, 260 - w)), int(rng.integers(0, 180 - h))
+        mn = (-bx - 72, -by - 72)
+        mx = (260 + 72 - w - bx, 180 + 72 - h - by)
+        cands = [(0, 0)] + [(int(a), int(b)) for a, b in rng.integers(-sw, sw + 1, size=(int(rng.integers(1, 12)), 2))]
+        pred = (int(rng.integers(-30, 30)), int(rng.integers(-30, 30)))
+        xm, om = _me_pair(rng, plane, cur, w, h, bx, by, pred, sw, 256, mn, mx, cands)
+        lib.Xg26xMotionEstDia(ctypes.byref(xm))
+        oracle.or_MotionEstDia(ctypes.byref(om))
+        assert (xm.bestMv.mvX, xm.bestMv.mvY, xm.bestCost, xm.bestSad) == \
+               (om.bestMvX, om.bestMvY, om.bestCost, om.bestSad), k
+        lib.Xg266FullSubPelMe(ctypes.byref(xm))
+        oracle.or_FullSubPelMe(ctypes.byref(om))
+        assert (xm.bestMv.mvX, xm.bestMv.mvY, xm.bestCost) == (om.bestMvX, om.bestMvY, om.bestCost), k
+    assert lib.xg_last_error() == 0
