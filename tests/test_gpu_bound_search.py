@@ -339,3 +339,42 @@ def test_large_blocks_take_one_launch():
     finally:
         for s in parts[0] + parts[1]:
             lib.xg_session_destroy(s)
+
+
+def call_us(lib, s, call, n=4, reps=7):
+    """Median time in us of a call, n in flight."""
+    import time
+    t = []
+    for _ in range(reps):
+        t0 = time.perf_counter()
+        for _ in range(n):
+            assert call() == 0
+        assert lib.xg_session_sync(s) == 0
+        t.append((time.perf_counter() - t0) / n * 1e6)
+    return float(np.median(t[1:]))
+
+
+EXHAUSTIVE = (1 << 21) + 1             # a rate weight past the rules: the same call, every SAD
+
+
+def test_flat_frames_cost_little_more_in_the_pipeline():
+    """A flat noisy frame, whose blocks all end in the exhaustive search, against the exhaustive form."""
+    lib = capi.load()
+    h, w, pad = 1088, 1920, 96
+    half = lambda p: np.ascontiguousarray(p[::2, ::2])
+    pics = [DevicePicture([p, half(p), half(p)], pad) for p in content("flat", h, w)]
+    pred = DevicePicture.empty(w, h)
+    s = ctypes.c_void_p()
+    assert lib.xg_session_create(ctypes.byref(s), (w // 16) * (h // 16)) == 0
+    try:
+        us = []
+        for lam in (1024, EXHAUSTIVE):
+            cfg = capi.XgPipelineCfg()
+            cfg.range, cfg.sadLambda, cfg.ctuSize = 64, lam, 64
+            cfg.refine = refine_cfg([(0, 0)], wl.LAMBDA_REFINE)
+            us.append(call_us(lib, s, lambda: lib.xg_me_pipeline(s, ctypes.byref(cfg), pics[0].ref(), pics[1].ref(),
+                                                                 pics[2].ref(), pred.ref(), capi.MODE_BATCHED)))
+        print(f"flat 1920x1088 +/-64: bounded {us[0]:.0f} us, exhaustive {us[1]:.0f}", flush=True)
+        assert us[0] < 1.24 * us[1]
+    finally:
+        lib.xg_session_destroy(s)

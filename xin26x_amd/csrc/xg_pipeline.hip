@@ -36,7 +36,6 @@
 #include <string.h>
 #include <vector>
 
-#include "xg_batch.hpp"
 #include "xg_device.hpp"
 #include "xg_runtime.hpp"
 #include "xg_sea.hpp"
@@ -171,7 +170,10 @@ __device__ __forceinline__ unsigned long long wave_min_u64(unsigned long long k)
 
 // ---------------------------------------------------------------------------
 // 1. Full search, exhaustive form: a workgroup per block and reference; LISTED:
-// those of the list a.dense, one after the other
+// per entry of the list a.dense, the workgroups past its end leave at once (with 1.5 %
+// of 64,800 listed the launch takes 36 us, as a resident grid that shares the entries
+// out; with all of them listed that grid took 13 % longer, some of its workgroups
+// being late)
 // ---------------------------------------------------------------------------
 // Each lane costs NQ quads (4 * NQ horizontally adjacent candidates) of one
 // search row: the window row's dwords D and their one-sample realignment F are
@@ -183,9 +185,8 @@ __global__ void __launch_bounds__(256) k_pipe_full(PipeArgs a)
     __shared__ __align__(16) uint16_t win[kPipeWinH * kPipeWinW];
     __shared__ __align__(16) uint32_t curL[kPB * kPB / 2];     // packed pairs
     __shared__ unsigned long long red[4];
-    const int listed = LISTED ? a.dense[0] : (int)blockIdx.x + 1;
-    for (int li = blockIdx.x; li < listed; li += gridDim.x) {
-    const int id = LISTED ? a.dense[1 + li] : li;
+    if (LISTED && (int)blockIdx.x >= a.dense[0]) return;
+    const int id = LISTED ? a.dense[1 + blockIdx.x] : (int)blockIdx.x;
     const int b = id >> 1, r = id & 1;
     const int x = (b % a.nbx) * kPB, y = (b / a.nbx) * kPB;
     const IWin w = int_window(x, y, a.fw, a.fh, a.ctu);
@@ -195,7 +196,6 @@ __global__ void __launch_bounds__(256) k_pipe_full(PipeArgs a)
     const xg_plane &RP = a.pics[r ? a.refSlot1 : a.refSlot0].plane[0];
     const xg_plane &CP = a.pics[a.curSlot].plane[0];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    if (LISTED) __syncthreads();                    // the previous block's readers are done
     {   // window rows (ny + 15) x (nx + 15) samples: a wave per row, lanes along it,
         // 4 rows x 3 columns of loads in flight per lane
         const int rows = ny + kPB - 1, cols = nx + kPB - 1;
@@ -304,7 +304,6 @@ __global__ void __launch_bounds__(256) k_pipe_full(PipeArgs a)
         best = min_u64(min_u64(red[0], red[1]), min_u64(red[2], red[3]));
         const int idx = (int)(uint32_t)best;
         a.found[id].best = (uint32_t)((y0 + idx / nx + 128) << 8 | (x0 + idx % nx + 128));
-    }
     }
 }
 
@@ -916,7 +915,6 @@ struct PipeState {
     int *dDense = nullptr;             // list of the exhaustive search
     PipeFound *dFound = nullptr;       // the full search's result per block and reference
     uint32_t *dLeft = nullptr;         // what the bounded search's scans leave
-    int denseGrid = 0;                 // its workgroups
     bool bounded = false;              // the full search takes the bounded form
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -975,7 +973,6 @@ static bool sums_prepare(PipeState *p, int range, int ctu, hipStream_t st)
         if (!XG_HIP(hipMalloc((void **)&p->dSums, need * sizeof(uint16_t)))) return false;
         p->sumsCap = need;
     }
-    if (!p->denseGrid) p->denseGrid = resident_slots((const void *)k_pipe_full<kPipeQuads, true>, 256);
     for (int k = 0; k < 2; k++)
         p->args.sums[k] = {p->dSums + 2 * k * one, p->dSums + (2 * k + 1) * one, stride, -left, -left, w, h};
     p->args.dense = p->dDense;
@@ -995,7 +992,7 @@ static bool enqueue_pipe(const PipeState *p, hipStream_t st, xg_session *s, bool
         k_pipe_bound<<<8 * per, 64 * kBoundWaves, 0, st>>>(p->args, per);
         const int perLeft = ((2 * p->nb + 3) / 4 + 7) / 8;
         k_pipe_left<<<8 * perLeft, 256, 0, st>>>(p->args, perLeft);
-        k_pipe_full<kPipeQuads, true><<<std::min(2 * p->nb, p->denseGrid), 256, 0, st>>>(p->args);
+        k_pipe_full<kPipeQuads, true><<<2 * p->nb, 256, 0, st>>>(p->args);
     } else {
         k_pipe_full<kPipeQuads, false><<<2 * p->nb, 256, 0, st>>>(p->args);
     }
