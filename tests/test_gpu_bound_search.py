@@ -25,6 +25,8 @@ def content(kind, h, w, seed=3):
         out = [cut(0, 0) + r.integers(-4, 5, (h, w)), cut(9, -23), cut(-31, 14) + r.integers(-2, 3, (h, w))]
     elif kind == "flat":
         out = [500 + np.rint(r.normal(0, 4, (h, w))) for _ in range(3)]
+    elif kind == "noise":
+        out = [p + np.rint(r.normal(0, 64, (h, w))) for p in content("texture", h, w, seed)]
     elif kind == "half":
         a, b = content("texture", h, w, seed), content("flat", h, w, seed)
         out = [np.where(np.arange(w) < w // 2, p, q) for p, q in zip(a, b)]
@@ -378,3 +380,24 @@ def test_flat_frames_cost_little_more_in_the_pipeline():
         assert us[0] < 1.24 * us[1]
     finally:
         lib.xg_session_destroy(s)
+
+
+def test_noisy_frames_cost_little_more():
+    """Frame search of content whose bounds exclude little, against the exhaustive form."""
+    import torch
+    lib = capi.load()
+    h, w = 720, 1280
+    cur, ref = (DevicePicture([p, p[::2, ::2].copy(), p[::2, ::2].copy()], 96) for p in content("noise", h, w)[:2])
+    nb = (w // 16) * (h // 16)
+    out = [torch.zeros(2 * nb, dtype=torch.int32, device="cuda") for _ in range(3)]
+    torch.cuda.synchronize()
+    s = ctypes.c_void_p()
+    assert lib.xg_session_create(ctypes.byref(s), 16) == 0
+    try:
+        us = [call_us(lib, s, lambda: lib.xg_full_search_frame(
+            s, ctypes.byref(cur.pic.plane[0]), ctypes.byref(ref.pic.plane[0]), 16, 16, 16, lam, 64,
+            *[t.data_ptr() for t in out]), n=20) for lam in (1024, EXHAUSTIVE)]
+    finally:
+        lib.xg_session_destroy(s)
+    print(f"noise, 1280x720 16x16 +/-16: bounded {us[0]:.0f} us, exhaustive {us[1]:.0f}", flush=True)
+    assert us[0] < 1.5 * us[1]

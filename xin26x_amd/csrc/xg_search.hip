@@ -312,9 +312,12 @@ __global__ void __launch_bounds__(1024) k_full_search_frame_p(FsFrameArgs a, int
 //   832x480 16x16 range 16: 22 -> 17; range 12: 13.5 -> 15
 //   640x360 16x16 range 16: 14 -> 15; 8x8 range 16: 21 -> 15; 8x8 range 12: 14 -> 14
 //   320x320 8x8 range 16: 11 -> 12; 480x400 8x8 range 16: 18 -> 14
-// With noise of +-64, where nearly every block is searched exhaustively, 1080p
-// range 16: 16x16 109 -> 109, 8x8 168 -> 200.
-// A lone 832x480 16x16 call at range 16 takes 37 -> 40 us, 640x360 8x8 34.5 -> 33.
+// Where nearly every block is searched exhaustively (flat with noise, or noise of
+// sigma 64) the limits and scans come on top, and small frames have too few
+// workgroups to hide it: 1920x1080 range 16 16x16 107 -> 106 to 111, 8x8 179 -> 172
+// to 181, range 32 380 -> 333; 1280x720 range 16 16x16 50 -> 61, 8x8 83 -> 91;
+// 832x480 8x8 39 -> 49.  With noise of sigma 16 nothing of this shows (1280x720
+// 16x16 50 -> 30).  A lone 640x360 8x8 call at range 16 takes 34.5 -> 33 us.
 // The rule: range 16 and over, and 1,750 blocks of 16x16 or 3,500 of 8x8.
 // ---------------------------------------------------------------------------
 constexpr int kSeaMinRange = 16;
@@ -330,6 +333,7 @@ struct SeaFrameArgs {
     int wp, sp;                                  // LDS pitches of window and sums in dwords (odd)
     int rows;                                    // LDS rows of the window
     int aligned;                                 // reference rows are dword aligned
+    int most;                                    // list entries past which every candidate is costed instead
 };
 
 // LDS dwords of the window, of the sums and in all for a range
@@ -349,7 +353,7 @@ __global__ void __launch_bounds__(256) k_search_bound(SeaFrameArgs a)
     constexpr int ND = BS / 2;
     extern __shared__ uint32_t smem32[];
     __shared__ unsigned long long found[4];      // lowest (cost, position) of each block
-    __shared__ int lists[4];                     // entries of each list; over kSeaList: exhaustive
+    __shared__ int lists[4];                     // entries of each list; over a.most: exhaustive
     const FsFrameArgs &f = a.f;
     const int R = f.range, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     uint32_t *win = smem32, *S = win + a.wp * a.rows;
@@ -557,7 +561,7 @@ __global__ void __launch_bounds__(256) k_search_bound(SeaFrameArgs a)
     const int items = K * nc, rem = items & 63;
     const bool spread = 2 * ((rem * steps + 63) >> 6) < steps;
     const int whole = spread ? items - rem : items, tasks = spread ? rem * steps : 0;
-    for (int i0 = 0; i0 < whole + tasks && n <= kSeaList; i0 += 64) {
+    for (int i0 = 0; i0 < whole + tasks && n <= a.most; i0 += 64) {
         const int i = i0 + lane;
         int it, u0 = 0;
         bool in;
@@ -602,14 +606,16 @@ __global__ void __launch_bounds__(256) k_search_bound(SeaFrameArgs a)
     }
     __syncthreads();
 
-    // all waves: every block's list, or every candidate of a block whose list overflowed
+    // all waves: every block's list, or every candidate of a block whose list overflowed, 64 items
+    // (four adjacent candidates of a row) a wave in turn over all such blocks
+    int turn = 0;
     for (int q = 0; q < 4; q++) {
         const int n = lists[q];
         if (!n) continue;
         const View v = view(2 * gx + (q & 1), 2 * gy + (q >> 1));
         const uint32_t *cl = curL + q * BS * ND;
         unsigned long long k = ~0ull;
-        if (n <= kSeaList) {
+        if (n <= a.most) {
             const uint32_t *cr = cl + (lane % LR) * ND;
 #pragma unroll
             for (int j = 0; j < ND; j++) c[j] = cr[j];
@@ -620,10 +626,12 @@ __global__ void __launch_bounds__(256) k_search_bound(SeaFrameArgs a)
             }
         } else {
             // four adjacent candidates of a row a thread, which come in raster order: strict < keeps the earliest
-            const int nq = (v.nx + v.p + 3) >> 2;
+            const int nq = (v.nx + v.p + 3) >> 2, items = v.ny * nq;
+            const int first = 64 * ((wave - turn) & 3) + lane;
+            turn += (items + 63) >> 6;
             uint32_t bcst = 0xFFFFFFFFu;
             int bpos = 0;
-            for (int it = tid; it < v.ny * nq; it += 256) {
+            for (int it = first; it < items; it += 256) {
                 const int dy = it / nq, qd = it - dy * nq;
                 const uint32_t *w = v.W + dy * a.wp + 2 * qd;
                 uint32_t acc[4] = {0, 0, 0, 0};
@@ -1595,6 +1603,8 @@ int32_t xg::full_search_frame_on(hipStream_t st, xg_session *timer, const xg_pla
         b.f = a;
         b.ngx = (nbx + 1) / 2;
         b.aligned = (a.rs & 1) == 0;
+        // costed four a lane at once, a candidate takes about a third of a listed one's instructions
+        b.most = std::min(kSeaList, (2 * range + 1) * (2 * range + 1) / 3);
         const int groups = b.ngx * ((nby + 1) / 2);
         if (bw == 8) k_search_bound<8><<<groups, 256, seaLds, st>>>(b);
         else k_search_bound<16><<<groups, 256, seaLds, st>>>(b);
