@@ -280,7 +280,8 @@ def searched(lib, pics, pred, blocks, rng, lam, ctu):
 
 @pytest.mark.parametrize("kind,rng,ctu,n,large,reach", [
     ("texture", 16, 64, 3700, 0.15, 2600), ("half", 24, 16, 6200, 0.5, 1500), ("periodic", 32, 33, 9100, 0.66, 2600),
-    ("texture", 17, 64, 3001, 0.0, 2600), ("flat", 16, 7, 3500, 0.1, 600)])
+    ("texture", 17, 64, 3001, 0.0, 2600), ("flat", 16, 7, 3500, 0.1, 600), ("flat", 25, 40, 3300, 0.0, 2600),
+    ("noise", 32, 64, 3200, 0.0, 1500), ("constant", 19, 64, 3100, 0.0, 300)])
 def test_block_search_is_that_of_short_lists(kind, rng, ctu, n, large, reach):
     """A long list of blocks in one call against the same blocks in calls below the rule, which search exhaustively:
     predictors far outside the window, many or no blocks too large for the bounds, at both ends of the list."""
@@ -302,7 +303,7 @@ def test_block_search_is_that_of_short_lists(kind, rng, ctu, n, large, reach):
     m = ctu + 8
     outside = sum(not (-x - m <= ((px >> 2) + 2) >> 2 <= w + m - bw - x and -y - m <= ((py >> 2) + 2) >> 2 <= h + m - bh - y)
                   for x, y, bw, bh, _, _, px, py in blocks)
-    assert outside > n // 20
+    assert outside > n // 20 or reach < 2000
     got = searched(lib, pics, pred, blocks, rng, 1024, ctu)
     exp = np.concatenate([searched(lib, pics, pred, blocks[k:k + 2500], rng, 1024, ctu) for k in range(0, n, 2500)])
     bad = np.flatnonzero((got != exp).any(1))
@@ -401,3 +402,18 @@ def test_noisy_frames_cost_little_more():
         lib.xg_session_destroy(s)
     print(f"noise, 1280x720 16x16 +/-16: bounded {us[0]:.0f} us, exhaustive {us[1]:.0f}", flush=True)
     assert us[0] < 1.5 * us[1]
+
+
+def test_flat_blocks_cost_little_more():
+    """Block search of flat noisy content, where the bounds exclude nothing, against the exhaustive form."""
+    lib = capi.load()
+    h, w = 1088, 1920
+    half = lambda p: np.ascontiguousarray(p[::2, ::2])
+    pics = [DevicePicture([p, half(p), half(p)], 96) for p in content("flat", h, w)[:2]]
+    s = search_session(lib, pics, [(x, y, 16, 16, 0, 0, 0, 0) for y in range(0, h, 16) for x in range(0, w, 16)])
+    try:
+        us = [call_us(lib, s, lambda: lib.xg_search_blocks(s, 16, lam, 64), n=10) for lam in (1024, EXHAUSTIVE)]
+    finally:
+        lib.xg_session_destroy(s)
+    print(f"flat 1920x1088 16x16 blocks +/-16: bounded {us[0]:.0f} us, exhaustive {us[1]:.0f}", flush=True)
+    assert us[0] < 1.2 * us[1]

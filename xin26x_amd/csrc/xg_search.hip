@@ -1062,17 +1062,21 @@ __global__ void __launch_bounds__(1024) k_search_blocks_rest(const xg_picture *p
 // lane each: their lowest cost limits the rest.  (2) Every candidate whose
 // bound is within the limit goes to its wave's list, which is costed 64 at a
 // time, a lane each, and may lower the wave's limit.  A lane that costs a whole candidate needs no
-// reduction, and flat content, where every candidate is listed, is searched at
-// the cost of the exhaustive form.  Up to three waves' worth of candidates are
-// costed without bounds.
+// reduction.  Where over 48 of the 128 lanes' first candidates lie within the limit
+// (flat or noisy content) no list is made and every candidate is costed, four a lane
+// at once, which takes 0.44 of a listed candidate's instructions.  Up to three
+// waves' worth of candidates are costed without bounds.
 //
 // 1280x720, 8,300 blocks, range 16: 124 us exhaustively; 68 us here, 21 M vector
 // instructions (35 us to issue) at 3 waves a SIMD, which is what 13 KB of window
 // and sums a block leave, and 20 us for the 2 % that go by the list.  Two waves a
-// block: one took 87 us.
+// block: one took 87 us.  32,400 blocks of 16x16 at range 16, exhaustively and here:
+// texture 623 and 302 us, noise of sigma 64 625 and 440, flat with noise 624 and 475
+// (1,068 by lists); 4,000 of 16x32 at range 32 flat 393 and 442, the worst measured.
 // ---------------------------------------------------------------------------
 constexpr int kBlkDirect = 192;                  // candidates costed without bounds at most
 constexpr int kBlkWaves = 2, kBlkWg = 64 * kBlkWaves;
+constexpr int kBlkDense = 48;                    // of the 128 lanes' first candidates within the limit, past which every one is costed
 constexpr int kBlkList = 192;                    // of a wave: under 64 when a step adds up to 128
 
 struct BlkLds {
@@ -1111,6 +1115,34 @@ __device__ __forceinline__ uint32_t lane_sad(const uint32_t *win, int wp, const 
             for (int j = 0; j < CH; j++) e = sad2(align16(D[j + 1], D[j], sh), cur[k + j], e);
         }
     return e;
+}
+
+// SADs of the four candidates from column 4 q of window row cy, by one lane.
+template <int W>
+__device__ __forceinline__ void lane_sad4(const uint32_t *win, int wp, const uint32_t *cur, int h, int q, int cy,
+                                          uint32_t (&e)[4])
+{
+    constexpr int CH = W < 16 ? W / 2 : 8;
+    const uint32_t *w = win + cy * wp + 2 * q;
+    e[0] = e[1] = e[2] = e[3] = 0;
+#pragma unroll 1
+    for (int i = 0; i < h; i++, w += wp, cur += W / 2)
+#pragma unroll
+        for (int k = 0; k < W / 2; k += CH) {
+            uint32_t D[CH + 2], F[CH + 1];
+#pragma unroll
+            for (int j = 0; j < CH + 2; j++) D[j] = w[k + j];
+#pragma unroll
+            for (int j = 0; j < CH + 1; j++) F[j] = align16(D[j + 1], D[j], 16);
+#pragma unroll
+            for (int j = 0; j < CH; j++) {
+                const uint32_t c = cur[k + j];
+                e[0] = sad2(D[j], c, e[0]);
+                e[1] = sad2(F[j], c, e[1]);
+                e[2] = sad2(D[j + 1], c, e[2]);
+                e[3] = sad2(F[j + 1], c, e[3]);
+            }
+        }
 }
 
 // Bounds of candidates 2 j and 2 j + 1 of a row (q: their dword of the sums) of a
@@ -1170,12 +1202,13 @@ __device__ __forceinline__ unsigned long long bound_search(uint32_t *lds, const 
         const uint32_t rcp = (65536u + (uint32_t)nc - 1) / (uint32_t)nc;
         const int dr = (int)(((uint32_t)kBlkWg * rcp) >> 16), dj = kBlkWg - dr * nc;
         const int r0 = (int)(((uint32_t)tid * rcp) >> 16), j0 = tid - r0 * nc;
-        uint32_t key = 0xFFFFFFFFu;
+        uint32_t key = 0xFFFFFFFFu, first = kSeaOver;    // first: the bound of the lane's first candidate
         int kpos = 0;
-        for (int i = tid, r = r0, j = j0; i < items; i += kBlkWg) {
+        for (int i = tid, s = 0, r = r0, j = j0; i < items; i += kBlkWg, s++) {
             uint32_t l = byq[r] + bxq[2 * j], h = byq[r] + bxq[2 * j + 1];
             lane_bounds<W>(S + r * wp + j, wp, C, hs, l, h);
             const uint32_t k = min(l, h);
+            first = s ? first : l;
             kpos = k < key ? r << 8 | (2 * j + (h < l)) : kpos;
             key = min(key, k);
             r += dr;
@@ -1187,9 +1220,14 @@ __device__ __forceinline__ unsigned long long bound_search(uint32_t *lds, const 
         }
         cost(kpos);                              // lanes without an item cost candidate 0
         uint32_t limit = wave_min((uint32_t)(best >> 32)) >> 8;
-        if (lane == 0) limits[wave] = limit;
+        const int within = (int)__popcll(__ballot(first <= limit));
+        if (lane == 0) {
+            limits[wave] = limit;
+            limits[kBlkWaves + wave] = (uint32_t)within;
+        }
         __syncthreads();
         limit = min(limits[0], limits[1]);
+        const bool dense = (int)uniform((int)(limits[kBlkWaves] + limits[kBlkWaves + 1])) > kBlkDense;
         int n = 0;
         auto flush = [&]() {                     // cost the first 64 of the list, keep the others
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1202,7 +1240,7 @@ __device__ __forceinline__ unsigned long long bound_search(uint32_t *lds, const 
             if (lane + 64 < rest) list[64 + lane] = b;
             n = max(rest, 0);
         };
-        for (int i0 = 64 * wave, r = r0, j = j0; i0 < items; i0 += kBlkWg) {
+        for (int i0 = 64 * wave, r = r0, j = j0; i0 < items && !dense; i0 += kBlkWg) {
             const bool in = i0 + lane < items;
             uint32_t l = kSeaOver, h = kSeaOver;
             if (in) {
@@ -1227,7 +1265,29 @@ __device__ __forceinline__ unsigned long long bound_search(uint32_t *lds, const 
                 r++;
             }
         }
-        if (n) flush();
+        if (dense) {
+            const int nq = (nx + 3) >> 2;
+            uint32_t bc = 0xFFFFFFFFu;
+            int bp = 0;                          // a lane's candidates come in raster order: strict < keeps the earliest
+            for (int i = tid; i < ny * nq; i += kBlkWg) {
+                const int cy = i / nq, q = i - cy * nq;
+                uint32_t e[4];
+                lane_sad4<W>(win, wp, cur, v.h, q, cy, e);
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    const int cx = 4 * q + m;
+                    const uint32_t k = (e[m] << 8) + (eg_bits(4 * (v.x0 + cx) - v.pmx) + eg_bits(4 * (v.y0 + cy) - v.pmy)) * v.lambda;
+                    if (cx < nx && k < bc) {
+                        bc = k;
+                        bp = cy << 8 | cx;
+                    }
+                }
+            }
+            const unsigned long long q = ((unsigned long long)bc << 32) | (uint32_t)bp;
+            best = q < best ? q : best;
+        } else if (n) {
+            flush();
+        }
     }
     const uint32_t lo = wave_min((uint32_t)(best >> 32));
     const uint32_t pos = wave_min((uint32_t)(best >> 32) == lo ? (uint32_t)best : 0xFFFFFFFFu);
@@ -1238,7 +1298,7 @@ __global__ void __launch_bounds__(kBlkWg) __attribute__((amdgpu_waves_per_eu(6))
                                                             uint32_t lambda, int ctu)
 {
     extern __shared__ uint32_t smem32[];
-    __shared__ uint32_t limits[kBlkWaves];
+    __shared__ uint32_t limits[2 * kBlkWaves];   // of the waves: limit, first candidates within it
     __shared__ unsigned long long found[kBlkWaves];
     const int tid = threadIdx.x;
     const xg_block &B = blocks[blockIdx.x];
