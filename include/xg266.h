@@ -7,7 +7,8 @@
  *     primitive table `xin_func_struct` (h266_encoder/include/h266_func_struct.h:719-799)
  *     and of its motion-estimation entry points.  Pointers are HOST pointers
  *     into the caller's buffers, as in the reference; each call stages the
- *     bytes it needs to HBM, runs one HIP kernel and returns synchronously.
+ *     bytes it needs (in page-locked memory that the GPU reads over the bus, or
+ *     in HBM), runs on the GPU and returns synchronously.
  *     A C encoder assigns these to its table after Xin266FuncInit; the
  *     Xg266FuncInit helper fills the mirror table below.
  *

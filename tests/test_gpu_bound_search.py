@@ -193,7 +193,7 @@ def test_frame_search(oracle, kind, size, bs, rng, ctu, lam, shift):
     ("flat", 16, 7, 0, 4000), ("extreme", 24, 64, 1024, 4000), ("extreme", 16, 64, 1 << 21, 4000),
     ("periodic", 19, 64, 0, 4000), ("constant", 16, 31, 0, 4000)])
 def test_block_search(oracle, kind, rng, ctu, lam, n):
-    """Session blocks of every shape, large ones listed over several launches, on both sides of the rule."""
+    """Session blocks of every shape, the large ones in their own launch, on both sides of the rule."""
     from tests.oracle_lib import OrMe
     from xin26x_amd.device import blocks_to_struct
     lib = capi.load()

@@ -27,9 +27,10 @@
 // every candidate with two v_sad_u16 instead of 128 and keeps those whose bound
 // does not exceed the cost already reached; k_pipe_left costs them.  Blocks that
 // keep too many (flat, noisy content) go to the exhaustive k_pipe_full through a
-// device list.  3840x2160, two references, +/-64, textured content: 1.02 ms
-// (sums 0.03, bounds 0.77, costs 0.14, exhaustive 0.08 for 1.5% of the blocks)
-// against 5.43 ms for k_pipe_full over every block.
+// device list.  3840x2160, two references, +/-64, textured content: 0.85 ms
+// (sums 0.02, bounds 0.71, costs 0.08, exhaustive 0.04 for 1.5% of the blocks)
+// against 5.24 ms for k_pipe_full over every block.  A whole frame that is flat with
+// noise takes 6.65 ms against 5.93.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -910,11 +911,11 @@ struct PipeState {
     uint64_t gridVersion = 0;          // session blocksVersion right after the grid was installed
     int16_t *dMv = nullptr;            // fullMv | predMv | intMv | qMv, 4 x nb x 4 int16
     uint32_t *dCost = nullptr;         // intCost | qCost, 2 x nb x 2
-    uint16_t *dSums = nullptr;         // box sums of both references
+    uint16_t *dSums = nullptr;         // box sums of both references, 8 B a sample (72 MB at 4K)
     size_t sumsCap = 0;
     int *dDense = nullptr;             // list of the exhaustive search
     PipeFound *dFound = nullptr;       // the full search's result per block and reference
-    uint32_t *dLeft = nullptr;         // what the bounded search's scans leave
+    uint32_t *dLeft = nullptr;         // what the bounded search's scans leave, 2 KB a block (66 MB at 4K)
     bool bounded = false;              // the full search takes the bounded form
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;

@@ -779,8 +779,8 @@ __device__ __forceinline__ void mc_block(ArgPtr a, ListPtr l, int b, const xg_bl
         }
 }
 
-// Bound by VALU issue.  1920x1080, 32 candidates, 18,600 blocks: 48.3 M vector
-// instructions, which take 79 us to issue; 86 us a launch with several in
+// Bound by VALU issue.  1920x1080, 32 candidates, 18,600 blocks: 47.8 M vector
+// instructions, which take 78 us to issue; 86 us a launch with several in
 // flight, 126 alone (62.2 M, 107 and 151 before).  About 30 M are the filters
 // and transforms; the rest, once as large as these, is what a task does beside
 // them: descriptors and windows addressed with scalars (a division-free copy

@@ -932,9 +932,9 @@ __global__ void __launch_bounds__(256) k_subpel_one(const uint16_t *greg, int rs
 // no gain; 960x540 (4,600) range 16: 115 -> 83; 640x360 (2,100) range 16: no gain,
 // and 416x240 (900) 43 -> 53.  The search alone at range 16, exhaustive then this
 // form: 3,000 blocks of 8x8 36 -> 20 us, of 16x16 62 -> 39, with 1,000 of 64x64
-// 263 -> 246; 8,000 of 32x32 stay exhaustive.  With noise of sigma 64, where most
-// candidates are listed, 3,000 blocks take 0.79 to 1.03 of the time, 2,000 up to
-// 1.11 of it and 1,000 up to 1.3: the line.
+// 263 -> 252; 8,000 of 32x32 stay exhaustive.  With noise of sigma 64, or flat with
+// noise, 3,000 blocks of up to 16x16 take 0.64 to 1.06 of the time (of 16x32 up to
+// 1.17, flat), 2,000 up to 1.17 of it and 1,000 up to 1.45: the line.
 constexpr int kBlkMinRange = 16, kBlkMinBlocks = 3000;
 static bool bound_blocks_rule(int n, int range, uint32_t lambda)
 {
@@ -1069,7 +1069,7 @@ __global__ void __launch_bounds__(1024) k_search_blocks_rest(const xg_picture *p
 //
 // 1280x720, 8,300 blocks, range 16: 124 us exhaustively; 68 us here, 21 M vector
 // instructions (35 us to issue) at 3 waves a SIMD, which is what 13 KB of window
-// and sums a block leave, and 20 us for the 2 % that go by the list.  Two waves a
+// and sums a block leave, and 20 us for the 2 % it leaves.  Two waves a
 // block: one took 87 us.  32,400 blocks of 16x16 at range 16, exhaustively and here:
 // texture 623 and 302 us, noise of sigma 64 625 and 440, flat with noise 624 and 475
 // (1,068 by lists); 4,000 of 16x32 at range 32 flat 393 and 442, the worst measured.
